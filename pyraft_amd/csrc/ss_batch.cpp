@@ -121,7 +121,7 @@ std::map<std::string, TuneEntry> g_tune;
 // A file of another format is ignored and a line that does not parse is skipped (that
 // geometry is timed again).  After each new choice the file is written whole to a
 // temporary name and renamed over the old one.  Callers hold g_tune_mu.
-const char* const kTuneFormat = "pyraft_amd tuning cache 3: backprojection variants x6, angle groups, radon shapes";
+const char* const kTuneFormat = "pyraft_amd tuning cache 4: backprojection variants x6 (paired), angle groups, radon shapes";
 bool g_tune_loaded = false;
 
 std::string tune_cache_path() {
@@ -506,6 +506,8 @@ struct GraphEntry {
   hipGraphExec_t exec = nullptr;
 };
 
+constexpr long long SS_BATCH_PAIR_TILES = 2048;
+
 int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace
@@ -597,6 +599,22 @@ int build_launch(raft_ss_batch* b, BatchLaunch& L, int kind, int S, int bsub, in
     if (S > 0) subset_range(p.g.nangles, S, bsub, &j0, &j1);
     blocks += ss_radon_blocks(p.nwaves, j0, j1);
   }
+  // Planes of the backprojection's tiles: whole ranges as the per-plan launch takes them.
+  // Subset ranges are short, so a block's time is latency and fewer blocks cost more than
+  // the planes save: two planes from SS_BATCH_PAIR_TILES tiles on.  An OSEM call of 8
+  // subsets: 12 slices of 261^2 to 1021^2 (4900 paired tiles) 1531 us with two planes and
+  // 1650 with one, 2 slices of 556^2 x 1242 (650 tiles) 689 and 629.
+  auto bp_planes = [&](const raft_ss_plan& p, int j0, int j1, bool pairs) {
+    if (mode == SS_BP_PLAIN && j0 == 0 && j1 == p.g.nangles) return ss_bp_planes(p.dev(v), j0, j1);
+    return pairs && p.bp_stage_v(v, 2) > 0 ? 2 : 1;
+  };
+  bool pairs = true;
+  if (kind == SS_KIND_BP) {
+    long long tiles = 0;
+    for (int i = 0; i < b->nslices; ++i)
+      if (b->variant[i] == v) tiles += ss_bp_tiles(b->plan(i).g.n, v, 2);
+    pairs = tiles >= SS_BATCH_PAIR_TILES;
+  }
   const bool radon = kind == SS_KIND_RADON || kind == SS_KIND_RADON_FINISH;
   L.slabs = radon && blocks < SS_RADON_SLAB_BLOCKS;
   L.part_floats = 0;
@@ -614,6 +632,7 @@ int build_launch(raft_ss_batch* b, BatchLaunch& L, int kind, int S, int bsub, in
     k.e.slab_rows = n;
     k.e.part_off = 0;
     k.e.which = SS_GATHER_BOTH;
+    k.e.planes = kind == SS_KIND_BP ? bp_planes(p, j0, j1, pairs) : 1;
     if (kind == SS_KIND_GATHER && S > 0) {  // a subset's gather: the layouts its angles read
       k.e.which = 0;
       for (int j = j0; j < j1; ++j) k.e.which |= p.h_angles[j].branch_a ? SS_GATHER_A : SS_GATHER_B;
@@ -648,7 +667,7 @@ int build_launch(raft_ss_batch* b, BatchLaunch& L, int kind, int S, int bsub, in
         break;
       default:  // SS_KIND_BP, only the slices of variant v
         if (b->variant[i] != v) continue;
-        k.items = j1 > j0 ? ss_bp_tiles(n, v) : 0;
+        k.items = j1 > j0 ? ss_bp_tiles(n, v, k.e.planes) : 0;
         k.cost = (double)(j1 - j0) * kSSBpRows[v];
         break;
     }
@@ -754,6 +773,8 @@ int run_body(raft_ss_batch* b, bool graph, const std::string& key, hipStream_t u
 
 }  // namespace
 
+static constexpr int kBatchVariant = 1;  // 2 pixel rows per thread, 2048 staged pairs
+
 extern "C" int raft_ss_batch_create(raft_ss_batch** out, int nslices, const int* n, const int* nrays,
                                     const int* nangles, const double* img_corners, const double* sino_corners,
                                     void* stream) {
@@ -785,7 +806,12 @@ extern "C" int raft_ss_batch_create(raft_ss_batch** out, int nslices, const int*
       it = by_geom.emplace(key, std::shared_ptr<raft_ss_plan>(p, raft_ss_plan_destroy)).first;
     }
     b->plans[i] = it->second;
-    b->variant[i] = it->second->bp_variant;
+    // Batched launches have no angle groups, and their OSEM ranges are short: images of up to
+    // 1024^2 start from the 2-rows-per-thread tiles, twice the blocks (12 slices of 261^2 to
+    // 1021^2, 8 subsets: 1531 us an iteration against 1675 with 4 rows, whole-range
+    // backprojection 333 against 418); one variant for all is one launch for all.
+    const raft_ss_plan& pl = *it->second;
+    b->variant[i] = pl.half_turn && n[i] <= 1024 && pl.bp_angles_v[kBatchVariant] > 0 ? kBatchVariant : pl.bp_variant;
     // 256-byte aligned slices in the packed buffers
     b->img_off[i] = b->img_total;
     b->img_total = align_up(b->img_total + (int64_t)n[i] * n[i], 64);
@@ -1076,9 +1102,10 @@ extern "C" int raft_ss_batch_tune(raft_ss_batch* b, int reps, int flags, void* s
         sl.sino_off = b->sino_off[i];
         sl.lay_off = b->lay_off[i];
         SSBatchEntry e{(int)h.size(), 0, std::min(sl.p.g.nangles, 360), (int)total};
+        e.planes = ss_bp_planes(sl.p, e.j0, e.j1);
         h.push_back(sl);
         L.entries.push_back(e);
-        total += ss_bp_tiles(sl.p.g.n, v);
+        total += ss_bp_tiles(sl.p.g.n, v, e.planes);
       }
       L.total = (int)total;
       L.grid = ss_batch_grid(SS_KIND_BP, v, SS_BP_PLAIN, L.total);

@@ -87,6 +87,15 @@ struct raft_ss_plan {
   bool bp_variant_fixed = false;  // set by raft_ss_plan_set_bp_variant: no per-range tuning
   int bp_window_v[SS_BP_NVARIANTS] = {0};  // per backprojection variant: staged window
   int bp_angles_v[SS_BP_NVARIANTS] = {0};  //   and angles per stage (0: not runnable)
+  // the grids map onto themselves under a half turn; and the angles under theta -> pi - theta
+  bool half_turn = false, mirror = false;
+  // angles per stage of the backprojection with `planes` planes (0: not available)
+  int bp_stage_v(int v, int planes) const {
+    if (!half_turn || (planes == 4 && !mirror) || bp_angles_v[v] <= 0) return 0;
+    // whole batches of the staging loop (ss_bp_stage) where they fit
+    const int j = std::min(64, kSSBpStage[v] / planes / bp_window_v[v]);
+    return j >= SS_BP_STAGE_BATCH ? j / SS_BP_STAGE_BATCH * SS_BP_STAGE_BATCH : j;
+  }
   int rt_variant = -1;                     // pixel-driven transpose: tile variant (-1: line form)
   int rt_window_v[SS_BP_NVARIANTS] = {0};  //   its staged window and angles per stage per variant
   int rt_angles_v[SS_BP_NVARIANTS] = {0};
@@ -113,6 +122,8 @@ struct raft_ss_plan {
     p.bp_variant = v;
     p.bp_window = bp_window_v[v];
     p.bp_angles = bp_angles_v[v];
+    p.bp_pair = bp_stage_v(v, 2);
+    p.bp_quad = bp_stage_v(v, 4);
     p.radon_slab_rows = 0;
     p.radon_shape = 0;
     p.rt_variant = rt_variant >= 0 ? rt_variant : 0;

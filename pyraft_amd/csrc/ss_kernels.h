@@ -28,6 +28,7 @@ enum { SS_BP_PLAIN = 0, SS_BP_EM_UPDATE = 1, SS_BP_PARTIAL = 2 };
 #define SS_BP_NVARIANTS 6
 #define SS_BP_DEFAULT_VARIANT 0
 #define SS_RT_DEFAULT_VARIANT 3  // pixel-driven transpose tile (4 rows per thread, 2048 staged pairs)
+#define SS_BP_STAGE_BATCH 16  // angles that a block's four waves stage in one batch of loads
 static const int kSSBpRows[SS_BP_NVARIANTS] = {4, 2, 8, 4, 2, 8};
 static const int kSSBpStage[SS_BP_NVARIANTS] = {4096, 2048, 4096, 2048, 4096, 2048};
 
@@ -44,6 +45,7 @@ struct SSDevPlan {
   int bp_variant;          // index into kSSBpRows / kSSBpStage
   int bp_window;           // rays staged per angle per pixel tile (for bp_variant)
   int bp_angles;           // angles per LDS stage (for bp_variant)
+  int bp_pair, bp_quad;    // angles per LDS stage with 2 and 4 planes (0: not available, see ss_bp_item)
   int radon_slab_rows;     // Radon: sample rows per slab (n: no division; 0: the default rule)
   int radon_shape;         // Radon: block shape (0: 4096 staged records, 32-row chunks; 1: 4864, 40)
   // exact transpose, pixel-driven form: tile variant (the backprojection's shapes), rays
@@ -70,6 +72,7 @@ struct SSBatchEntry {
   int nslab, slab_rows;
   int64_t part_off;
   int which;  // gather launches: the layouts to build (SS_GATHER_*), those angles j0..j1-1 read
+  int planes; // backprojection launches: the planes of the entry's tiles (ss_bp_item)
 };
 struct SSBatchLaunch {
   const SSBatchSlice* slices;  // device
@@ -136,14 +139,22 @@ struct SSEmUpdateArgs {
   float* x;            // image updated in place
   const float* weight; // BP_b(1)
 };
-// A launch of fewer than SS_BP_SPLIT_TILES pixel tiles (a small image) divides its angles
-// into groups taken by separate blocks, at least SS_BP_GROUP_ANGLES angles each, so that
-// the launch has about SS_BP_SPLIT_BLOCKS blocks; each group writes a partial image
-// (unscaled sums) to scratch and a finishing pass adds the groups in group order, scales by
-// dtheta and stores or applies the EM update.  ss_bp_groups: the group count (1: no
-// division); ss_bp_scratch: the bytes of the partial images (0 when not divided).
-#define SS_BP_SPLIT_TILES 512
-#define SS_BP_SPLIT_BLOCKS 1024
+// A launch may divide its angles into groups taken by separate blocks, at least
+// SS_BP_GROUP_ANGLES angles each; every group writes a partial image (unscaled sums) to
+// scratch and a finishing pass adds the groups in group order, scales by dtheta and stores
+// or applies the EM update.  More blocks even out the CUs' work (a launch of few tiles
+// leaves CUs idle; one round of equal tiles ends when the slowest CU does), more groups
+// write and read more partial images: with T tiles the first costs ~ total / (G T), the
+// second ~ G images, so G = SS_BP_GROUP_SCALE sqrt(SS_BP_ROUND_BLOCKS angles / T), the
+// blocks of one round over the chip counted as 1024.  The scale is fitted to full-range
+// launches (us with 1 / 4 / 8 / 16 / 32 groups, variant 0): 2048^2 x 1500 680 / 621 / 596 /
+// 630 / 734; 1448^2 x 720 288 / 195 / 179 / 184 / 251; 1024^2 x 720 285 / 145 / 104 / 102 /
+// 120; 768^2 x 500 203 / 105 / 65 / 57 / 66; 512^2 x 720 312 / 143 / 79 / 54 / 48; the rule
+// takes 8, 8, 12, 13, 24.
+// ss_bp_groups: the group count (1: no division); ss_bp_scratch: the bytes of the partial
+// images (0 when not divided).
+#define SS_BP_GROUP_SCALE 0.22
+#define SS_BP_ROUND_BLOCKS 1024
 #define SS_BP_GROUP_ANGLES 8
 int ss_bp_groups(const SSDevPlan& p, int j0, int j1, int nslices);
 size_t ss_bp_scratch(const SSDevPlan& p, int j0, int j1, int nslices);
@@ -161,7 +172,8 @@ hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int
 // ---- batched forms (items: gather = SS_GATHER_TILE^2 tiles; radon = 64-ray groups x blocks of
 //      8 angles x row slabs; finish = 256 rays of an entry; fixup = irregular rays; bp = pixel
 //      tiles of the variant; transpose = 32x32 tiles)
-int ss_bp_tiles(int n, int variant);
+int ss_bp_planes(const SSDevPlan& p, int j0, int j1);
+int ss_bp_tiles(int n, int variant, int planes);
 // gather tile side for a batch of images with sides n[0..count): SS_GATHER_TILE when the
 // batch has at least 1024 such tiles, else 32 (items are tiles of that side)
 int ss_batch_gather_tile(const int* n, int count);

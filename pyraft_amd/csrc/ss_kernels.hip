@@ -941,9 +941,11 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
 
 #define BP_TILE_W 32
 
-struct BPAngle {
-  float f0, b, c;
-  int flag;  // 0 outside, 1 interior, 2 boundary
+typedef float ss_f32x4 __attribute__((ext_vector_type(4)));
+
+struct alignas(16) BPAngle {
+  float f0, b, c;  // read together with flag by one 16-byte LDS read
+  int flag;        // 0 outside, 1 interior, 2 boundary
   int base;
   int pad0, pad1, pad2;
 };
@@ -955,41 +957,178 @@ __device__ __forceinline__ int ss_bp_exact_valid(const SSDevPlan& p, int j, int 
 
 template <int STAGE>
 struct SSBpLds {
-  float2 win[STAGE];  // per staged ray w: (value - w * difference, difference to the next ray)
+  // per staged ray w the PL records (value - w * difference, difference to the next ray),
+  // in pairs of planes; planes 2, 3 in the second half
+  alignas(16) float2 win[STAGE];
   BPAngle par[64];
 };
 
+// raw buffer load of one float at a byte offset; an offset past the buffer (also a negative
+// one, as unsigned) reads 0
+__device__ float ss_raw_load_f32(__amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset,
+                                 int aux) __asm("llvm.amdgcn.raw.ptr.buffer.load.f32");
+
+// the value of the next lane (lane 63: 0)
+__device__ __forceinline__ float ss_next_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
+}
+
+// Column of a lane in its 32-pixel tile row.  A 16-byte LDS read serves 16 lanes of a half
+// wave per pass, the lanes 0-3, 12-15, 20-27 and then the others; giving each of the two
+// sets 16 neighbouring columns keeps a pass within 16 neighbouring records, so that no two
+// of them share a bank (pixels are at most one ray apart).
+__device__ __forceinline__ int ss_bp_column(int lane) {
+  const int q = (lane >> 2) & 7;
+  return ((0x73261540 >> (4 * q)) & 7) * 4 + (lane & 3);
+}
+
+// The sinogram row that the mirrored planes of angle j read (PL = 4): that of the angle
+// pi - theta_j, A - j on the grid [0, pi); for theta = 0 its own row reversed.
+struct SSBpMirror {
+  int row;
+  bool flip;
+};
+__device__ __forceinline__ SSBpMirror ss_bp_mirror(int j, int A) { return SSBpMirror{j > 0 ? A - j : 0, j == 0}; }
+
+#define BP_BATCH (SS_BP_STAGE_BATCH / 4)  // angle windows whose loads a wave issues together
+
+// One stage's windows of the angles jb + wv, jb + wv + 4, ... < jb + nj: the records w in
+// [0, W) of each, ray base + w of every plane (lane js + jj holds base).  The loads of BP_BATCH windows are issued
+// before the first is used, so that a stage waits for memory once per BP_BATCH windows and
+// not once per window; a record's second ray comes from the next lane (63 records a pass);
+// rays off the detector read 0 through the buffer's range check.
+template <int PL, int STAGE>
+__device__ __forceinline__ void ss_bp_stage(const float* __restrict__ sl, int R, int A, int W, int jb, int nj, int wv,
+                                            int lane, int base, int js, float2* __restrict__ win) {
+  for (int w0 = 0; w0 < W; w0 += SS_WAVE - 1) {
+    const int w = w0 + lane;
+    const float fw = -(float)w;
+    for (int j4 = wv; j4 < nj; j4 += 4 * BP_BATCH) {
+      float v[BP_BATCH][PL];
+#pragma unroll
+      for (int b = 0; b < BP_BATCH; ++b) {
+        const int jj = min(j4 + 4 * b, nj - 1);  // past the last: its window again, not stored
+        const int ray = __builtin_amdgcn_readlane(base, js + jj) + w;
+        // the whole offset in the register, so that the range check sees a ray below 0
+        int fwd = 4 * ray, rev = 4 * (R - 1) - 4 * ray;
+        __asm__ volatile("" : "+v"(fwd), "+v"(rev));
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(sl + (size_t)(jb + jj) * R), (short)0, R * (int)sizeof(float), SS_RSRC_DWORD3);
+        v[b][0] = ss_raw_load_f32(rs, fwd, 0, 0);
+        if (PL >= 2) v[b][PL >= 2 ? 1 : 0] = ss_raw_load_f32(rs, rev, 0, 0);
+        if (PL == 4) {
+          const SSBpMirror m = ss_bp_mirror(jb + jj, A);
+          const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+              (void*)(sl + (size_t)m.row * R), (short)0, R * (int)sizeof(float), SS_RSRC_DWORD3);
+          v[b][PL == 4 ? 2 : 0] = ss_raw_load_f32(rm, m.flip ? rev : fwd, 0, 0);
+          v[b][PL == 4 ? 3 : 0] = ss_raw_load_f32(rm, m.flip ? fwd : rev, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < BP_BATCH; ++b) {
+        const int jj = j4 + 4 * b;
+        // (v0 - w d, d): the value at u in [w, w + 1) is then fma(u, d, first), so the
+        // interpolation needs no fraction of u
+        float f[PL], d[PL];
+#pragma unroll
+        for (int z = 0; z < PL; ++z) {  // every lane takes part in the lane shift
+          d[z] = ss_next_lane(v[b][z]) - v[b][z];
+          f[z] = fmaf(fw, d[z], v[b][z]);
+        }
+        if (jj < nj && lane < SS_WAVE - 1 && w < W) {
+          if (PL == 1) {
+            win[jj * W + w] = make_float2(f[0], d[0]);
+          } else {
+            // planes 2, 3 in a window array of their own: neighbouring rays 16 bytes apart
+            ss_f32x4* dst = reinterpret_cast<ss_f32x4*>(win) + jj * W + w;
+#pragma unroll
+            for (int z = 0; z + 1 < PL; z += 2)
+              dst[z / 2 * (STAGE / 4)] = ss_f32x4{f[z], d[z], f[z + 1], d[z + 1]};
+          }
+        }
+      }
+    }
+  }
+}
+
+// The values of the planes at ray offset u of one window.
+template <int PL, int STAGE>
+__device__ __forceinline__ void ss_bp_lerp(const float2* __restrict__ wrow, float u, float (&val)[PL]) {
+  if (PL == 1) {
+    const float2 t = wrow[(int)u];
+    val[0] = fmaf(u, t.y, t.x);
+  } else {
+    const ss_f32x4* t = reinterpret_cast<const ss_f32x4*>(wrow) + (int)u;
+#pragma unroll
+    for (int z = 0; z + 1 < PL; z += 2) {
+      const ss_f32x4 q = t[z / 2 * (STAGE / 4)];
+      val[z] = fmaf(u, q.y, q.x);
+      val[z + 1] = fmaf(u, q.w, q.z);
+    }
+  }
+}
+
+// the pixel of plane z that goes with pixel (row, col) of plane 0, and whether it is stored
+// (not where it coincides with another plane's pixel, on the middle row or column)
+template <int PL>
+__device__ __forceinline__ bool ss_bp_plane_pixel(int z, int n, int row, int col, int* zr, int* zc) {
+  *zr = (z == 1 || z == 3) ? n - 1 - row : row;
+  *zc = (z == 1 || z == 2) ? n - 1 - col : col;
+  if (PL == 1) return row < n && col < n;
+  if (PL == 2) return 2 * row + z <= n - 1 && col < n;
+  const int mr = z == 1 || z == 3, mc = z == 1 || z == 2;
+  return 2 * row + mr <= n - 1 && 2 * col + mc <= n - 1;
+}
+
 // One pixel tile [c0, c0+32) x [r0, r0+8*ROWS) over angles [j0, j1).  sl points at this
 // slice's angle-major sinogram; out (plain) or x/weight (EM update) at its image.
-template <int MODE, int ROWS, int STAGE>
+//
+// The planes of the tile share each pixel's ray coordinate, its conversion and its address;
+// only the interpolation and the sum are their own, and a ray's records lie together, so
+// that one 16-byte LDS read returns two of them:
+//   PL = 1  the pixel alone.
+//   PL = 2  (SSDevPlan::bp_pair) on a grid symmetric about the rotation axis, pixel
+//           (n-1-r, n-1-c) has the coordinate R - 1 - u of pixel (r, c)'s u: a window
+//           holds for each ray also the record of ray R - 1 - ray.  Tiles cover the rows
+//           r <= n-1-r.
+//   PL = 4  (SSDevPlan::bp_quad) over all angles of a symmetric grid [0, pi): at the angle
+//           pi - theta, pixel (r, n-1-c) has pixel (r, c)'s coordinate, and (n-1-r, c) its
+//           reverse; a window also holds the rows of that angle.  Tiles cover a quadrant.
+// Each pixel's range test is its own (a mirrored pixel re-evaluates its own FP64 expression).
+// VALU instructions per update in the loop: 5 / 3.5 / 2.75.
+template <int MODE, int ROWS, int STAGE, int PL>
 __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __restrict__ sl, int j0, int j1, int c0,
                                            int r0, float* __restrict__ out, float* __restrict__ xs,
                                            const float* __restrict__ ws, SSBpLds<STAGE>& lds) {
-  const int n = p.g.n, R = p.g.nrays;
+  const int n = p.g.n, R = p.g.nrays, A = p.g.nangles;
   const int W = p.bp_window;
-  const int J = p.bp_angles;
+  const int J = PL == 4 ? p.bp_quad : (PL == 2 ? p.bp_pair : p.bp_angles);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tx = tid & 31, ty = tid >> 5;
+  const int tx = PL == 1 ? tid & 31 : ss_bp_column(tid), ty = tid >> 5;
   const int col = c0 + tx;
   constexpr int TH = 8 * ROWS;
-  float acc[ROWS];
+  float acc[ROWS][PL];
   float fty[ROWS];
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
-    acc[i] = 0.f;
+#pragma unroll
+    for (int z = 0; z < PL; ++z) acc[i][z] = 0.f;
     fty[i] = (float)(ty + 8 * i);
   }
   const float ftx = (float)tx;
   const float lo_rel_eps = 1e-3f;
 
-  for (int jb = j0; jb < j1; jb += J) {
-    const int nj = min(J, j1 - jb);
-    // every wave: lane l holds the parameters of angle jb + l (J <= 64)
+  // Parameters of up to 64 angles at a time: lane l of every wave holds those of angle
+  // ja + l, for as many whole stages as fit (in FP64: redone per stage they were 7% of the
+  // kernel's instructions).
+  const int JP = SS_WAVE / J * J;
+  for (int ja = j0; ja < j1; ja += JP) {
+    const int np = min(JP, j1 - ja);
     BPAngle q{0.f, 0.f, 0.f, 0, 0, 0, 0, 0};
-    if (lane < nj) {
-      const SSAngle& a = p.angles[jb + lane];
+    if (lane < np) {
+      const SSAngle& a = p.angles[ja + lane];
       const double U = a.bp_a + (double)c0 * a.bp_b + (double)r0 * a.bp_c;
       const double ec = (double)(BP_TILE_W - 1) * a.bp_b, er = (double)(TH - 1) * a.bp_c;
       const double umin = U + fmin(0.0, ec) + fmin(0.0, er);
@@ -1007,108 +1146,101 @@ __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __re
         q.flag = 2;
       q.base = (int)base;
     }
-    // a stage whose angles are all interior for this tile runs without predicates
-    const bool mixed = __ballot(lane < nj && q.flag != 1) != 0ull;
-    __syncthreads();  // the previous stage (or item) is done with win / par
-    if (wv == 0) {  // the used fields only (whole-struct copies kept the padding in scratch)
-      lds.par[lane].f0 = q.f0;
-      lds.par[lane].b = q.b;
-      lds.par[lane].c = q.c;
-      lds.par[lane].flag = q.flag;
-      lds.par[lane].base = q.base;
-    }
-    // staging: wave wv fills the windows of angles wv, wv+4, ...; base is at least one
-    // ray below the tile's lowest U, so every pixel has u >= 1 and (int)u < W - 1
-    for (int jj = wv; jj < nj; jj += 4) {
-      const int fl = __builtin_amdgcn_readlane(q.flag, jj);
-      const int bs = __builtin_amdgcn_readlane(q.base, jj);
-      const float* row = sl + (size_t)(jb + jj) * R;
-      for (int w = lane; w < W; w += 64) {
-        const int ray = bs + w;
-        float v0 = 0.f, v1 = 0.f;
-        if (fl != 0) {
-          if ((unsigned)ray < (unsigned)R) v0 = row[ray];
-          if ((unsigned)(ray + 1) < (unsigned)R) v1 = row[ray + 1];
-        }
-        // (v0 - w d, d): the value at u in [w, w + 1) is then fma(u, d, first), so the
-        // interpolation needs no fraction of u
-        const float d = v1 - v0;
-        lds.win[jj * W + w] = make_float2(fmaf(-(float)w, d, v0), d);
+    // the angles that are interior for this tile run without predicates
+    const unsigned long long interior = __ballot(lane < np && q.flag == 1);
+    for (int js = 0; js < np; js += J) {
+      const int jb = ja + js, nj = min(J, np - js);
+      const bool mixed = __popcll(interior >> js & (~0ull >> (SS_WAVE - nj))) != nj;
+      __syncthreads();  // the previous stage (or item) is done with win / par
+      if (js == 0 && wv == 0) {  // the used fields only (whole-struct copies kept the padding in scratch)
+        lds.par[lane].f0 = q.f0;
+        lds.par[lane].b = q.b;
+        lds.par[lane].c = q.c;
+        lds.par[lane].flag = q.flag;
+        lds.par[lane].base = q.base;
       }
-    }
-    __syncthreads();
-    if (!mixed) {
+      // base is at least one ray below the tile's lowest U, so every pixel has u >= 1 and
+      // (int)u < W - 1
+      ss_bp_stage<PL, STAGE>(sl, R, A, W, jb, nj, wv, lane, q.base, js, lds.win);
+      __syncthreads();
+      // one angle's updates from its window: u >= 1, so truncation is the floor
+      auto add = [&](const ss_f32x4& par, const float2* wrow) {
+        const float t0 = fmaf(ftx, par.y, par.x);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+          float val[PL];
+          ss_bp_lerp<PL, STAGE>(wrow, fmaf(fty[i], par.z, t0), val);
+#pragma unroll
+          for (int z = 0; z < PL; ++z) acc[i][z] += val[z];
+        }
+      };
+      constexpr int RW = PL == 1 ? 1 : 2;  // records of a ray in a window array
+      if (!mixed) {
 #pragma unroll 2
-      for (int jj = 0; jj < nj; ++jj) {
-        const float f0 = lds.par[jj].f0, pb = lds.par[jj].b, pc = lds.par[jj].c;
-        const float2* wrow = lds.win + jj * W;
-        const float t0 = fmaf(ftx, pb, f0);
-        // u >= 1 here, so truncation is the floor
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-          const float u = fmaf(fty[i], pc, t0);
-          const float2 t = wrow[(int)u];
-          acc[i] += fmaf(u, t.y, t.x);
-        }
-      }
-    } else {
-      for (int jj = 0; jj < nj; ++jj) {
-        BPAngle qa;
-        qa.f0 = lds.par[jj].f0;
-        qa.b = lds.par[jj].b;
-        qa.c = lds.par[jj].c;
-        qa.flag = lds.par[jj].flag;
-        qa.base = lds.par[jj].base;
-        const int flag = __builtin_amdgcn_readfirstlane(qa.flag);
-        if (flag == 0) continue;
-        const float2* wrow = lds.win + jj * W;
-        const float t0 = fmaf(ftx, qa.b, qa.f0);
-        float us[ROWS], vals[ROWS];
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-          us[i] = fmaf(fty[i], qa.c, t0);
-          const float2 t = wrow[(int)us[i]];
-          vals[i] = fmaf(us[i], t.y, t.x);
-        }
-        if (flag == 2) {
-          // boundary tile: per-pixel 0 <= m <= R-2 test; pixels within 1e-3 bins of an
-          // edge take the reference's FP64 expression.  The result is an integer mask
-          // applied by select, keeping the divergent region free of value phis.
-          const float lo_rel = (float)(-qa.base), hi_rel = (float)(R - 1 - qa.base);
+        for (int jj = 0; jj < nj; ++jj)
+          add(*reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]), lds.win + jj * RW * W);  // f0, b, c, flag
+      } else {
+        for (int jj = 0; jj < nj; ++jj) {
+          const ss_f32x4 par = *reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]);
+          const float2* wrow = lds.win + jj * RW * W;
+          const int flag = __builtin_amdgcn_readfirstlane(__float_as_int(par.w));
+          if (flag == 0) continue;
+          if (flag == 1) {
+            add(par, wrow);
+            continue;
+          }
+          // boundary tile: per-pixel 0 <= m <= R-2 test; pixels within 1e-3 bins of an edge
+          // take the reference's FP64 expression.  The result is an integer mask applied by
+          // select, keeping the divergent region free of value phis.
+          const int base = lds.par[js + jj].base;
+          const float t0 = fmaf(ftx, par.y, par.x);
+          const float lo_rel = (float)(-base), hi_rel = (float)(R - 1 - base);
           int keep = 0;
 #pragma unroll
           for (int i = 0; i < ROWS; ++i) {
-            const float u = us[i];
+            const float u = fmaf(fty[i], par.z, t0);
             const bool inside = (u > lo_rel + lo_rel_eps) && (u < hi_rel - lo_rel_eps);
             const bool outside = (u < lo_rel - lo_rel_eps) || (u > hi_rel + lo_rel_eps);
-            int ok = inside ? 1 : 0;
-            if (!inside && !outside) ok = ss_bp_exact_valid(p, jb + jj, r0 + ty + 8 * i, col);
-            keep |= ok << i;
+            int ok = inside ? (1 << PL) - 1 : 0;
+            if (!inside && !outside) {
+              const int jm = PL == 4 ? ss_bp_mirror(jb + jj, A).row : jb + jj;
+              for (int z = 0; z < PL; ++z) {
+                int zr, zc;
+                (void)ss_bp_plane_pixel<PL>(z, n, r0 + ty + 8 * i, col, &zr, &zc);
+                ok |= ss_bp_exact_valid(p, z >= 2 ? jm : jb + jj, zr, zc) << z;
+              }
+            }
+            keep |= ok << (PL * i);
           }
 #pragma unroll
-          for (int i = 0; i < ROWS; ++i) vals[i] = ((keep >> i) & 1) ? vals[i] : 0.f;
-        }
+          for (int i = 0; i < ROWS; ++i) {
+            float val[PL];
+            ss_bp_lerp<PL, STAGE>(wrow, fmaf(fty[i], par.z, t0), val);
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i) acc[i] += vals[i];
+            for (int z = 0; z < PL; ++z) acc[i][z] += ((keep >> (PL * i + z)) & 1) ? val[z] : 0.f;
+          }
+        }
       }
     }
   }
-  if (col >= n) return;
   const float dth = (float)p.g.dth;
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
-    const int row = r0 + ty + 8 * i;
-    if (row >= n) continue;
-    const size_t idx = (size_t)row * n + col;
-    const float bp = acc[i] * dth;
-    if (MODE == SS_BP_PLAIN) {
-      out[idx] = bp;
-    } else if (MODE == SS_BP_PARTIAL) {
-      out[idx] = acc[i];
-    } else {
-      const float wgt = ws[idx];
-      const float x = xs[idx];
-      xs[idx] = wgt > 0.f ? x * bp / wgt : x;
+#pragma unroll
+    for (int z = 0; z < PL; ++z) {
+      int zr, zc;
+      if (!ss_bp_plane_pixel<PL>(z, n, r0 + ty + 8 * i, col, &zr, &zc)) continue;
+      const size_t idx = (size_t)zr * n + zc;
+      const float bp = acc[i][z] * dth;
+      if (MODE == SS_BP_PLAIN) {
+        out[idx] = bp;
+      } else if (MODE == SS_BP_PARTIAL) {
+        out[idx] = acc[i][z];
+      } else {
+        const float wgt = ws[idx];
+        const float x = xs[idx];
+        xs[idx] = wgt > 0.f ? x * bp / wgt : x;
+      }
     }
   }
 }
@@ -1116,7 +1248,7 @@ __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __re
 // blockIdx.z = slice * ngroups + g.  SS_BP_PARTIAL: group g takes angles
 // [j0 + g*nj/ngroups, j0 + (g+1)*nj/ngroups) and writes its unscaled sums to
 // out[slice][g][n][n]; the other modes have ngroups = 1.
-template <int MODE, int ROWS, int STAGE>
+template <int MODE, int ROWS, int STAGE, int PL>
 __global__ __launch_bounds__(256) void k_backprojection(SSDevPlan p, const float* __restrict__ sinoT, int j0, int j1,
                                                         int ngroups, float* __restrict__ out, SSEmUpdateArgs em) {
   __shared__ SSBpLds<STAGE> lds;
@@ -1132,7 +1264,7 @@ __global__ __launch_bounds__(256) void k_backprojection(SSDevPlan p, const float
     jb = j0 + (int)((g + 1) * nj / ngroups);
   }
   float* dst = MODE == SS_BP_PLAIN ? out + io : (MODE == SS_BP_PARTIAL ? out + (slice * ngroups + g) * per : nullptr);
-  ss_bp_item<MODE, ROWS, STAGE>(p, sinoT + so, ja, jb, blockIdx.x * BP_TILE_W, blockIdx.y * 8 * ROWS, dst,
+  ss_bp_item<MODE, ROWS, STAGE, PL>(p, sinoT + so, ja, jb, blockIdx.x * BP_TILE_W, blockIdx.y * 8 * ROWS, dst,
                                 MODE == SS_BP_EM_UPDATE ? em.x + io : nullptr,
                                 MODE == SS_BP_EM_UPDATE ? em.weight + io : nullptr, lds);
 }
@@ -1148,6 +1280,7 @@ __global__ __launch_bounds__(256) void k_bp_groups_finish(const float* __restric
   const size_t slice = blockIdx.y;
   const float* src = part + slice * ngroups * per + idx;
   float sum = 0.f;
+#pragma unroll 8
   for (int g = 0; g < ngroups; ++g) sum += src[(size_t)g * per];
   const float bp = sum * dth;
   const size_t o = slice * per + idx;
@@ -1160,17 +1293,28 @@ __global__ __launch_bounds__(256) void k_bp_groups_finish(const float* __restric
   }
 }
 
-int ss_bp_tiles(int n, int variant) {
+// Planes of a backprojection over angles [j0, j1) (see ss_bp_item)
+int ss_bp_planes(const SSDevPlan& p, int j0, int j1) {
+  if (p.bp_quad > 0 && j0 == 0 && j1 == p.g.nangles) return 4;
+  return p.bp_pair > 0 ? 2 : 1;
+}
+
+// columns and rows that the tiles of an n x n image cover
+static int ss_bp_cols(int n, int planes) { return planes == 4 ? (n + 1) / 2 : n; }
+static int ss_bp_rows(int n, int planes) { return planes >= 2 ? (n + 1) / 2 : n; }
+static int ss_bp_tile_cols(int n, int planes) { return (ss_bp_cols(n, planes) + BP_TILE_W - 1) / BP_TILE_W; }
+
+int ss_bp_tiles(int n, int variant, int planes) {
   const int th = 8 * kSSBpRows[variant];
-  return ((n + BP_TILE_W - 1) / BP_TILE_W) * ((n + th - 1) / th);
+  return ss_bp_tile_cols(n, planes) * ((ss_bp_rows(n, planes) + th - 1) / th);
 }
 
 int ss_bp_groups(const SSDevPlan& p, int j0, int j1, int nslices) {
-  const long long tiles = (long long)ss_bp_tiles(p.g.n, p.bp_variant) * std::max(nslices, 1);
+  const long long tiles = (long long)ss_bp_tiles(p.g.n, p.bp_variant, ss_bp_planes(p, j0, j1)) * std::max(nslices, 1);
   const int nj = j1 - j0;
-  if (tiles >= SS_BP_SPLIT_TILES || nj < 2 * SS_BP_GROUP_ANGLES) return 1;
-  const long long want = (SS_BP_SPLIT_BLOCKS + tiles - 1) / tiles;
-  return (int)std::max(1LL, std::min(want, (long long)(nj / SS_BP_GROUP_ANGLES)));
+  if (tiles <= 0 || nj < 2 * SS_BP_GROUP_ANGLES) return 1;
+  const double g = SS_BP_GROUP_SCALE * sqrt((double)SS_BP_ROUND_BLOCKS * nj / (double)tiles);
+  return (int)std::max(1.0, std::min(floor(g + 0.5), (double)(nj / SS_BP_GROUP_ANGLES)));
 }
 
 size_t ss_bp_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
@@ -1189,18 +1333,28 @@ hipError_t ss_launch_backprojection(const SSDevPlan& p, const float* sinoT, int 
   const int G = scratch ? ss_bp_groups(p, j0, j1, nslices) : 1;
   const int kmode = G > 1 ? SS_BP_PARTIAL : mode;
   float* kout = G > 1 ? scratch : out;
-  dim3 grid((n + BP_TILE_W - 1) / BP_TILE_W, (n + th - 1) / th, nslices * G);
-#define SS_BP_LAUNCH(V, ROWS, STAGE)                                                                               \
-  case V:                                                                                                          \
-    if (kmode == SS_BP_PLAIN)                                                                                      \
-      hipLaunchKernelGGL((k_backprojection<SS_BP_PLAIN, ROWS, STAGE>), grid, dim3(256), 0, stream, p, sinoT, j0,  \
-                         j1, 1, kout, em);                                                                         \
-    else if (kmode == SS_BP_PARTIAL)                                                                               \
-      hipLaunchKernelGGL((k_backprojection<SS_BP_PARTIAL, ROWS, STAGE>), grid, dim3(256), 0, stream, p, sinoT, j0, \
-                         j1, G, kout, em);                                                                         \
-    else                                                                                                           \
-      hipLaunchKernelGGL((k_backprojection<SS_BP_EM_UPDATE, ROWS, STAGE>), grid, dim3(256), 0, stream, p, sinoT,  \
-                         j0, j1, 1, kout, em);                                                                     \
+  const int planes = ss_bp_planes(p, j0, j1);
+  dim3 grid(ss_bp_tile_cols(n, planes), (ss_bp_rows(n, planes) + th - 1) / th, nslices * G);
+#define SS_BP_LAUNCH_PL(ROWS, STAGE, PL)                                                                          \
+  do {                                                                                                            \
+    if (kmode == SS_BP_PLAIN)                                                                                     \
+      hipLaunchKernelGGL((k_backprojection<SS_BP_PLAIN, ROWS, STAGE, PL>), grid, dim3(256), 0, stream, p, sinoT, \
+                         j0, j1, 1, kout, em);                                                                    \
+    else if (kmode == SS_BP_PARTIAL)                                                                              \
+      hipLaunchKernelGGL((k_backprojection<SS_BP_PARTIAL, ROWS, STAGE, PL>), grid, dim3(256), 0, stream, p,      \
+                         sinoT, j0, j1, G, kout, em);                                                             \
+    else                                                                                                          \
+      hipLaunchKernelGGL((k_backprojection<SS_BP_EM_UPDATE, ROWS, STAGE, PL>), grid, dim3(256), 0, stream, p,    \
+                         sinoT, j0, j1, 1, kout, em);                                                             \
+  } while (0)
+#define SS_BP_LAUNCH(V, ROWS, STAGE)     \
+  case V:                                \
+    if (planes == 4)                     \
+      SS_BP_LAUNCH_PL(ROWS, STAGE, 4);   \
+    else if (planes == 2)                \
+      SS_BP_LAUNCH_PL(ROWS, STAGE, 2);   \
+    else                                 \
+      SS_BP_LAUNCH_PL(ROWS, STAGE, 1);   \
     break;
   switch (p.bp_variant) {
     SS_BP_FOR_VARIANTS(SS_BP_LAUNCH)
@@ -1208,6 +1362,7 @@ hipError_t ss_launch_backprojection(const SSDevPlan& p, const float* sinoT, int 
       return hipErrorInvalidValue;
   }
 #undef SS_BP_LAUNCH
+#undef SS_BP_LAUNCH_PL
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || G == 1) return e;
   const size_t per = (size_t)n * n;
@@ -2369,6 +2524,7 @@ __device__ __forceinline__ SSBatchEntry ss_entry_of(const SSBatchLaunch& L, int 
   e.slab_rows = __builtin_amdgcn_readfirstlane(e.slab_rows);
   e.part_off = ss_rfl64(e.part_off);
   e.which = __builtin_amdgcn_readfirstlane(e.which);
+  e.planes = __builtin_amdgcn_readfirstlane(e.planes);
   return e;
 }
 
@@ -2506,13 +2662,20 @@ __global__ __launch_bounds__(256) void k_batch_bp(SSBatchLaunch L, const float* 
   for (int item = blockIdx.x; item < L.total; item += gridDim.x) {
     const SSBatchEntry e = ss_entry_of(L, item);
     const SSBatchSlice s = ss_uniform_copy(L.slices + e.slice);
-    const int tiles_x = (s.p.g.n + BP_TILE_W - 1) / BP_TILE_W;
+    const int planes = e.planes;  // uniform over the block; 4 only over whole ranges (SS_BP_PLAIN)
+    const int tiles_x = ((planes == 4 ? (s.p.g.n + 1) / 2 : s.p.g.n) + BP_TILE_W - 1) / BP_TILE_W;
     const int local = item - e.item0;
     const int ty = local / tiles_x, tx = local - ty * tiles_x;
-    ss_bp_item<MODE, ROWS, STAGE>(s.p, sinoT + s.sino_off, e.j0, e.j1, tx * BP_TILE_W, ty * TH,
-                                  MODE == SS_BP_PLAIN ? out + s.img_off : nullptr,
-                                  MODE == SS_BP_PLAIN ? nullptr : x + s.img_off,
-                                  MODE == SS_BP_PLAIN ? nullptr : weight + s.img_off, lds);
+    float* o = MODE == SS_BP_PLAIN ? out + s.img_off : nullptr;
+    float* xs = MODE == SS_BP_PLAIN ? nullptr : x + s.img_off;
+    const float* ws = MODE == SS_BP_PLAIN ? nullptr : weight + s.img_off;
+    if (MODE == SS_BP_PLAIN && planes == 4)
+      ss_bp_item<MODE, ROWS, STAGE, MODE == SS_BP_PLAIN ? 4 : 2>(s.p, sinoT + s.sino_off, e.j0, e.j1, tx * BP_TILE_W,
+                                                                 ty * TH, o, xs, ws, lds);
+    else if (planes == 2)
+      ss_bp_item<MODE, ROWS, STAGE, 2>(s.p, sinoT + s.sino_off, e.j0, e.j1, tx * BP_TILE_W, ty * TH, o, xs, ws, lds);
+    else
+      ss_bp_item<MODE, ROWS, STAGE, 1>(s.p, sinoT + s.sino_off, e.j0, e.j1, tx * BP_TILE_W, ty * TH, o, xs, ws, lds);
     __syncthreads();
   }
 }

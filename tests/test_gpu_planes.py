@@ -1,0 +1,52 @@
+"""Symmetric geometries, where one ray coordinate serves several pixels or rays: against the
+FP64 oracle at the edges of the form (odd and even sides, bins and angles, tiles and
+windows that end inside the image, the grids that only one of the symmetries fits)."""
+import math
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+REL = 1e-5  # the FP32 operators' bar against the oracle
+PI = math.pi
+
+# (n, R, A, sinogram corners): [0, pi) on the default grid has both symmetries, [0, 2 pi) and
+# a limited arc only the half turn, a shifted detector none
+GEO = [
+    (2, 2, 1, (0.0, 1.0, PI, -1.0)), (3, 2, 2, (0.0, 1.0, PI, -1.0)), (5, 7, 3, (0.0, 1.0, PI, -1.0)),
+    (31, 33, 8, (0.0, 1.0, PI, -1.0)), (32, 64, 9, (0.0, 1.0, PI, -1.0)), (33, 31, 16, (0.0, 1.0, PI, -1.0)),
+    (63, 65, 17, (0.0, 1.42, PI, -1.42)), (64, 63, 40, (0.0, 0.7, PI, -0.7)), (65, 128, 41, (0.0, 1.0, PI, -1.0)),
+    (97, 97, 66, (0.0, 1.0, PI, -1.0)), (130, 131, 47, (0.0, 1.0, PI, -1.0)), (96, 160, 65, (0.0, 1.0, 2 * PI, -1.0)),
+    (65, 65, 20, (0.0, 1.0, 2.0, -1.0)), (66, 90, 34, (0.1, 1.0, PI + 0.1, -1.0)), (67, 67, 33, (0.0, 1.03, PI, -0.97)),
+]
+
+
+def _rel(a, b):
+    return np.linalg.norm(np.asarray(a, np.float64) - b) / max(np.linalg.norm(b), 1e-300)
+
+
+def _geo(sc):
+    return dict(sino_tl=(sc[0], sc[1]), sino_br=(sc[2], sc[3]))
+
+
+@pytest.mark.parametrize("n,R,A,sc", GEO)
+def test_backprojection_planes(n, R, A, sc):
+    import torch
+    from pyraft_amd.device import BP_NVARIANTS, Plan
+    s = np.random.default_rng(n + R + A).random((3, R, A)).astype(np.float32)
+    ref = np.stack([O.backprojection(v.astype(np.float64), n, **_geo(sc)) for v in s])
+    j0, j1 = A // 3, max(A // 3 + 1, A - 1)
+    part = np.zeros_like(s, dtype=np.float64)
+    part[:, :, j0:j1] = s[:, :, j0:j1]
+    pref = np.stack([O.backprojection(v, n, **_geo(sc)) for v in part])
+    x = torch.from_numpy(s).cuda()
+    for v in range(BP_NVARIANTS):
+        p = Plan(n, R, A, sino_corners=sc)
+        p.set_bp_variant(v)
+        print("planes", n, R, A, sc, "variant", v, flush=True)
+        assert _rel(p.backprojection(x).cpu().numpy(), ref) <= REL
+        assert _rel(p.backprojection(x[1]).cpu().numpy(), ref[1]) <= REL
+        assert _rel(p.backprojection(x, angles=(j0, j1)).cpu().numpy(), pref) <= REL
