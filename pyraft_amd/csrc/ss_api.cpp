@@ -219,6 +219,32 @@ static bool mirror_symmetric(const SSGeom& g, const std::vector<SSAngle>& angles
   return true;
 }
 
+// The same of the Radon's sample positions u = alpha + k gamma + s beta (branch B's rows start
+// at xmin, so its grid can lack a symmetry that the backprojection's has).  turn: ray R-1-k at
+// sample n-1-s lies at n-1-u.  mirror (with turn): angle A-j is on angle j's branch, at n-1-u on
+// the same row (branch B) or at u on column n-1-s (branch A).  Theta = 0 needs no mirror: its
+// own half turn is the angle pi.  Within 1e-9 cells, as above.
+static void radon_symmetry(const SSGeom& g, const std::vector<SSAngle>& angles, bool* turn, bool* mirror) {
+  const double R1 = g.nrays - 1, n1 = g.n - 1, tol = 1e-9;
+  *turn = *mirror = true;
+  for (int j = 0; j < g.nangles; ++j) {
+    const SSTraj a = ss_trajectory(g, angles[j]);
+    *turn = *turn && fabs(2.0 * a.alpha0 + R1 * a.gamma + n1 * a.beta - n1) <= tol;
+    if (j == 0) {
+      *mirror = *mirror && fabs(angles[0].sint) <= tol;
+      continue;
+    }
+    const SSAngle& other = angles[g.nangles - j];
+    const SSTraj m = ss_trajectory(g, other);
+    const bool rows = angles[j].branch_a != 0;  // branch A: the cells are rows, which stay
+    const double d0 = rows ? m.alpha0 + n1 * m.beta - a.alpha0 : m.alpha0 + a.alpha0 - n1;
+    const double dg = rows ? m.gamma - a.gamma : m.gamma + a.gamma;
+    *mirror = *mirror && other.branch_a == angles[j].branch_a && fabs(d0) <= tol && R1 * fabs(dg) <= tol &&
+              n1 * fabs(m.beta + a.beta) <= tol;
+  }
+  *mirror = *mirror && *turn;
+}
+
 // all variants' staging; the default variant, or the first runnable one
 static int bp_variants(raft_ss_plan* p) {
   p->rt_variant = -1;
@@ -284,6 +310,7 @@ static int plan_create(raft_ss_plan** out, int n, int nrays, int nangles, const 
   if (!p->mesh) {
     p->half_turn = half_turn_symmetric(g, p->h_angles);
     p->mirror = mirror_symmetric(g, p->h_angles);
+    radon_symmetry(g, p->h_angles, &p->radon_turn, &p->radon_mirror);
     if ((rc = bp_variants(p.get()))) return rc;
   }
 
@@ -624,7 +651,7 @@ extern "C" int raft_ss_radon_range(const raft_ss_plan* p, const float* d_image, 
   hipStream_t stream = as_stream(stream_);
   SSDevPlan dp = p->dev();
   if ((rc = ss_plan_radon_rows(p, j0, j1, nslices, stream, true, &dp))) return rc;
-  const size_t layout = (size_t)nslices * p->g.n * p->g.pitch;
+  const size_t layout = ss_radon_layout_bytes(dp, nslices) / sizeof(float2);
   Scratch ws;
   HIP_TRY(ws.alloc(2 * layout * sizeof(float2) + ss_radon_scratch(dp, j0, j1, nslices), stream));
   float2* gA = ws.as<float2>();
@@ -766,11 +793,13 @@ int ss_em_prepare(const raft_ss_plan* p, int nsubsets, int nslices, int niter, h
   L->poff.assign(nsubsets + 1, 0);
   L->dps.assign(nsubsets, L->dp);
   size_t slab_bytes = 0;  // the largest subset's slab partial sums
+  L->layout_bytes = 0;    // and layouts
   for (int b = 0; b < nsubsets; ++b) {
     const int j0 = (int)(((long long)b * A) / nsubsets), j1 = (int)(((long long)(b + 1) * A) / nsubsets);
     if ((rc = ss_plan_radon_rows(p, j0, j1, nslices, stream, true, &L->dps[b]))) return rc;
     L->poff[b + 1] = L->poff[b] + ss_radon_partials(L->dps[b], j0, j1, nslices);
     slab_bytes = std::max(slab_bytes, ss_radon_scratch(L->dps[b], j0, j1, nslices));
+    L->layout_bytes = std::max(L->layout_bytes, ss_radon_layout_bytes(L->dps[b], nslices));
   }
   int bv = p->bp_variant;
   if ((rc = ss_plan_range_variant(const_cast<raft_ss_plan*>(p), 0, (int)(A / nsubsets), stream, &bv))) return rc;
@@ -783,8 +812,7 @@ int ss_em_prepare(const raft_ss_plan* p, int nsubsets, int nslices, int niter, h
   // workspace: two gather layouts, the measured and ratio sinograms (detector-major),
   // the S weight images, the LL partials, the LL trace, slab sums, BP partial images
   const size_t sino_sz = (size_t)nslices * R * A, img_sz = (size_t)nslices * n * n;
-  const size_t layout = (size_t)nslices * n * p->g.pitch;
-  size_t off = sizeof(float2) * 2 * layout;
+  size_t off = 2 * L->layout_bytes;
   L->meas_off = off;
   off += sizeof(float) * sino_sz;
   L->rho_off = off;
@@ -811,11 +839,10 @@ int ss_em_launch(const raft_ss_plan* p, const SSEmLaunch& L, const float* d_sino
                  int nslices, void* ws, double* d_ll, hipStream_t stream) {
   const int R = p->g.nrays, A = p->g.nangles, n = p->g.n, S = L.S;
   const size_t sino_sz = (size_t)nslices * R * A, img_sz = (size_t)nslices * n * n;
-  const size_t layout = (size_t)nslices * n * p->g.pitch;
   const int npartials = L.poff[S];
   char* base = static_cast<char*>(ws);
   float2* gA = reinterpret_cast<float2*>(base);
-  float2* gB = gA + layout;
+  float2* gB = reinterpret_cast<float2*>(base + L.layout_bytes);
   float* measT = reinterpret_cast<float*>(base + L.meas_off);
   float* rhoT = reinterpret_cast<float*>(base + L.rho_off);
   float* weights = reinterpret_cast<float*>(base + L.weights_off);
@@ -839,7 +866,7 @@ int ss_em_launch(const raft_ss_plan* p, const SSEmLaunch& L, const float* d_sino
       // only the layouts the subset's angles read (its Radon reads no other)
       int need = 0;
       for (int j = j0; j < j1; ++j) need |= p->h_angles[j].branch_a ? SS_GATHER_A : SS_GATHER_B;
-      HIP_TRY(ss_launch_gather_layouts(L.dp, d_x, gA, gB, nslices, stream, need));
+      HIP_TRY(ss_launch_gather_layouts(L.dps[b], d_x, gA, gB, nslices, stream, need));
       SSEmRatioArgs ea{measT, partials + L.poff[b]};
       HIP_TRY(ss_launch_radon(L.dps[b], gA, gB, j0, j1, nslices, SS_OUT_EM_RATIO, rhoT, ea, slabs, stream));
       SSEmUpdateArgs ua{d_x, weights + (size_t)b * img_sz};
@@ -898,7 +925,7 @@ extern "C" int raft_ss_tr_em(raft_ss_plan* p, const float* d_raw, const float* d
   if ((rc = ss_plan_radon_rows(p, 0, A, nslices, stream, true, &dp))) return rc;
   const size_t sino_sz = (size_t)nslices * R * A;
   const size_t img_sz = (size_t)nslices * n * n;
-  const size_t layout = (size_t)nslices * n * p->g.pitch;
+  const size_t layout = ss_radon_layout_bytes(dp, nslices) / sizeof(float2);
   Scratch ws;
   const size_t slab_bytes = ss_radon_scratch(dp, 0, A, nslices);
   HIP_TRY(ws.alloc(sizeof(float2) * 2 * layout + sizeof(float) * (3 * sino_sz + 2 * img_sz) + slab_bytes +

@@ -121,7 +121,7 @@ std::map<std::string, TuneEntry> g_tune;
 // A file of another format is ignored and a line that does not parse is skipped (that
 // geometry is timed again).  After each new choice the file is written whole to a
 // temporary name and renamed over the old one.  Callers hold g_tune_mu.
-const char* const kTuneFormat = "pyraft_amd tuning cache 4: backprojection variants x6 (paired), angle groups, radon shapes";
+const char* const kTuneFormat = "pyraft_amd tuning cache 4: backprojection variants x6 in planes, angle groups, radon shapes and planes";
 bool g_tune_loaded = false;
 
 std::string tune_cache_path() {
@@ -358,10 +358,18 @@ int ss_plan_range_variant(raft_ss_plan* p, int j0, int j1, hipStream_t stream, i
   return 0;
 }
 
+// The planes that a Radon launch can take (k_radon_planes)
+static int ss_plan_planes(const raft_ss_plan* p, int j0, int j1, int nslices) {
+  if (p->radon_mirror && j0 == 0 && j1 == p->g.nangles) return SS_PLANES_QUAD;
+  if (p->radon_turn && nslices >= 2) return SS_PLANES_PAIR;
+  return nslices >= 3 ? SS_PLANES_SLICES : SS_PLANES_NONE;
+}
+
 int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipStream_t stream, bool may_time,
                        SSDevPlan* out) {
   out->radon_slab_rows = 0;
   out->radon_shape = 0;
+  out->radon_planes = SS_PLANES_NONE;
   const int n = p->g.n;
   if (p->radon_rows_fixed > 0) {  // raft_ss_plan_set_radon_slab_rows
     out->radon_slab_rows = p->radon_rows_fixed;
@@ -369,6 +377,7 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
   }
   if (j1 <= j0) return 0;
   SSDevPlan dp = p->dev();
+  const int planes = ss_plan_planes(p, j0, j1, nslices);
   int r0 = n;
   const bool divides = ss_radon_slabs(dp, j0, j1, nslices, &r0) > 1;
   const long long pk = ((long long)(j1 - j0) << 20) | (long long)std::min(nslices, (1 << 20) - 1);
@@ -377,14 +386,35 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
     auto it = p->radon_rows.find(pk);
     if (it != p->radon_rows.end()) {
       out->radon_slab_rows = it->second & 0xffffff;
-      out->radon_shape = it->second >> 24;
+      out->radon_shape = it->second >> 24 & 1;
+      out->radon_planes = it->second >> 25;
       return 0;
     }
   }
+  // a planes launch that fills the chip undivided wins without timing: 2048^2 x 1500 780 us
+  // against 1070 with one ray per trajectory, 1448^2 x 500 204 against 266, 16 x 512^2 x 720
+  // 495 against 595, 8 x 768^2 x 600 on a mesh 429 against 572
+  SSDevPlan dpp = dp;
+  dpp.radon_planes = planes;
+  if (planes && ss_planes_blocks(dpp, j0, j1, nslices) >= SS_RADON_SLAB_BLOCKS) {
+    out->radon_slab_rows = n;
+    out->radon_planes = planes;
+    return 0;
+  }
   if (!may_time) return 0;  // the rule, shape 0 (no lookups that allocate)
-  // candidates (slab rows, shape); rows 0 is the default rule, which does not divide here
+  // candidates (slab rows, shape | planes << 1); rows 0 is the default rule, which does not
+  // divide here
   std::vector<std::pair<int, int>> cand;
-  if (divides) {
+  if (planes) {
+    int rp = n;
+    (void)ss_radon_slabs(dpp, j0, j1, nslices, &rp);
+    cand = {{rp, planes << 1}};
+    if (2 * rp < n) cand.push_back({2 * rp, planes << 1});
+    if (rp < n) cand.push_back({n, planes << 1});
+    cand.push_back({r0, 0});
+    cand.push_back({r0, 1});
+    if (divides && 2 * r0 < n) cand.push_back({2 * r0, 0});
+  } else if (divides) {
     cand = {{r0, 0}, {r0, 1}};
     if (2 * r0 < n) cand.push_back({2 * r0, 0});
     if (r0 / 2 >= RADON_SLAB_ALIGN && (r0 / 2) % RADON_SLAB_ALIGN == 0) cand.push_back({r0 / 2, 0});
@@ -405,10 +435,11 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(stream, &cs));
     if (cs != hipStreamCaptureStatusNone) return 0;  // the rule, untimed
-    const size_t layout = (size_t)nslices * n * p->g.pitch;
-    size_t slab_bytes = 0;
+    size_t layout = 0, slab_bytes = 0;
     for (const auto& c : cand) {
       dp.radon_slab_rows = c.first;
+      dp.radon_planes = c.second >> 1;
+      layout = std::max(layout, ss_radon_layout_bytes(dp, nslices) / sizeof(float2));
       slab_bytes = std::max(slab_bytes, ss_radon_scratch(dp, j0, j1, nslices));
     }
     const size_t img = (size_t)nslices * n * n, sino = (size_t)nslices * p->g.nrays * p->g.nangles;
@@ -420,15 +451,16 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
     float* sout = x + img;
     float* slabs = sout + sino;
     HIP_TRY(ss_launch_fill(x, 1.0f, img, stream));
-    HIP_TRY(ss_launch_gather_layouts(dp, x, gA, gB, nslices, stream));
     TuneEntry te;
     for (int v = 0; v < SS_BP_NVARIANTS; ++v) te.times[v] = -1.0;
     int best = 0, rc = 0;
     for (int c = 0; c < (int)cand.size() && c < SS_BP_NVARIANTS; ++c) {
       dp.radon_slab_rows = cand[c].first;
-      dp.radon_shape = cand[c].second;
+      dp.radon_shape = cand[c].second & 1;
+      dp.radon_planes = cand[c].second >> 1;
       SSEmRatioArgs none{nullptr, nullptr};
       auto run = [&]() -> int {
+        HIP_TRY(ss_launch_gather_layouts(dp, x, gA, gB, nslices, stream));
         HIP_TRY(ss_launch_radon(dp, gA, gB, j0, j1, nslices, SS_OUT_SINOT, sout, none, slabs, stream));
         return 0;
       };
@@ -442,7 +474,8 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
   std::lock_guard<std::mutex> lock(p->radon_mutex);
   p->radon_rows[pk] = cand[chosen].first | (cand[chosen].second << 24);
   out->radon_slab_rows = cand[chosen].first;
-  out->radon_shape = cand[chosen].second;
+  out->radon_shape = cand[chosen].second & 1;
+  out->radon_planes = cand[chosen].second >> 1;
   return 0;
 }
 

@@ -48,6 +48,7 @@ struct SSEmLaunch {
   std::vector<SSDevPlan> dps;  // per subset: the Radon with its slab choice
   std::vector<int> poff;       // LL partial offsets of the subsets (S + 1)
   // byte offsets in the workspace (the gather layouts start it) and its size
+  size_t layout_bytes = 0;  // one of the two layouts
   size_t meas_off = 0, rho_off = 0, weights_off = 0, partials_off = 0, ll_off = 0, slabs_off = 0, bp_off = 0;
   size_t bytes = 0;
 };
@@ -89,6 +90,7 @@ struct raft_ss_plan {
   int bp_angles_v[SS_BP_NVARIANTS] = {0};  //   and angles per stage (0: not runnable)
   // the grids map onto themselves under a half turn; and the angles under theta -> pi - theta
   bool half_turn = false, mirror = false;
+  bool radon_turn = false, radon_mirror = false;  // the same of the Radon's samples (radon_symmetry)
   // angles per stage of the backprojection with `planes` planes (0: not available)
   int bp_stage_v(int v, int planes) const {
     if (!half_turn || (planes == 4 && !mirror) || bp_angles_v[v] <= 0) return 0;
@@ -126,6 +128,7 @@ struct raft_ss_plan {
     p.bp_quad = bp_stage_v(v, 4);
     p.radon_slab_rows = 0;
     p.radon_shape = 0;
+    p.radon_planes = SS_PLANES_NONE;
     p.rt_variant = rt_variant >= 0 ? rt_variant : 0;
     p.rt_window = rt_variant >= 0 ? rt_window_v[rt_variant] : 0;
     p.rt_angles = rt_variant >= 0 ? rt_angles_v[rt_variant] : 0;

@@ -48,6 +48,7 @@ struct SSDevPlan {
   int bp_pair, bp_quad;    // angles per LDS stage with 2 and 4 planes (0: not available, see ss_bp_item)
   int radon_slab_rows;     // Radon: sample rows per slab (n: no division; 0: the default rule)
   int radon_shape;         // Radon: block shape (0: 4096 staged records, 32-row chunks; 1: 4864, 40)
+  int radon_planes;        // Radon: SS_PLANES_* of the launch (0: one ray per trajectory, radon_shape)
   // exact transpose, pixel-driven form: tile variant (the backprojection's shapes), rays
   // staged per angle and angles per stage; rt_angles = 0: not available (rays closer than
   // one cell on some angle), the line form runs instead
@@ -89,6 +90,15 @@ hipError_t ss_launch_plan_bounds(const SSGeom& g, const SSAngle* angles, int2* b
 hipError_t ss_launch_plan_wave_bounds(const SSGeom& g, const int2* bounds, int4* wbounds, hipStream_t stream);
 
 // ---- layouts
+// The Radon in planes (k_radon_planes): what the four planes of a launch are, the slices that
+// a group of planes covers, and the groups of a launch
+enum { SS_PLANES_NONE = 0, SS_PLANES_QUAD = 1, SS_PLANES_PAIR = 2, SS_PLANES_SLICES = 3 };
+static inline __host__ __device__ int ss_planes_slices(int kind) {
+  return kind == SS_PLANES_QUAD ? 1 : (kind == SS_PLANES_PAIR ? 2 : 4);
+}
+static inline int ss_planes_groups(int kind, int nslices) {
+  return (nslices + ss_planes_slices(kind) - 1) / ss_planes_slices(kind);
+}
 // the gather layouts are built in square tiles of SS_GATHER_TILE records per direction;
 // records q = 0..n+1 of each row
 #define SS_GATHER_TILE 64
@@ -100,6 +110,11 @@ static inline __host__ __device__ int ss_gather_tiles(int n) { return (n + 2 + S
 #define SS_GATHER_BOTH 3
 hipError_t ss_launch_gather_layouts(const SSDevPlan& p, const float* image, float2* gatherA, float2* gatherB,
                                     int nslices, hipStream_t stream, int which = SS_GATHER_BOTH);
+hipError_t ss_launch_gather_planes(const SSDevPlan& p, const float* image, float2* lA, float2* lB, int nslices,
+                                   hipStream_t stream, int which);
+// bytes of one layout (gatherA or gatherB) in the launch's form
+size_t ss_radon_layout_bytes(const SSDevPlan& p, int nslices);
+long long ss_planes_blocks(const SSDevPlan& p, int j0, int j1, int nslices);
 hipError_t ss_launch_sino_to_t(const float* sino, float* sinoT, int R, int A, int nslices, hipStream_t stream);
 hipError_t ss_launch_t_to_sino(const float* sinoT, float* sino, int R, int A, int nslices, hipStream_t stream);
 
@@ -116,8 +131,11 @@ struct SSEmRatioArgs {
 #define RADON_WAVES 8  // angles (one per wave) of a Radon block
 #endif
 #define SS_RADON_SLAB_BLOCKS (8192 / RADON_WAVES)
+// the planes form (two blocks per CU): 1024^2 x 720, 384 blocks, 160 us undivided, 138 in four
+// slabs
+#define SS_PLANES_SLAB_BLOCKS 1536
 #define RADON_SLAB_ALIGN 32  // rows per row slab: a multiple of this
-int ss_radon_slab_plan(int n, long long blocks, int* rows);
+int ss_radon_slab_plan(int n, long long blocks, int* rows, int target = SS_RADON_SLAB_BLOCKS);
 // blocks of the Radon of angles [j0, j1) on an image with `nwaves` ray groups
 static inline long long ss_radon_blocks(int nwaves, int j0, int j1) {
   return (long long)nwaves * ((j1 - j0 + RADON_WAVES - 1) / RADON_WAVES);

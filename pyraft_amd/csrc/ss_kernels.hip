@@ -179,6 +179,7 @@ hipError_t ss_launch_gather_layouts(const SSDevPlan& p, const float* image, floa
   const int n = p.g.n;
   const int tiles = ss_gather_tiles(n);
   if (!(which & SS_GATHER_BOTH)) return hipSuccess;
+  if (p.radon_planes) return ss_launch_gather_planes(p, image, gatherA, gatherB, nslices, stream, which);
   if ((long long)tiles * tiles * nslices >= 1024) {  // at least 4 large tiles per CU
     hipLaunchKernelGGL((k_gather_pairs<SS_GATHER_TILE, 8>), dim3(tiles, tiles, nslices), dim3(8 * SS_WAVE), 0, stream,
                        image, gatherA, gatherB, n, p.g.pitch, which);
@@ -286,6 +287,17 @@ __device__ __forceinline__ void ss_radon_store(const SSRadonView& p, int j, int 
 // rows into slabs taken by separate blocks instead (ss_radon_slab_plan).
 
 typedef float ss_f32x2 __attribute__((ext_vector_type(2)));
+typedef float ss_f32x4 __attribute__((ext_vector_type(4)));
+
+// Column of a lane in its 32-pixel tile row.  A 16-byte LDS read serves 16 lanes of a half
+// wave per pass, the lanes 0-3, 12-15, 20-27 and then the others; giving each of the two
+// sets 16 neighbouring columns keeps a pass within 16 neighbouring records, so that no two
+// of them share a bank (pixels are at most one ray apart).
+__device__ __forceinline__ int ss_bp_column(int lane) {
+  const int q = (lane >> 2) & 7;
+  return ((0x73261540 >> (4 * q)) & 7) * 4 + (lane & 3);
+}
+
 #define SS_RSRC_DWORD3 0x00020000  // gfx9 buffer word 3: 32-bit data format, no swizzle
 
 // Structured buffer load of one 8-byte record: address = base + soffset + vindex * stride.
@@ -457,9 +469,8 @@ __device__ __forceinline__ void ss_radon_rows(const Rd& rd, int sa, int sb, int 
 // [-1, n-1]), and the RADON_WAVES lanes of a chunk take the union.  Returns the widest
 // Wc of the table (block-uniform); `pass` selects the reduction slots, so that a second
 // pass right after the first needs no barrier in between.
-template <int CAP>
-__device__ __forceinline__ int ss_radon_windows(SSRadonLds<CAP>& lds, int pass, int sc, int rows, int nch, int s_hi,
-                                                int n) {
+template <bool PAIRS, class Lds>
+__device__ __forceinline__ int ss_radon_windows(Lds& lds, int pass, int sc, int rows, int nch, int s_hi, int n) {
   const int t = threadIdx.x;
   const int c = t / RADON_WAVES, w = t % RADON_WAVES;
   int cmin = 0x7fffffff, cmax = -0x7fffffff;
@@ -481,10 +492,12 @@ __device__ __forceinline__ int ss_radon_windows(SSRadonLds<CAP>& lds, int pass, 
     cmin = min(cmin, __shfl_xor(cmin, off));
     cmax = max(cmax, __shfl_xor(cmax, off));
   }
-  // cells c_lo..c_hi need records c_lo+1..c_hi+1; rec0 is even so that rows of the
-  // window start 16-byte aligned in the layout (even pitch) and in LDS (even Wc)
-  const int rec0 = (cmin + 1) & ~1;
-  int wc = cmax >= cmin ? ((cmax + 2 - rec0) + 1) & ~1 : 0;
+  // pair records: cells c_lo..c_hi need records c_lo+1..c_hi+1; rec0 is even so that rows of
+  // the window start 16-byte aligned in the layout (even pitch) and in LDS (even Wc).  Plane
+  // cells (16 bytes each): c_lo+1..c_hi+2, the upper tap being the next cell
+  const int rec0 = PAIRS ? (cmin + 1) & ~1 : cmin + 1;
+  int wc = 0;
+  if (cmax >= cmin) wc = PAIRS ? ((cmax + 2 - rec0) + 1) & ~1 : cmax + 3 - rec0;
   if (c >= nch) wc = 0;
   if (c < nch && w == 0) lds.table[c] = make_int2(rec0, wc);
   for (int off = 32; off > 0; off >>= 1) wc = max(wc, __shfl_xor(wc, off));
@@ -596,13 +609,13 @@ __device__ __forceinline__ void ss_radon_item(const SSRadonView& p, const float2
       for (int sc = s_lo; sc <= s_hi;) {
         int rows = CHUNK;
         int nch = min(RADON_TABLE, (s_hi - sc + rows) / rows);
-        const int wmax = ss_radon_windows(lds, 0, sc, rows, nch, s_hi, n);
+        const int wmax = ss_radon_windows<true>(lds, 0, sc, rows, nch, s_hi, n);
         if (wmax * rows > CAP) {
           int r2 = CAP / wmax;
           if (r2 >= RADON_ROW_ROUND) r2 = r2 / RADON_ROW_ROUND * RADON_ROW_ROUND;
           rows = max(r2, 1);
           nch = min(RADON_TABLE, (s_hi - sc + rows) / rows);
-          (void)ss_radon_windows(lds, 1, sc, rows, nch, s_hi, n);
+          (void)ss_radon_windows<true>(lds, 1, sc, rows, nch, s_hi, n);
         }
         const int64_t chunk_step = (int64_t)rows * beta;
         for (int c = 0; c < nch; ++c) {
@@ -718,6 +731,443 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE) void k_radon(SSDevPlan p, co
                       slot, po, lds);
 }
 
+// =====================================================================================
+// Radon in planes: four rays per trajectory
+//
+// The one-ray kernel above is bound by its LDS reads (8-byte records gamma = 1..1.41 cells
+// apart: two-way bank conflicts, 7.9 lane-reads per CU-clock where the stride exceeds ~1.05)
+// and issues 5 VALU instructions per update, three of them for the trajectory, its weight
+// and the address.  Here a lane's trajectory serves four rays whose samples lie at the same
+// cell of four images, the planes:
+//   SS_PLANES_QUAD    on a grid symmetric about the rotation axis, over all angles of
+//                     [0, pi): the image, its half turn (ray -t), its mirror x -> -x (angle
+//                     pi - theta) and the half turn of that (pi - theta, -t);
+//   SS_PLANES_PAIR    two slices and their half turns (any angle range);
+//   SS_PLANES_SLICES  four slices (any geometry).
+// The layouts hold the planes' values of a cell together (16 bytes), so one 16-byte LDS
+// read gives the lower taps and another the upper taps of all four; the lanes of a read
+// pass hold 16 neighbouring rays (ss_plane_ray), which keeps its conflicts two-way.  Per
+// four updates: 4 VALU for the trajectory, address and the two weights, 8 FMAs, two reads
+// (16 updates per CU-clock at any stride).  Sums are taken in FP32 over 8 samples, those over
+// a chunk's rows and those over the ray: 1e-7 from the 64-bit sums at 2048^2 x 1500 (one
+// running sum per ray: 6e-7).  2048^2 x 1500: 1.07 -> 0.78 ms, the layouts' 27 us included; the
+// kernel issues VALU 0.85 and reads LDS 0.75 of the clocks a CU is busy, which is 0.85 of its
+// time (2.9 rounds of blocks).
+//
+// Every plane's ray keeps its own exact sample range, delta and output; rays computed twice
+// (the middle ray of an odd detector, theta = 0 and pi/2, slices past the last) are stored
+// once.  Irregular rays have empty ranges here and go to k_radon_fixup.
+// =====================================================================================
+
+#define SS_PLANES 4
+
+// plane z of a launch: its slice within the group, whether it is the half turn of its image
+// and whether the mirror
+struct SSPlane {
+  int slice;
+  bool turn, mirror;
+};
+__device__ __host__ __forceinline__ SSPlane ss_plane(int kind, int z) {
+  if (kind == SS_PLANES_QUAD) return SSPlane{0, (z & 1) != 0, (z & 2) != 0};
+  if (kind == SS_PLANES_PAIR) return SSPlane{z >> 1, (z & 1) != 0, false};
+  return SSPlane{z, false, false};
+}
+
+// Ray of a lane within its group of 64: a 16-byte LDS read serves the lanes 0-3, 12-15,
+// 20-27 of a half wave in one pass and the others in the next; each set gets 16 neighbours.
+__device__ __forceinline__ int ss_plane_ray(int lane) { return (lane & 32) + ss_bp_column(lane); }
+
+// Layout row r of B (image rows) and row c of A (image columns), cells q in [0, n + 1]:
+//   LB[r][q] = (G_0, .., G_3)(r, q - 1),  LA[c][q] = (G_0, .., G_3)(q - 1, c)
+// with G_z plane z's image and 0 outside.  A block moves one 32 x 32 pixel tile.
+__global__ __launch_bounds__(256) void k_gather_planes(const float* __restrict__ img, ss_f32x4* __restrict__ lA,
+                                                       ss_f32x4* __restrict__ lB, int n, int pitch, int nslices,
+                                                       int kind, int which) {
+  __shared__ float T[SS_PLANES][32][33];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
+  const int per = ss_planes_slices(kind);
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) {
+    const SSPlane pl = ss_plane(kind, z);
+    const size_t slice = (size_t)min((int)blockIdx.z * per + pl.slice, nslices - 1);
+    const float* src = img + slice * n * n;
+#pragma unroll
+    for (int yy = ty; yy < 32; yy += 8) {
+      const int r = by + yy, c = bx + tx;
+      const int sr = pl.turn ? n - 1 - r : r, sc = pl.turn != pl.mirror ? n - 1 - c : c;
+      T[z][yy][tx] = r < n && c < n ? src[(size_t)sr * n + sc] : 0.f;
+    }
+  }
+  __syncthreads();
+  ss_f32x4* dA = lA + (size_t)blockIdx.z * n * pitch;
+  ss_f32x4* dB = lB + (size_t)blockIdx.z * n * pitch;
+  const ss_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int yy = ty; yy < 32; yy += 8) {
+    if (which & SS_GATHER_B) {
+      const int r = by + yy, q = bx + tx + 1;
+      if (r < n && q <= n) dB[(size_t)r * pitch + q] = ss_f32x4{T[0][yy][tx], T[1][yy][tx], T[2][yy][tx], T[3][yy][tx]};
+      if (r < n && q == 1) dB[(size_t)r * pitch] = zero;
+      if (r < n && q == n) dB[(size_t)r * pitch + n + 1] = zero;
+    }
+    if (which & SS_GATHER_A) {
+      const int c = bx + yy, q = by + tx + 1;
+      if (c < n && q <= n) dA[(size_t)c * pitch + q] = ss_f32x4{T[0][tx][yy], T[1][tx][yy], T[2][tx][yy], T[3][tx][yy]};
+      if (c < n && q == 1) dA[(size_t)c * pitch] = zero;
+      if (c < n && q == n) dA[(size_t)c * pitch + n + 1] = zero;
+    }
+  }
+}
+
+// staged cells per block and sample rows per chunk at most: two 512-thread blocks per CU
+#ifndef PLANES_CAP
+#define PLANES_CAP 4864
+#define PLANES_CHUNK 40
+#define PLANES_BLOCKS 2
+#endif
+
+struct SSPlanesLds {
+  double red[RADON_WAVES];
+  int64_t wpar[RADON_WAVES][3];  // as SSRadonLds
+  int wmeta[RADON_WAVES][4];
+  int wred[2][RADON_WAVES];
+  int2 table[RADON_TABLE];
+  alignas(16) ss_f32x4 stage[PLANES_CAP + 2];  // chunk window; cells CAP, CAP + 1 stay 0
+};
+
+typedef __attribute__((address_space(3))) const ss_f32x4* ss_lds_cell;
+
+// the sample range of a lane's ray on each plane, in the sample order of plane 0's ray
+struct SSPlaneRanges {
+  int lo[SS_PLANES];
+  unsigned span[SS_PLANES];  // valid samples lo .. lo + span
+};
+
+// G samples s, s + 1, ... from the staged window.  CHECK: a sample at or beyond `end`, or
+// outside the ray's range, reads the zero cells; with OWN each plane tests its own range
+// (they differ at knife-edge samples), else the planes share plane 0's.
+template <int G, bool CHECK, bool OWN>
+__device__ __forceinline__ void ss_planes_group(const ss_f32x4* __restrict__ st, int s, int end, int64_t& u,
+                                                int64_t step, const SSPlaneRanges& rg, float (&acc)[SS_PLANES]) {
+  float part[SS_PLANES];
+  const unsigned stb = (unsigned)(size_t)(ss_lds_cell)st;
+#pragma unroll
+  for (int h = 0; h < G; h += 4) {  // four samples' reads in flight
+    ss_f32x4 a[4], b[4];
+    float w[4];
+    int keep[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      int idx = (int)(u >> 32);
+      keep[g] = 0;
+      if (CHECK) {
+        const int t = s + h + g;
+        if (OWN) {
+#pragma unroll
+          for (int z = 0; z < SS_PLANES; ++z) keep[g] |= (t < end && (unsigned)(t - rg.lo[z]) <= rg.span[z]) << z;
+          idx = keep[g] ? idx : PLANES_CAP;
+        } else {
+          idx = t < end && (unsigned)(t - rg.lo[0]) <= rg.span[0] ? idx : PLANES_CAP;
+        }
+      }
+      w[g] = (float)(uint32_t)u;
+      u += step;
+      __asm__ volatile("" : "+v"(u));  // one 64-bit add per sample
+      // one byte address for both cells (the second in the read's offset field)
+      const ss_lds_cell c = (ss_lds_cell)(size_t)(stb + ((unsigned)idx << 4));
+      a[g] = c[0];
+      b[g] = c[1];
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float w1 = 4294967296.f - w[g];
+#pragma unroll
+      for (int z = 0; z < SS_PLANES; ++z) {
+        float lo = a[g][z], hi = b[g][z];
+        if (CHECK && OWN) {
+          lo = keep[g] >> z & 1 ? lo : 0.f;
+          hi = keep[g] >> z & 1 ? hi : 0.f;
+        }
+        part[z] = h + g == 0 ? w1 * lo : fmaf(w1, lo, part[z]);
+        part[z] = fmaf(w[g], hi, part[z]);
+      }
+    }
+  }
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) acc[z] += part[z];
+}
+
+// samples [sa, sb): checked groups before zlo and from zhi1 on, unchecked between
+template <bool OWN>
+__device__ __forceinline__ void ss_planes_rows(const ss_f32x4* __restrict__ st, int sa, int sb, int zlo, int zhi1,
+                                               int64_t u, int64_t step, const SSPlaneRanges& rg,
+                                               float (&acc)[SS_PLANES]) {
+  int s = sa;
+  const int h_end = min(sb, zlo);
+  if (s < h_end) {
+    const int64_t u0 = u;
+    for (; s < h_end; s += 4) ss_planes_group<4, true, OWN>(st, s, h_end, u, step, rg, acc);
+    s = h_end;
+    u = u0 + (int64_t)(h_end - sa) * step;
+  }
+  const int m_end = min(sb, zhi1);
+  for (; s + 8 <= m_end; s += 8) ss_planes_group<8, false, OWN>(st, s, 0, u, step, rg, acc);
+  for (; s < sb; s += 4) ss_planes_group<4, true, OWN>(st, s, sb, u, step, rg, acc);
+}
+
+// One block: the rays of group `grp` of the RADON_WAVES angles from j0 + ablk*RADON_WAVES
+// (clipped to j1: plane 0's angles), sample rows [row_lo, row_hi).  A block whose angles lie
+// on both sides of a branch switch makes a pass for each.
+template <int MODE>
+__device__ __forceinline__ void ss_planes_item(const SSRadonView& p, const ss_f32x4* __restrict__ lA,
+                                               const ss_f32x4* __restrict__ lB, int kind, int slice0, int nslices,
+                                               int j0, int j1, int jpart, int npart, int nrays, int grp, int ablk,
+                                               int row_lo, int row_hi, float* __restrict__ out,
+                                               const float* __restrict__ meas, double* ll_slot,
+                                               float* __restrict__ part_out, size_t part_slice, SSPlanesLds& lds) {
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = j0 + ablk * RADON_WAVES + wv;
+  const int R = p.R, A = p.A, n = p.n, pitch = p.pitch;
+  const int k = grp * SS_WAVE + ss_plane_ray(lane);
+  const bool active = j < j1, on = active && k < nrays;
+  int branch = -1;
+  int64_t a_k = 0, beta = 0;
+  SSPlaneRanges rg;
+  // the group's rows: union and common range over its rays and planes
+  int ulo = 0x7fffffff, uhi = -1, clo = -0x7fffffff, chi = 0x7fffffff;
+  bool any = false, own = false;
+  if (active) {
+    const SSAngle& a = p.angles[j];
+    branch = ss_rfl(a.branch_a);
+    beta = ss_rfl64(a.beta);
+    a_k = ss_rfl64(a.alpha0) + (int64_t)k * ss_rfl64(a.gamma);
+    if (p.ray_alpha && k < R) a_k = p.ray_alpha[(size_t)j * R + k];
+  }
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) {
+    const SSPlane pl = ss_plane(kind, z);
+    rg.lo[z] = 0x40000000;  // empty: no sample passes the test
+    rg.span[z] = 0;
+    if (on) {
+      const int jz = pl.mirror ? (j > 0 ? A - j : 0) : j;
+      const bool rev = pl.turn != (pl.mirror && j == 0);  // angle pi is angle 0 with the rays reversed
+      int2 b = p.bounds[(size_t)jz * R + (rev ? R - 1 - k : k)];
+      if (b.y >= b.x) {
+        // image rows (branch B) are reversed by the half turn, columns (A) by either
+        if (pl.turn != (pl.mirror && branch == 1)) b = make_int2(n - 1 - b.y, n - 1 - b.x);
+        rg.lo[z] = b.x;
+        rg.span[z] = (unsigned)(b.y - b.x);
+        any = true;
+        ulo = min(ulo, b.x);
+        uhi = max(uhi, b.y);
+        clo = max(clo, b.x);
+        chi = min(chi, b.y);
+      }
+    }
+    own = own || rg.lo[z] != rg.lo[0] || rg.span[z] != rg.span[0];
+  }
+  if (own && any) {  // no common range: every sample of the ray is tested per plane
+    bool whole = true;
+#pragma unroll
+    for (int z = 0; z < SS_PLANES; ++z) whole = whole && rg.lo[z] != 0x40000000;
+    if (!whole) clo = 0x7fffffff, chi = -1;
+  }
+  const bool own_wave = __ballot(own) != 0ull;
+  int64_t amin = on ? a_k : INT64_MAX, amax = on ? a_k : INT64_MIN;
+  for (int off = 32; off > 0; off >>= 1) {
+    ulo = min(ulo, __shfl_xor(ulo, off));
+    uhi = max(uhi, __shfl_xor(uhi, off));
+    clo = max(clo, __shfl_xor(clo, off));
+    chi = min(chi, __shfl_xor(chi, off));
+    amin = min(amin, (int64_t)__shfl_xor((long long)amin, off));
+    amax = max(amax, (int64_t)__shfl_xor((long long)amax, off));
+  }
+  ulo = ss_rfl(ulo);
+  uhi = ss_rfl(uhi);
+  clo = ss_rfl(clo);
+  chi = ss_rfl(chi);
+  if (uhi < ulo) branch = -1;
+  if (lane == 0) {
+    lds.wmeta[wv][0] = branch;
+    lds.wmeta[wv][1] = ulo;
+    lds.wmeta[wv][2] = uhi;
+    lds.wmeta[wv][3] = branch;
+    lds.wpar[wv][0] = amin;
+    lds.wpar[wv][1] = amax;
+    lds.wpar[wv][2] = beta;
+  }
+  if (threadIdx.x < 2) lds.stage[PLANES_CAP + threadIdx.x] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
+  float tot[SS_PLANES] = {0.f, 0.f, 0.f, 0.f};
+  for (int pass = 0; pass < 2; ++pass) {
+    __syncthreads();
+    if (lane == 0) lds.wmeta[wv][0] = branch == pass ? branch : -1;  // this pass's waves
+    __syncthreads();
+    int s_lo = 0x7fffffff, s_hi = -1;
+    for (int w = 0; w < RADON_WAVES; ++w)
+      if (lds.wmeta[w][0] >= 0) {
+        s_lo = min(s_lo, lds.wmeta[w][1]);
+        s_hi = max(s_hi, lds.wmeta[w][2]);
+      }
+    s_lo = max(ss_rfl(s_lo), row_lo);
+    s_hi = min(ss_rfl(s_hi), row_hi - 1);
+    const bool mine = branch == pass;
+    const ss_f32x4* lay = pass ? lA : lB;
+    int64_t t0 = s_lo <= s_hi ? a_k + (int64_t)s_lo * beta : 0;
+    for (int sc = s_lo; sc <= s_hi;) {  // block-uniform; super-chunks as in ss_radon_item
+      int rows = PLANES_CHUNK;
+      int nch = min(RADON_TABLE, (s_hi - sc + rows) / rows);
+      const int wmax = ss_radon_windows<false>(lds, 0, sc, rows, nch, s_hi, n);
+      if (wmax * rows > PLANES_CAP) {
+        int r2 = PLANES_CAP / wmax;
+        if (r2 >= RADON_ROW_ROUND) r2 = r2 / RADON_ROW_ROUND * RADON_ROW_ROUND;
+        rows = max(r2, 1);
+        nch = min(RADON_TABLE, (s_hi - sc + rows) / rows);
+        (void)ss_radon_windows<false>(lds, 1, sc, rows, nch, s_hi, n);
+      }
+      const int64_t chunk_step = (int64_t)rows * beta;
+      for (int c = 0; c < nch; ++c) {
+        const int s0 = sc + c * rows, s1 = min(s0 + rows, s_hi + 1);
+        const int2 tw = lds.table[c];
+        const int rec0 = ss_rfl(tw.x), Wc = ss_rfl(tw.y);
+        const bool fits = Wc > 0 && (s1 - s0) * Wc <= PLANES_CAP;  // block-uniform
+        if (c > 0) __syncthreads();  // every wave is done with the previous chunk
+        if (fits) {
+          const ss_f32x4* src0 = lay + (size_t)(s0 + wv) * pitch + rec0 + lane;
+          for (int seg = 0; seg < Wc; seg += SS_WAVE) {
+            if (seg + lane < Wc) {
+              const ss_f32x4* src = src0 + seg;
+              ss_f32x4* dst = lds.stage + wv * Wc + seg;
+              for (int r = wv; r < s1 - s0; r += RADON_WAVES) {
+                __builtin_amdgcn_global_load_lds((ss_global_cptr)src, (ss_lds_ptr)dst, 16, 0, 0);
+                src += (size_t)RADON_WAVES * pitch;
+                dst += RADON_WAVES * Wc;
+              }
+            }
+          }
+        }
+        __syncthreads();  // window staged
+        const int ra2 = max(s0, ulo), rb2 = min(s1 - 1, uhi);
+        if (mine && ra2 <= rb2 && Wc > 0) {
+          const int64_t t = t0 + (int64_t)(ra2 - s0) * beta;
+          float acc[SS_PLANES] = {0.f, 0.f, 0.f, 0.f};  // the chunk's sum
+          if (fits) {
+            // high word: staged cell index (cell + 1 - rec0) + (row - s0) * Wc
+            int64_t u = t + ((int64_t)(1 - rec0 + (ra2 - s0) * Wc) << 32);
+            int64_t step = beta + ((int64_t)Wc << 32);
+            if (!any) {
+              u = (int64_t)PLANES_CAP << 32;
+              step = 0;
+            }
+            if (own_wave)
+              ss_planes_rows<true>(lds.stage, ra2, rb2 + 1, clo, chi + 1, u, step, rg, acc);
+            else
+              ss_planes_rows<false>(lds.stage, ra2, rb2 + 1, clo, chi + 1, u, step, rg, acc);
+          } else if (any) {  // the window does not fit the LDS: read the layout
+            int64_t u = t + ((int64_t)1 << 32);
+            for (int s = ra2; s <= rb2; ++s, u += beta) {
+              int keep = 0;
+#pragma unroll
+              for (int z = 0; z < SS_PLANES; ++z) keep |= ((unsigned)(s - rg.lo[z]) <= rg.span[z]) << z;
+              if (keep) {
+                const ss_f32x4* cell = lay + (size_t)s * pitch + (int)(u >> 32);
+                const ss_f32x4 a = cell[0], b = cell[1];
+                const float w = (float)(uint32_t)u, w1 = 4294967296.f - w;
+#pragma unroll
+                for (int z = 0; z < SS_PLANES; ++z) {
+                  const float v = fmaf(w, b[z], w1 * a[z]);
+                  acc[z] += keep >> z & 1 ? v : 0.f;
+                }
+              }
+            }
+          }
+#pragma unroll
+          for (int z = 0; z < SS_PLANES; ++z) tot[z] += acc[z];
+        }
+        t0 += chunk_step;
+      }
+      sc += nch * rows;
+    }
+  }
+  double ll = 0.0;
+  if (on) {
+#pragma unroll
+    for (int z = 0; z < SS_PLANES; ++z) {
+      const SSPlane pl = ss_plane(kind, z);
+      const int kz = pl.turn ? R - 1 - k : k;
+      const int jz = pl.mirror ? A - j : j;
+      if (slice0 + pl.slice >= nslices) continue;     // a group past the last slice
+      if (pl.turn && kz == k) continue;               // the middle ray, its own half turn
+      if (pl.mirror && (j == 0 || jz == j)) continue;  // angles that are their own mirror
+      const float sum = tot[z] * SS_INV_FIX;
+      const size_t so = (size_t)(slice0 + pl.slice) * A * R;
+      if (MODE == SS_OUT_PARTIAL) {
+        part_out[(size_t)pl.slice * part_slice + (size_t)(jz - jpart) * R + kz] = sum;
+      } else {
+        ss_radon_store<MODE>(p, jz, kz, sum * p.angles[jz].delta, out + so,
+                             MODE == SS_OUT_EM_RATIO ? meas + so : nullptr, &ll);
+      }
+    }
+  }
+  if (MODE == SS_OUT_EM_RATIO) {
+    const double tot = ss_block_sum_f64(ll, lds.red);
+    if (threadIdx.x == 0) *ll_slot = tot;
+  }
+}
+
+// Order of a planes launch's blocks: consecutive blocks go to the 8 XCDs in turn, each with an
+// L2 of its own.  A unit is a ray group's angle blocks [c yc, (c + 1) yc); the units, from the
+// long rays at the detector's centre to the short ones at its edge, are dealt to the XCDs
+// there and back, so that each XCD gets the same mix and walks one strip of the image with
+// slowly turning angles at a time.
+struct SSPlanesOrder {
+  int g, y;       // ray groups, angle blocks
+  int c, yc;      // units per ray group (g c a multiple of 16), angle blocks per unit
+  int blocks;     // blocks launched; those past a group's angle blocks have no work
+};
+static SSPlanesOrder ss_planes_order(int nrays, int nangles) {
+  SSPlanesOrder o;
+  o.g = (nrays + SS_WAVE - 1) / SS_WAVE;
+  o.y = (nangles + RADON_WAVES - 1) / RADON_WAVES;
+  o.c = 1;
+  while (o.g * o.c % 16) o.c *= 2;
+  o.yc = (o.y + o.c - 1) / o.c;
+  o.blocks = o.g * o.c * o.yc;
+  return o;
+}
+
+// blockIdx.z = group * nslab + z.  The block's rays and angles come from `order`, over plane
+// 0's angles [j0, jd1) and rays [0, nrays); partial sums are laid out over [j0, j1).
+template <int MODE>
+__global__ __launch_bounds__(RADON_WAVES * SS_WAVE, PLANES_BLOCKS) void k_radon_planes(
+    SSDevPlan p, const ss_f32x4* __restrict__ lA, const ss_f32x4* __restrict__ lB, int kind, int nslices, int j0,
+    int j1, int jd1, int nrays, SSPlanesOrder order, int nslab, int slab_rows, float* __restrict__ out,
+    float* __restrict__ part, SSEmRatioArgs em) {
+  __shared__ SSPlanesLds lds;
+  const int z = (int)(blockIdx.z % (unsigned)nslab);
+  const int group = (int)(blockIdx.z / (unsigned)nslab);
+  const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
+  const int deal = turn / order.yc;
+  const int unit = deal * 8 + (deal & 1 ? 7 - xcd : xcd);
+  const int grp = order.g - 1 - unit / order.c;
+  const int ablk = unit % order.c * order.yc + turn % order.yc;
+  const size_t lay = (size_t)group * p.g.n * p.g.pitch;
+  const int slice0 = group * ss_planes_slices(kind);
+  const size_t per = (size_t)(j1 - j0) * p.g.nrays;
+  double* slot = nullptr;
+  if (MODE == SS_OUT_EM_RATIO) slot = em.ll_partials + (size_t)group * gridDim.x + blockIdx.x;
+  if (ablk >= order.y) {  // block-uniform
+    if (MODE == SS_OUT_EM_RATIO && threadIdx.x == 0) *slot = 0.0;
+    return;
+  }
+  float* po = MODE == SS_OUT_PARTIAL ? part + ((size_t)slice0 * nslab + z) * per : nullptr;
+  ss_planes_item<MODE>(ss_radon_view(p), lA + lay, lB + lay, kind, slice0, nslices, j0, jd1, j0, j1 - j0, nrays,
+                       grp, ablk,
+                       z * slab_rows, min(p.g.n, (z + 1) * slab_rows), out, em.meas, slot, po,
+                       (size_t)nslab * per, lds);
+}
+
 // Sums the slabs' partial sums of rays [j0, j1) x [0, R) of each slice and stores them
 // as k_radon does (delta applied; in EM mode the ratio, and one FP64 log-likelihood
 // partial per block at ll_partials[slice * gridDim.x + blockIdx.x]).
@@ -806,10 +1256,10 @@ __global__ __launch_bounds__(256) void k_radon_fixup(SSDevPlan p, const float2* 
 // slabs' partial sums.  Rows per slab are a multiple of RADON_SLAB_ALIGN, and the divided
 // launch stays within SS_RADON_SLAB_BLOCKS blocks (4 per CU, one round: a second round
 // for a few blocks would double the launch time).
-int ss_radon_slab_plan(int n, long long blocks, int* rows) {
+int ss_radon_slab_plan(int n, long long blocks, int* rows, int target) {
   *rows = n;
-  if (blocks >= SS_RADON_SLAB_BLOCKS) return 1;
-  const long long want = SS_RADON_SLAB_BLOCKS / std::max(blocks, 1LL);
+  if (blocks >= target) return 1;
+  const long long want = target / std::max(blocks, 1LL);
   if (want <= 1) return 1;
   int L = (int)((n + want - 1) / want);
   L = (L + RADON_SLAB_ALIGN - 1) / RADON_SLAB_ALIGN * RADON_SLAB_ALIGN;
@@ -830,10 +1280,41 @@ int ss_radon_slabs(const SSDevPlan& p, int j0, int j1, int nslices, int* rows) {
     *rows = L;
     return count;
   }
+  if (p.radon_planes)
+    return ss_radon_slab_plan(n, ss_planes_blocks(p, j0, j1, nslices), rows, SS_PLANES_SLAB_BLOCKS);
   return ss_radon_slab_plan(n, ss_radon_blocks(p.nwaves, j0, j1) * nslices, rows);
 }
 
 static int ss_radon_finish_blocks(int nj, int R) { return (int)(((long long)nj * R + 255) / 256); }
+
+size_t ss_radon_layout_bytes(const SSDevPlan& p, int nslices) {
+  const size_t records = (size_t)p.g.n * p.g.pitch;
+  if (!p.radon_planes) return sizeof(float2) * records * nslices;
+  return sizeof(ss_f32x4) * records * ss_planes_groups(p.radon_planes, nslices);
+}
+
+// Plane 0's angles and rays of a launch over [j0, j1): a quad launch's blocks walk theta in
+// [0, pi/2] and half the detector, the pair form half the detector
+static int ss_planes_j1(const SSDevPlan& p, int j1) {
+  return p.radon_planes == SS_PLANES_QUAD ? p.g.nangles / 2 + 1 : j1;
+}
+static int ss_planes_rays(const SSDevPlan& p) {
+  return p.radon_planes == SS_PLANES_SLICES ? p.g.nrays : (p.g.nrays + 1) / 2;
+}
+
+hipError_t ss_launch_gather_planes(const SSDevPlan& p, const float* image, float2* lA, float2* lB, int nslices,
+                                   hipStream_t stream, int which) {
+  const int t = (p.g.n + 31) / 32;
+  hipLaunchKernelGGL(k_gather_planes, dim3(t, t, ss_planes_groups(p.radon_planes, nslices)), dim3(256), 0, stream,
+                     image, reinterpret_cast<ss_f32x4*>(lA), reinterpret_cast<ss_f32x4*>(lB), p.g.n, p.g.pitch,
+                     nslices, p.radon_planes, which);
+  return hipGetLastError();
+}
+
+long long ss_planes_blocks(const SSDevPlan& p, int j0, int j1, int nslices) {
+  return (long long)ss_planes_order(ss_planes_rays(p), ss_planes_j1(p, j1) - j0).blocks *
+         ss_planes_groups(p.radon_planes, nslices);
+}
 
 size_t ss_radon_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
   int rows;
@@ -844,6 +1325,7 @@ size_t ss_radon_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
 int ss_radon_partials(const SSDevPlan& p, int j0, int j1, int nslices) {
   int rows;
   const int nslab = ss_radon_slabs(p, j0, j1, nslices, &rows);
+  if (nslab == 1 && p.radon_planes) return (int)ss_planes_blocks(p, j0, j1, nslices) + p.nirregular * nslices;
   const int main = nslab > 1 ? ss_radon_finish_blocks(j1 - j0, p.g.nrays)
                              : p.nwaves * ((j1 - j0 + RADON_WAVES - 1) / RADON_WAVES);
   return (main + p.nirregular) * nslices;
@@ -858,10 +1340,17 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
   dim3 grid(p.nwaves, (j1 - j0 + RADON_WAVES - 1) / RADON_WAVES, nslices * nslab);
   dim3 block(RADON_WAVES * SS_WAVE);
   int partial_base;
-  // the main pass in the plan's block shape (0 or 1)
+  const int jd1 = ss_planes_j1(p, j1), half = ss_planes_rays(p);
+  const SSPlanesOrder order = ss_planes_order(half, jd1 - j0);
+  if (p.radon_planes) grid = dim3(order.blocks, 1, ss_planes_groups(p.radon_planes, nslices) * nslab);
+  // the main pass in the plan's form: planes, or block shape 0 or 1
 #define SS_RADON_LAUNCH(MODE, OUTP, PARTP, NSLAB, ROWS, EM)                                                        \
   do {                                                                                                            \
-    if (p.radon_shape == 1)                                                                                       \
+    if (p.radon_planes)                                                                                           \
+      hipLaunchKernelGGL(k_radon_planes<MODE>, grid, block, 0, stream, p,                                         \
+                         reinterpret_cast<const ss_f32x4*>(gatherA), reinterpret_cast<const ss_f32x4*>(gatherB),  \
+                         p.radon_planes, nslices, j0, j1, jd1, half, order, NSLAB, ROWS, OUTP, PARTP, EM);        \
+    else if (p.radon_shape == 1)                                                                                       \
       hipLaunchKernelGGL((k_radon<MODE, 1>), grid, block, 0, stream, p, gatherA, gatherB, j0, j1, NSLAB, ROWS,    \
                          OUTP, PARTP, EM);                                                                        \
     else                                                                                                          \
@@ -901,7 +1390,7 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
         break;
     }
 #undef SS_RADON_LAUNCH
-    partial_base = (int)(grid.x * grid.y) * nslices;
+    partial_base = (int)(grid.x * grid.y) * (p.radon_planes ? (int)grid.z : nslices);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.nirregular == 0) return e;
@@ -941,8 +1430,6 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
 
 #define BP_TILE_W 32
 
-typedef float ss_f32x4 __attribute__((ext_vector_type(4)));
-
 struct alignas(16) BPAngle {
   float f0, b, c;  // read together with flag by one 16-byte LDS read
   int flag;        // 0 outside, 1 interior, 2 boundary
@@ -971,15 +1458,6 @@ __device__ float ss_raw_load_f32(__amdgpu_buffer_rsrc_t rsrc, int voffset, int s
 // the value of the next lane (lane 63: 0)
 __device__ __forceinline__ float ss_next_lane(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
-}
-
-// Column of a lane in its 32-pixel tile row.  A 16-byte LDS read serves 16 lanes of a half
-// wave per pass, the lanes 0-3, 12-15, 20-27 and then the others; giving each of the two
-// sets 16 neighbouring columns keeps a pass within 16 neighbouring records, so that no two
-// of them share a bank (pixels are at most one ray apart).
-__device__ __forceinline__ int ss_bp_column(int lane) {
-  const int q = (lane >> 2) & 7;
-  return ((0x73261540 >> (4 * q)) & 7) * 4 + (lane & 3);
 }
 
 // The sinogram row that the mirrored planes of angle j read (PL = 4): that of the angle

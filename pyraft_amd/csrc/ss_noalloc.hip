@@ -13,7 +13,9 @@
 #include "../../include/raft_noalloc.h"
 #include "ss_internal.h"
 
-static __device__ __align__(256) unsigned char scratch[RAFT_SS_NOALLOC_SCRATCH_BYTES];
+// twice the limit that callers see: the limit counts the one-ray layouts, the layouts of a
+// launch in planes (one slice: its four symmetric images) take up to twice their bytes
+static __device__ __align__(256) unsigned char scratch[2 * RAFT_SS_NOALLOC_SCRATCH_BYTES];
 
 namespace {
 
@@ -49,9 +51,10 @@ extern "C" int raft_ss_radon_noalloc(const raft_ss_plan* p, const float* d_image
   // the plan's slab choice when an earlier call made one (this entry never times)
   hipStream_t stream = as_stream(stream_);
   if ((rc = ss_plan_radon_rows(p, j0, j1, nslices, stream, false, &dp))) return rc;
-  const size_t layout = (size_t)nslices * p->g.n * p->g.pitch;
+  const size_t layout = ss_radon_layout_bytes(dp, nslices) / sizeof(float2);
   const size_t layout_bytes = 2 * layout * sizeof(float2);
-  const size_t need = layout_bytes + ss_radon_scratch(dp, j0, j1, nslices);
+  // the limit counts the one-ray layouts in any form
+  const size_t need = 16 * (size_t)nslices * p->g.n * p->g.pitch + ss_radon_scratch(dp, j0, j1, nslices);
   if (need > (size_t)RAFT_SS_NOALLOC_SCRATCH_BYTES)
     return ss_set_error(RAFT_SS_EINVAL,
                         "radon_noalloc: %d slice(s) of %d x %d need %zu bytes of workspace, more than the %zu of "

@@ -50,3 +50,46 @@ def test_backprojection_planes(n, R, A, sc):
         assert _rel(p.backprojection(x).cpu().numpy(), ref) <= REL
         assert _rel(p.backprojection(x[1]).cpu().numpy(), ref[1]) <= REL
         assert _rel(p.backprojection(x, angles=(j0, j1)).cpu().numpy(), pref) <= REL
+
+
+def _radon_close(got, ref):
+    return _rel(got, ref) <= REL
+
+
+@pytest.mark.parametrize("n,R,A,sc", GEO)
+def test_radon_planes(n, R, A, sc):
+    """Every slice count that a group of planes can end on, whole and partial ranges, and
+    enough slices that the launch takes the planes undivided."""
+    import torch
+    from pyraft_amd.device import Plan
+    from pyraft_amd.raftypes import libraft  # noqa: F401  (the library under test)
+    p = Plan(n, R, A, sino_corners=sc)
+    blocks = ((R + 127) // 128) * ((A // 2 + 8) // 8)
+    many = min(-(-1024 // blocks), 1200) * 4 + 1  # odd, past SS_RADON_SLAB_BLOCKS in every form
+    x = np.random.default_rng(n * A + R).random((7, n, n)).astype(np.float32)
+    ref = np.stack([O.radon(v.astype(np.float64), R, A, **_geo(sc)) for v in x])
+    xs = torch.from_numpy(x).cuda()
+    j0, j1 = A // 3, max(A // 3 + 1, A - 1)
+    for s in (1, 2, 3, 5, many):
+        print("radon planes", n, R, A, sc, "slices", s, flush=True)
+        idx = torch.arange(s, device="cuda") % 7
+        own = ref[np.arange(s) % 7]
+        got = p.radon(xs[idx]).cpu().numpy()
+        assert _radon_close(got, own), s
+        assert _radon_close(got[-1], own[-1]), s
+        part = p.radon(xs[idx], angle_major=True, angles=(j0, j1)).cpu().numpy()
+        assert _radon_close(part[:, j0:j1], own.transpose(0, 2, 1)[:, j0:j1]), s
+
+
+@pytest.mark.parametrize("n,R,A,slices", [(33, 40, 9, 5), (64, 63, 17, 4), (65, 66, 24, 1201)])
+def test_mesh_radon_planes(n, R, A, slices):
+    import torch
+    from pyraft_amd.device import Plan
+    r = np.random.default_rng(n)
+    t, th = np.sort(r.uniform(-1.0, 1.0, R)), np.sort(r.uniform(0.0, PI, A))
+    x = r.random((4, n, n)).astype(np.float32)
+    ref = np.stack([O.radon_withmesh(v.astype(np.float64), t, th) for v in x])
+    p = Plan.mesh(n, t, th)
+    idx = np.arange(slices) % 4
+    got = p.radon(torch.from_numpy(x).cuda()[torch.from_numpy(idx).cuda()]).cpu().numpy()
+    assert _rel(got, ref[idx]) <= REL and _rel(got[-1], ref[idx[-1]]) <= REL
