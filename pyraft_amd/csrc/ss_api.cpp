@@ -249,7 +249,9 @@ static void radon_symmetry(const SSGeom& g, const std::vector<SSAngle>& angles, 
 static int bp_variants(raft_ss_plan* p) {
   p->rt_variant = -1;
   for (int v = 0; v < SS_BP_NVARIANTS; ++v) rt_staging(p->h_angles, v, &p->rt_window_v[v], &p->rt_angles_v[v]);
-  for (int v : {SS_RT_DEFAULT_VARIANT, 0, 1, 2, 4, 5})
+  // small images take 2 rows per thread (us, 4 rows against 2: 256^2 x 180 27 / 23, 512^2 x 720
+  // 58 / 55, 64 of those 1426 / 1500, 2048^2 x 1500 627 / 660)
+  for (int v : {p->g.n <= 384 ? 1 : SS_RT_DEFAULT_VARIANT, SS_RT_DEFAULT_VARIANT, 0, 1, 2, 4, 5})
     if (p->rt_variant < 0 && p->rt_angles_v[v] > 0) p->rt_variant = v;
   int first = -1;
   for (int v = 0; v < SS_BP_NVARIANTS; ++v) {
@@ -708,16 +710,17 @@ extern "C" int raft_ss_radon_transpose_range(const raft_ss_plan* p, const float*
   hipStream_t stream = as_stream(stream_);
   const SSDevPlan dp = p->dev();
   const float* sT = d_sino;
-  const size_t sino_floats = angle_major ? 0 : (size_t)nslices * p->g.nrays * p->g.nangles;
-  const size_t scratch = ss_radon_transpose_scratch(dp, nslices);
+  const bool pixels = dp.rt_angles > 0;  // reads either layout
+  const size_t sino_floats = angle_major || pixels ? 0 : (size_t)nslices * p->g.nrays * p->g.nangles;
+  const size_t scratch = ss_radon_transpose_scratch(dp, j0, j1, nslices);
   Scratch ws;
   HIP_TRY(ws.alloc(sino_floats * sizeof(float) + scratch, stream));
-  if (!angle_major) {
+  if (sino_floats) {
     HIP_TRY(ss_launch_sino_to_t(d_sino, ws.as<float>(), p->g.nrays, p->g.nangles, nslices, stream));
     sT = ws.as<float>();
   }
-  HIP_TRY(ss_launch_radon_transpose(dp, sT, j0, j1, nslices, d_image, scratch ? ws.as<float>() + sino_floats : nullptr,
-                                    stream));
+  HIP_TRY(ss_launch_radon_transpose(dp, sT, !angle_major && pixels, j0, j1, nslices, d_image,
+                                    scratch ? ws.as<float>() + sino_floats : nullptr, stream));
   return 0;
 }
 

@@ -283,22 +283,31 @@ extern "C" int raft_ss_plan_tune_transpose(raft_ss_plan* p, int nslices, int rep
     return p->rt_variant;
   }
   const int n = p->g.n, R = p->g.nrays, A = p->g.nangles;
+  size_t scratch_bytes = 0;  // the largest variant's planes and partial images
+  const int keep = p->rt_variant;
+  for (int v = 0; v < SS_BP_NVARIANTS; ++v)
+    if (p->rt_angles_v[v] > 0) {
+      p->rt_variant = v;
+      scratch_bytes = std::max(scratch_bytes, ss_radon_transpose_scratch(p->dev(), 0, A, nslices));
+    }
+  p->rt_variant = keep;
   DevBuf ws;
-  HIP_TRY(ws.alloc(sizeof(float) * (size_t)nslices * (2 * (size_t)R * A + (size_t)n * n), stream));
+  const size_t sino_floats = ((size_t)nslices * R * A + 3) & ~(size_t)3;
+  const size_t img_floats = ((size_t)nslices * n * n + 3) & ~(size_t)3;
+  HIP_TRY(ws.alloc(sizeof(float) * (sino_floats + img_floats) + scratch_bytes, stream));
   float* sinoT = ws.as<float>();
-  float* img = sinoT + (size_t)nslices * R * A;
-  float* scratch = img + (size_t)nslices * n * n;  // the pre-scaled sinogram
+  float* img = sinoT + sino_floats;
+  float* scratch = img + img_floats;
   HIP_TRY(ss_launch_fill(sinoT, 1.0f, (size_t)nslices * R * A, stream));
   TuneEntry te;
   int best = -1;
-  const int keep = p->rt_variant;
   for (int v = 0; v < SS_BP_NVARIANTS; ++v) {
     te.times[v] = -1.0;
     if (p->rt_angles_v[v] <= 0) continue;
     p->rt_variant = v;
     const SSDevPlan dp = p->dev();
     auto run = [&]() -> int {
-      HIP_TRY(ss_launch_radon_transpose(dp, sinoT, 0, A, nslices, img, scratch, stream));
+      HIP_TRY(ss_launch_radon_transpose(dp, sinoT, 0, 0, A, nslices, img, scratch, stream));
       return 0;
     };
     rc = time_best(run, reps, stream, &te.times[v]);

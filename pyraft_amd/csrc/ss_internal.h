@@ -132,6 +132,7 @@ struct raft_ss_plan {
     p.rt_variant = rt_variant >= 0 ? rt_variant : 0;
     p.rt_window = rt_variant >= 0 ? rt_window_v[rt_variant] : 0;
     p.rt_angles = rt_variant >= 0 ? rt_angles_v[rt_variant] : 0;
+    p.rt_sym = (radon_turn ? 1 : 0) | (radon_mirror ? 2 : 0);
     return p;
   }
   ~raft_ss_plan() {

@@ -53,6 +53,7 @@ struct SSDevPlan {
   // staged per angle and angles per stage; rt_angles = 0: not available (rays closer than
   // one cell on some angle), the line form runs instead
   int rt_variant, rt_window, rt_angles;
+  int rt_sym;  // the Radon's symmetries: 1 half turn, 2 mirror
 };
 
 // ---- batched execution over slices of different geometry
@@ -96,6 +97,15 @@ enum { SS_PLANES_NONE = 0, SS_PLANES_QUAD = 1, SS_PLANES_PAIR = 2, SS_PLANES_SLI
 static inline __host__ __device__ int ss_planes_slices(int kind) {
   return kind == SS_PLANES_QUAD ? 1 : (kind == SS_PLANES_PAIR ? 2 : 4);
 }
+// the exact transpose's further forms: a slice and its half turn, two slices, one
+enum { SS_RT_TURN = 4, SS_RT_TWO = 5, SS_RT_ONE = 6 };
+static inline __host__ __device__ int ss_rt_slices(int kind) {
+  return kind <= SS_PLANES_SLICES ? ss_planes_slices(kind) : (kind == SS_RT_TWO ? 2 : 1);
+}
+static inline __host__ __device__ int ss_rt_planes(int kind) {
+  return kind <= SS_PLANES_SLICES ? 4 : (kind == SS_RT_ONE ? 1 : 2);
+}
+#define SS_RT_SAME_SLICES 8  // launches of up to this many slices sum in one slice's order
 static inline int ss_planes_groups(int kind, int nslices) {
   return (nslices + ss_planes_slices(kind) - 1) / ss_planes_slices(kind);
 }
@@ -181,10 +191,12 @@ hipError_t ss_launch_backprojection(const SSDevPlan& p, const float* sinoT, int 
                                     float* out, SSEmUpdateArgs em, float* scratch, hipStream_t stream);
 
 // ---- exact transpose of the Radon (reads angle-major sinogram)
-// scratch bytes the transpose needs: one transposed n x n FP32 image per slice, where the
-// lines of the angles that walk image columns accumulate before k_transpose_add
-size_t ss_radon_transpose_scratch(const SSDevPlan& p, int nslices);
-hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int j0, int j1, int nslices,
+// scratch bytes the transpose needs: the pre-scaled planes and, with angle groups, the partial
+// images; the line form's transposed n x n FP32 image per slice (where the lines of the angles
+// that walk image columns accumulate before k_transpose_add)
+size_t ss_radon_transpose_scratch(const SSDevPlan& p, int j0, int j1, int nslices);
+// in_cols: sinoT is in the (R, A) layout (pixel-driven form only: p.rt_angles > 0)
+hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int in_cols, int j0, int j1, int nslices,
                                      float* out, float* scratch, hipStream_t stream);
 
 // ---- batched forms (items: gather = SS_GATHER_TILE^2 tiles; radon = 64-ray groups x blocks of

@@ -1787,12 +1787,16 @@ int ss_bp_tiles(int n, int variant, int planes) {
   return ss_bp_tile_cols(n, planes) * ((ss_bp_rows(n, planes) + th - 1) / th);
 }
 
-int ss_bp_groups(const SSDevPlan& p, int j0, int j1, int nslices) {
-  const long long tiles = (long long)ss_bp_tiles(p.g.n, p.bp_variant, ss_bp_planes(p, j0, j1)) * std::max(nslices, 1);
-  const int nj = j1 - j0;
+// angle groups of a launch of `tiles` blocks over nj angles (the rule at SS_BP_GROUP_SCALE)
+static int ss_angle_groups(long long tiles, int nj) {
   if (tiles <= 0 || nj < 2 * SS_BP_GROUP_ANGLES) return 1;
   const double g = SS_BP_GROUP_SCALE * sqrt((double)SS_BP_ROUND_BLOCKS * nj / (double)tiles);
   return (int)std::max(1.0, std::min(floor(g + 0.5), (double)(nj / SS_BP_GROUP_ANGLES)));
+}
+
+int ss_bp_groups(const SSDevPlan& p, int j0, int j1, int nslices) {
+  return ss_angle_groups((long long)ss_bp_tiles(p.g.n, p.bp_variant, ss_bp_planes(p, j0, j1)) * std::max(nslices, 1),
+                         j1 - j0);
 }
 
 size_t ss_bp_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
@@ -2207,15 +2211,16 @@ __global__ __launch_bounds__(256) void k_transpose_add(const float* __restrict__
 }
 
 // irregular rays: scatter their exact contributions
-__global__ __launch_bounds__(256) void k_radon_transpose_fixup(SSDevPlan p, const float* __restrict__ qT, int j0,
-                                                               int j1, float* __restrict__ out) {
+// (qT angle-major, or with in_cols in the (R, A) layout)
+__global__ __launch_bounds__(256) void k_radon_transpose_fixup(SSDevPlan p, const float* __restrict__ qT, int in_cols,
+                                                               int j0, int j1, float* __restrict__ out) {
   const int id = p.irregular[blockIdx.x];
   const int slice = blockIdx.y;
   const int n = p.g.n, R = p.g.nrays, A = p.g.nangles;
   const int j = id / R, k = id % R;
   if (j < j0 || j >= j1) return;
   const SSAngle& a = p.angles[j];
-  const float v = qT[((size_t)slice * A + j) * R + k] * a.delta;
+  const float v = qT[(size_t)slice * A * R + (in_cols ? (size_t)k * A + j : (size_t)j * R + k)] * a.delta;
   float* img = out + (size_t)slice * n * n;
   for (int s = threadIdx.x; s < n; s += blockDim.x) {
     if (!ss_radon_sample_valid(p.g, a, k, s)) continue;
@@ -2251,257 +2256,384 @@ __global__ __launch_bounds__(256) void k_radon_transpose_fixup(SSDevPlan p, cons
 // to a staged base ray, FP32 offsets per pixel, and staged (Delta q_k, Delta q_{k+1})
 // pairs.  Both branches add into the same pixels in one pass.
 //
-// Validity.  A sample is valid when its FP64 predicate coordinate x lies in [0, n-1); on
-// a regular angle x is within ~(k + s) 2^-33 cells of the Q32.32 trajectory, so every
-// sample whose cell lies in [1, n-3] is valid and pixels p in [2, n-3] need no test.  In
-// tiles holding pixels p < 2 or p > n-3 a regular angle tests, at those pixels, each
-// candidate's position on its line, u = p - f gs or p + (1 - f) gs (gs the signed
-// spacing), which the FP32
-// evaluation gives within ~2e-5 cells: u in [eps, n-1-eps) is valid, u < -eps or
-// u >= n-1+eps is not, and only u within eps = 1e-3 of 0 or n-1 reads the candidate's
-// exact range (s in [lo_k, hi_k]).  An angle that is not regular (degenerate, or with
-// irregular rays) reads the exact range of every candidate; irregular rays have empty
-// ranges here and the fixup kernel adds them.  The weights are FP32 evaluations of the
-// forward's (~1e-5 cells).
+// Validity.  A sample is valid when its FP64 predicate coordinate x lies in [0, n-1), and x is
+// within ~(k + s) 2^-33 cells of the Q32.32 trajectory.  A candidate with weight lies within a
+// cell of its pixel, so on pixels p in [1, n-2] every candidate that counts is valid (one at
+// the very end of the line has weight zero there), and the tiles test nothing; the image's
+// first and last rows and columns are made by blocks of their own (ss_rtp_border), with the
+// tests.  Irregular rays enter as zeros and the fixup kernel adds them.  The weights are FP32
+// evaluations of the forward's (~1e-5 cells).
+//
+// What bounds it: VALU issue (8 instructions per update with one plane, 5 with two, 3.5 with
+// four), once the launch has enough blocks and none of the slow border tiles runs last.
+// From the (R, A) layout, us before and after the planes, angle groups and border blocks:
+// 2048^2 x 1500 2440 -> 660; 1024^2 x 720 550 -> 115; 512^2 x 720 490 -> 57, 64 of those
+// 4110 -> 1590; 231^2 x 1000 (a limited arc) 920 -> 35.  Border tiles that test every pixel in
+// place of the border blocks: 980 at 2048^2 x 1500 (the slow tiles end last).
 // =====================================================================================
 
 #ifndef RTP_UNROLL
 #define RTP_UNROLL 2  // angles per unrolled step of the pixel-driven transpose
 #endif
 
-struct RTPAngle {
-  float f0, b, c, g;
-  int flag;  // 0: no candidate ray on the detector, 1: no validity test, 2: test by position
-             // (regular angle, tile at a line end), 3: exact ranges (angle not regular)
+struct alignas(16) RTPAngle {
+  float f0, b, c, g;  // read together by one 16-byte LDS read
+  int flag;  // 0: no candidate ray on the detector, 1: regular angle, 2: not regular
   int base;
   int branch_a;
   float gs;  // signed ray spacing in cells (gamma 2^-32)
 };
 
-// SL = 2: the block takes two slices of a launch and shares each pixel's geometry (kappa,
-// floor, fraction, weights) between them.  win holds, per staged angle, the window of
-// Delta q_k for rays base .. base + W (rt_window W; windows WS = W + 4 rays apart),
-// copied straight from the pre-scaled sinogram into LDS: one float per ray, or with two
-// slices the pair (slice 0, slice 1) per ray, as the pre-scaled copy interleaves them.  A
-// pixel reads its two candidates with one two-word (two-pair) LDS read.
-template <int STAGE, int SL>
+// Parameters of angle j for the tile [c0, c0 + 32) x [r0, r0 + th): the tile origin's kappa
+// relative to the base ray, its slopes, the spacing
+__device__ __forceinline__ RTPAngle ss_rtp_params(const SSDevPlan& p, int j, int c0, int r0, int th) {
+  RTPAngle q{0.f, 0.f, 0.f, 0.f, 0, 0, 0, 0.f};
+  const SSAngle& a = p.angles[j];
+  const double kb = a.branch_a ? -a.rt_b : a.rt_ig;  // kappa per column
+  const double kc = a.branch_a ? a.rt_ig : -a.rt_b;  // kappa per row
+  const double K = -a.rt_a0 + (double)c0 * kb + (double)r0 * kc;
+  const double eb = (double)(BP_TILE_W - 1) * kb, ec = (double)(th - 1) * kc;
+  const double kmin = K + fmin(0.0, eb) + fmin(0.0, ec);
+  const double kmax = K + fmax(0.0, eb) + fmax(0.0, ec);
+  const double base = floor(kmin) - 1.0;
+  q.f0 = (float)(K - base);
+  q.b = (float)kb;
+  q.c = (float)kc;
+  q.g = (float)(fabs((double)a.gamma) * (1.0 / SS_FIX_ONE));
+  q.gs = (float)((double)a.gamma * (1.0 / SS_FIX_ONE));
+  q.base = (int)base;
+  q.branch_a = a.branch_a;
+  q.flag = kmax < -1.0 || kmin >= (double)p.g.nrays ? 0 : (a.regular ? 1 : 2);
+  return q;
+}
+
+// The planes of a launch (SSRtPlanes; ss_launch_radon_transpose chooses): a block's pixel tile
+// and PL planes that share each pixel's geometry (kappa, floor, weights).  QUAD, PAIR and
+// SLICES as for the Radon (ss_plane): the half turn of pixel (r, c) has the ray coordinate
+// R - 1 - kappa, the mirror (r, n-1-c) has kappa at the angle pi - theta.  TURN: one slice and
+// its half turn; TWO: two slices; ONE: the pixel alone.
+__device__ __host__ __forceinline__ SSPlane ss_rt_plane(int kind, int z) {
+  if (kind == SS_RT_TURN) return SSPlane{0, z != 0, false};
+  return ss_plane(kind, z);  // SS_RT_TWO and SS_RT_ONE: slices
+}
+
+// win holds, per staged angle, the planes' values of rays base .. base + W (rt_window W;
+// windows WS = W + 4 rays apart), copied straight from the pre-scaled copy (k_rtp_planes) into
+// LDS: the PL values of a ray together.  A pixel reads its two candidates with two reads of
+// 4 PL bytes.
+template <int STAGE>
 struct SSRtpLds {
-  alignas(16) float win[2 * STAGE];  // STAGE pairs' worth: rt_angles x WS floats
+  alignas(16) float win[2 * STAGE];  // J windows of PL x WS floats (border: partial sums)
   RTPAngle par[64];
 };
 
-// sl: the sinogram [A][R] pre-scaled by each angle's Delta; with SL = 2 the two slices
-// interleaved, [A][R][2]
-template <int ROWS, int STAGE, int SL>
-__device__ __forceinline__ void ss_rtp_item(const SSDevPlan& p, const float* __restrict__ sl, int j0, int j1,
-                                            int c0, int r0, float* __restrict__ out0, float* __restrict__ out1,
-                                            SSRtpLds<STAGE, SL>& lds) {
-  const int n = p.g.n, R = p.g.nrays;
+#define RTP_EDGE_SLICES 4  // slices of a border block (they share the geometry)
+
+// A border block: 32 pixels of an image's first or last row or column (`side` 0, 1: rows, 2,
+// 3: columns; segment `seg`), over angles [j0, j1), for slices s0 .. s0 + RTP_EDGE_SLICES - 1
+// (out: the first slice's image, or its partial image).
+// Only here can a candidate's sample be off its line: on a regular angle the position on
+// the line decides, u = p - f gs or p + (1 - f) gs, which FP32 gives within ~2e-5 cells (u in
+// [eps, n-1-eps) is valid, u < -eps or u >= n-1+eps is not) except within eps = 1e-3 of an end
+// and on other angles, which read the candidate's exact range.  Thread: pixel tid % 32,
+// angles tid / 32 mod 8; the eight sums are added in order.
+template <int STAGE>
+__device__ __forceinline__ void ss_rtp_border(const SSDevPlan& p, const float* __restrict__ planes, int kind,
+                                              int nslices, int j0, int j1, int side, int seg, int s0, int ngroups,
+                                              float* __restrict__ out, SSRtpLds<STAGE>& lds) {
+  const int n = p.g.n, R = p.g.nrays, A = p.g.nangles, PL = ss_rt_planes(kind);
+  const int tid = threadIdx.x, lane = tid & 63, i = tid & 31, sub = tid >> 5;
+  const bool is_row = side < 2;
+  const int fixed = side & 1 ? n - 1 : 0;
+  const int row = is_row ? fixed : seg * 32 + i, col = is_row ? seg * 32 + i : fixed;
+  const int c0 = col & ~31, r0 = row & ~31;  // the pixel's 32 x 32 tile
+  const bool on = row < n && col < n && (is_row || (row > 0 && row < n - 1));
+  const float ftx = (float)(col - c0), fty = (float)(row - r0), top = (float)(n - 1);
+  constexpr float eps = 1e-3f;
+  const float* src[RTP_EDGE_SLICES];
+#pragma unroll
+  for (int s = 0; s < RTP_EDGE_SLICES; ++s) {
+    const int slice = min(s0 + s, nslices - 1), per = ss_rt_slices(kind);
+    // the slice's own plane in its group
+    const int z = kind == SS_PLANES_PAIR ? 2 * (slice % 2) : slice % per;
+    src[s] = planes + (size_t)(slice / per) * A * R * PL + z;
+  }
+  float acc[RTP_EDGE_SLICES];
+#pragma unroll
+  for (int s = 0; s < RTP_EDGE_SLICES; ++s) acc[s] = 0.f;
+  for (int ja = j0; ja < j1; ja += SS_WAVE) {
+    const int np = min(SS_WAVE, j1 - ja);
+    __syncthreads();
+    if (tid < np) lds.par[lane] = ss_rtp_params(p, ja + lane, is_row ? seg * 32 : c0, is_row ? r0 : seg * 32, 32);
+    __syncthreads();
+    if (!on) continue;
+    for (int jj = sub; jj < np; jj += 8) {
+      const RTPAngle q = lds.par[jj];
+      if (q.flag == 0) continue;
+      const float kap = fmaf(fty, q.c, fmaf(ftx, q.b, q.f0));
+      const int k = q.base + (int)kap;
+      const float f = __builtin_amdgcn_fractf(kap);
+      float w0 = __builtin_amdgcn_fmed3f(fmaf(-q.g, f, 1.f), 0.f, 1.f);
+      float w1 = __builtin_amdgcn_fmed3f(fmaf(q.g, f, 1.f - q.g), 0.f, 1.f);
+      const int pix = q.branch_a ? row : col;  // the pixel's cell on its sample line
+      if (q.flag == 2 || pix == 0 || pix == n - 1) {
+        const float u0 = fmaf(-f, q.gs, (float)pix), u1 = u0 + q.gs;
+        const int2* rng = p.bounds + (size_t)(ja + jj) * R;
+        const int sline = q.branch_a ? col : row;  // the candidates' sample line
+        bool in0 = q.flag == 1 && u0 >= eps && u0 < top - eps, in1 = q.flag == 1 && u1 >= eps && u1 < top - eps;
+        if ((q.flag == 2 || fabsf(u0) < eps || fabsf(u0 - top) < eps) && (unsigned)k < (unsigned)R) {
+          const int2 b = rng[k];
+          in0 = in0 || (sline >= b.x && sline <= b.y);
+        }
+        if ((q.flag == 2 || fabsf(u1) < eps || fabsf(u1 - top) < eps) && (unsigned)(k + 1) < (unsigned)R) {
+          const int2 b = rng[k + 1];
+          in1 = in1 || (sline >= b.x && sline <= b.y);
+        }
+        w0 = in0 ? w0 : 0.f;
+        w1 = in1 ? w1 : 0.f;
+      }
+      const size_t at = (size_t)(ja + jj) * R;
+      const int k0 = min(max(k, 0), R - 1), k1 = min(max(k + 1, 0), R - 1);
+#pragma unroll
+      for (int s = 0; s < RTP_EDGE_SLICES; ++s) {
+        const float v0 = src[s][(at + k0) * PL], v1 = src[s][(at + k1) * PL];
+        acc[s] = fmaf(w0, k0 == k ? v0 : 0.f, acc[s]);  // 0 off the detector
+        acc[s] = fmaf(w1, k1 == k + 1 ? v1 : 0.f, acc[s]);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < RTP_EDGE_SLICES; ++s) lds.win[(s * 8 + sub) * 32 + i] = acc[s];
+  __syncthreads();
+  // thread (pixel i, slice sub < 4)
+  if (!on || sub >= RTP_EDGE_SLICES || s0 + sub >= nslices) return;
+  float sum = 0.f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) sum += lds.win[(sub * 8 + t) * 32 + i];
+  const size_t img = (size_t)n * n;
+  out[(size_t)(s0 + sub) * ngroups * img + (size_t)row * n + col] = sum;
+}
+
+template <int PL>
+struct SSRtVec {
+  typedef float type __attribute__((ext_vector_type(PL)));
+};
+template <>
+struct SSRtVec<1> {
+  typedef float type;
+};
+template <int PL>
+__device__ __forceinline__ float ss_rt_get(const typename SSRtVec<PL>::type& v, int z) {
+  if constexpr (PL == 1)
+    return v;
+  else
+    return v[z];
+}
+
+// sp: the group's pre-scaled planes [A][R][PL].  out + plane offset: the planes' images (or,
+// PARTIAL, their partial images).
+template <int ROWS, int STAGE, int PL>
+__device__ __forceinline__ void ss_rtp_item(const SSDevPlan& p, const float* __restrict__ sp, int kind, int slice0,
+                                            int nslices, int j0, int j1, int c0, int r0, float* __restrict__ out,
+                                            size_t out_slice, SSRtpLds<STAGE>& lds) {
+  typedef typename SSRtVec<PL>::type vec;
+  const int n = p.g.n, R = p.g.nrays, A = p.g.nangles;
   const int W = p.rt_window;
   const int WS = W + 4;
-  const int J = SL == 2 ? p.rt_angles / 2 : p.rt_angles;  // two windows per angle with two slices
+  const int J = min(SS_WAVE, 2 * STAGE / PL / WS);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tx = tid & 31, ty = tid >> 5;
+  const int tx = PL == 4 ? ss_bp_column(tid) : tid & 31, ty = tid >> 5;
   const int col = c0 + tx;
   constexpr int TH = 8 * ROWS;
-  // two accumulators per pixel and slice (the two candidates' terms) keep the FMA chains short
-  float acc0[SL][ROWS], acc1[SL][ROWS];
+  float acc[ROWS][PL];
   float fty[ROWS];
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
     fty[i] = (float)(ty + 8 * i);
 #pragma unroll
-    for (int z = 0; z < SL; ++z) acc0[z][i] = acc1[z][i] = 0.f;
+    for (int z = 0; z < PL; ++z) acc[i][z] = 0.f;
   }
   const float ftx = (float)tx;
-  // tile pixels along each branch's cell axis: columns (branch B), rows (branch A)
-  const bool inner_b = c0 >= 2 && c0 + BP_TILE_W - 1 <= n - 3;
-  const bool inner_a = r0 >= 2 && r0 + TH - 1 <= n - 3;
+  const int JP = SS_WAVE / J * J;  // parameters of whole stages, up to 64 angles at a time
 
-  for (int jb = j0; jb < j1; jb += J) {
-    const int nj = min(J, j1 - jb);
+  for (int ja = j0; ja < j1; ja += JP) {
+    const int np = min(JP, j1 - ja);
     RTPAngle q{0.f, 0.f, 0.f, 0.f, 0, 0, 0, 0.f};
-    if (lane < nj) {
-      const SSAngle& a = p.angles[jb + lane];
-      const double kb = a.branch_a ? -a.rt_b : a.rt_ig;  // kappa per column
-      const double kc = a.branch_a ? a.rt_ig : -a.rt_b;  // kappa per row
-      const double K = -a.rt_a0 + (double)c0 * kb + (double)r0 * kc;
-      const double eb = (double)(BP_TILE_W - 1) * kb, ec = (double)(TH - 1) * kc;
-      const double kmin = K + fmin(0.0, eb) + fmin(0.0, ec);
-      const double kmax = K + fmax(0.0, eb) + fmax(0.0, ec);
-      const double base = floor(kmin) - 1.0;
-      q.f0 = (float)(K - base);
-      q.b = (float)kb;
-      q.c = (float)kc;
-      q.g = (float)(fabs((double)a.gamma) * (1.0 / SS_FIX_ONE));
-      q.gs = (float)((double)a.gamma * (1.0 / SS_FIX_ONE));
-      q.base = (int)base;
-      q.branch_a = a.branch_a;
-      if (kmax < -1.0 || kmin >= (double)R)
-        q.flag = 0;
-      else if (!a.regular)
-        q.flag = 3;
-      else if (a.branch_a ? inner_a : inner_b)
-        q.flag = 1;
-      else
-        q.flag = 2;
-    }
-    const bool checked = __ballot(lane < nj && q.flag >= 2) != 0ull;
-    __syncthreads();  // the previous stage is done with win / par
-    if (wv == 0) {
-      lds.par[lane].f0 = q.f0;
-      lds.par[lane].b = q.b;
-      lds.par[lane].c = q.c;
-      lds.par[lane].g = q.g;
-      lds.par[lane].flag = q.flag;
-      lds.par[lane].base = q.base;
-      lds.par[lane].branch_a = q.branch_a;
-      lds.par[lane].gs = q.gs;
-    }
-    // staging: wave wv fills the windows of angles wv, wv+4, ... with direct buffer -> LDS
-    // copies, one ray per lane; rays outside [0, R) (and every ray of an angle without
-    // candidates) read 0 through the buffer's range check.  kappa - base >= 1 for every
-    // pixel, so the truncated offset is the floor and stays below W.
-    for (int jj = wv; jj < nj; jj += 4) {
-      const int fl = __builtin_amdgcn_readlane(q.flag, jj);
-      const int bs = __builtin_amdgcn_readlane(q.base, jj);
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(sl + (size_t)(jb + jj) * R * SL), (short)0, R * SL * (int)sizeof(float), 0x00020000);
-      float* dst = lds.win + jj * SL * WS;
-      for (int w = 0; w < SL * (W + 1); w += 64) {
-        // the whole offset in the register (none in the instruction's offset field), so
-        // the range check sees a ray below 0 as out of range
-        int off = fl != 0 ? (SL * bs + w + lane) * (int)sizeof(float) : 0x7ffffff0;
-        __asm__ volatile("" : "+v"(off));
-        if (w + lane < SL * (W + 1))  // active lanes write dst[w + lane]: stay in this window
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (ss_lds_ptr)(dst + w), 4, off, 0, 0, 0);
+    if (lane < np) q = ss_rtp_params(p, ja + lane, c0, r0, TH);
+    const unsigned long long near = __ballot(lane < np && q.flag != 0);
+    for (int js = 0; js < np; js += J) {
+      const int jb = ja + js, nj = min(J, np - js);
+      const bool every = __popcll(near >> js & (~0ull >> (SS_WAVE - nj))) == nj;
+      __syncthreads();  // the previous stage is done with win / par
+      if (js == 0 && wv == 0) {
+        lds.par[lane].f0 = q.f0;
+        lds.par[lane].b = q.b;
+        lds.par[lane].c = q.c;
+        lds.par[lane].g = q.g;
+        lds.par[lane].flag = q.flag;
       }
-    }
-    __syncthreads();
-    if (!checked) {
+      // staging: wave wv fills the windows of angles wv, wv+4, ... with direct buffer -> LDS
+      // copies: with four planes a ray per lane, else a float per lane.  Rays outside [0, R)
+      // (and every ray of an angle without candidates) read 0 through the buffer's range
+      // check.  kappa - base >= 1 for every pixel, so the truncated offset is the floor and
+      // stays below W.
+      for (int jj = wv; jj < nj; jj += 4) {
+        const int fl = __builtin_amdgcn_readlane(q.flag, js + jj);
+        const int bs = __builtin_amdgcn_readlane(q.base, js + jj);
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(sp + (size_t)(jb + jj) * R * PL), (short)0,
+                                              R * PL * (int)sizeof(float), SS_RSRC_DWORD3);
+        float* dst = lds.win + jj * PL * WS;
+        constexpr int UNIT = PL == 4 ? 4 : 1;         // floats per lane
+        const int units = PL * (W + 1) / UNIT;
+        for (int w = 0; w < units; w += 64) {
+          // the whole offset in the register (none in the instruction's offset field), so
+          // the range check sees a ray below 0 as out of range
+          int off = fl != 0 ? (PL * bs + UNIT * (w + lane)) * (int)sizeof(float) : 0x7ffffff0;
+          __asm__ volatile("" : "+v"(off));
+          if (w + lane < units) {  // active lanes write their unit: stay in this window
+            if constexpr (PL == 4)
+              __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (ss_lds_ptr)(dst + UNIT * w), 16, off, 0, 0, 0);
+            else
+              __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (ss_lds_ptr)(dst + UNIT * w), 4, off, 0, 0, 0);
+          }
+        }
+      }
+      __syncthreads();
+      auto add = [&](const ss_f32x4& par, const vec* wrow) {  // par: f0, b, c, g
+        const float g1 = 1.f - par.w;
+        const float t0 = fmaf(ftx, par.y, par.x);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+          const float kap = fmaf(fty[i], par.z, t0);
+          const int kr = (int)kap;
+          const float f = __builtin_amdgcn_fractf(kap);
+          const float w0 = __builtin_amdgcn_fmed3f(fmaf(-par.w, f, 1.f), 0.f, 1.f);
+          const float w1 = __builtin_amdgcn_fmed3f(fmaf(par.w, f, g1), 0.f, 1.f);
+          const vec q0 = wrow[kr], q1 = wrow[kr + 1];
+#pragma unroll
+          for (int z = 0; z < PL; ++z)
+            acc[i][z] = fmaf(w1, ss_rt_get<PL>(q1, z), fmaf(w0, ss_rt_get<PL>(q0, z), acc[i][z]));
+        }
+      };
+      if (every) {
 #pragma unroll RTP_UNROLL
-      for (int jj = 0; jj < nj; ++jj) {
-        const float f0 = lds.par[jj].f0, pb = lds.par[jj].b, pc = lds.par[jj].c, g = lds.par[jj].g;
-        const float g1 = 1.f - g;
-        const float* wrow = lds.win + jj * SL * WS;
-        const float t0 = fmaf(ftx, pb, f0);
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-          const float kap = fmaf(fty[i], pc, t0);
-          const int kr = (int)kap;
-          const float f = __builtin_amdgcn_fractf(kap);
-          const float w0 = __builtin_amdgcn_fmed3f(fmaf(-g, f, 1.f), 0.f, 1.f);
-          const float w1 = __builtin_amdgcn_fmed3f(fmaf(g, f, g1), 0.f, 1.f);
-          if constexpr (SL == 2) {
-            const float2 t0 = reinterpret_cast<const float2*>(wrow)[kr];
-            const float2 t1 = reinterpret_cast<const float2*>(wrow)[kr + 1];
-            acc0[0][i] = fmaf(w0, t0.x, acc0[0][i]);
-            acc1[0][i] = fmaf(w1, t1.x, acc1[0][i]);
-            acc0[1][i] = fmaf(w0, t0.y, acc0[1][i]);
-            acc1[1][i] = fmaf(w1, t1.y, acc1[1][i]);
-          } else {
-            acc0[0][i] = fmaf(w0, wrow[kr], acc0[0][i]);
-            acc1[0][i] = fmaf(w1, wrow[kr + 1], acc1[0][i]);
-          }
-        }
-      }
-    } else {
-      for (int jj = 0; jj < nj; ++jj) {
-        const int flag = __builtin_amdgcn_readfirstlane(lds.par[jj].flag);
-        if (flag == 0) continue;
-        const float f0 = lds.par[jj].f0, pb = lds.par[jj].b, pc = lds.par[jj].c, g = lds.par[jj].g;
-        const float g1 = 1.f - g;
-        const float* wrow = lds.win + jj * SL * WS;
-        const float t0 = fmaf(ftx, pb, f0);
-        const int base = lds.par[jj].base;
-        const int branch_a = __builtin_amdgcn_readfirstlane(lds.par[jj].branch_a);
-        const float gs = lds.par[jj].gs;
-        const int2* rng = p.bounds + (size_t)(jb + jj) * R;
-        const float top = (float)(n - 1);
-        constexpr float eps = 1e-3f;
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-          const float kap = fmaf(fty[i], pc, t0);
-          const int kr = (int)kap;
-          const float f = __builtin_amdgcn_fractf(kap);
-          float w0 = __builtin_amdgcn_fmed3f(fmaf(-g, f, 1.f), 0.f, 1.f);
-          float w1 = __builtin_amdgcn_fmed3f(fmaf(g, f, g1), 0.f, 1.f);
-          const int row = r0 + ty + 8 * i;
-          const int pix = branch_a ? row : col;  // the pixel's cell on its sample line
-          if (flag == 3 || (flag == 2 && (pix <= 1 || pix >= n - 2))) {
-            const int sline = branch_a ? col : row;  // the candidates' sample line
-            const float pcell = (float)pix;
-            const int k0 = base + kr;
-            int keep;
-            if (flag == 2) {
-              // position on the line decides, except within eps of either end
-              const float u0 = fmaf(-f, gs, pcell), u1 = u0 + gs;
-              keep = ((u0 >= eps && u0 < top - eps) ? 1 : 0) | ((u1 >= eps && u1 < top - eps) ? 2 : 0);
-              const bool amb0 = fabsf(u0) < eps || fabsf(u0 - top) < eps;
-              const bool amb1 = fabsf(u1) < eps || fabsf(u1 - top) < eps;
-              if (amb0 && (unsigned)k0 < (unsigned)R) {
-                const int2 b0 = rng[k0];
-                keep |= (sline >= b0.x && sline <= b0.y) ? 1 : 0;
-              }
-              if (amb1 && (unsigned)(k0 + 1) < (unsigned)R) {
-                const int2 b1 = rng[k0 + 1];
-                keep |= (sline >= b1.x && sline <= b1.y) ? 2 : 0;
-              }
-            } else {
-              // the candidates' exact ranges
-              int2 b0 = make_int2(0, -1), b1 = make_int2(0, -1);
-              if ((unsigned)k0 < (unsigned)R) b0 = rng[k0];
-              if ((unsigned)(k0 + 1) < (unsigned)R) b1 = rng[k0 + 1];
-              keep = ((sline >= b0.x && sline <= b0.y) ? 1 : 0) | ((sline >= b1.x && sline <= b1.y) ? 2 : 0);
-            }
-            w0 = (keep & 1) ? w0 : 0.f;
-            w1 = (keep & 2) ? w1 : 0.f;
-          }
-          if constexpr (SL == 2) {
-            const float2 t0 = reinterpret_cast<const float2*>(wrow)[kr];
-            const float2 t1 = reinterpret_cast<const float2*>(wrow)[kr + 1];
-            acc0[0][i] = fmaf(w0, t0.x, acc0[0][i]);
-            acc1[0][i] = fmaf(w1, t1.x, acc1[0][i]);
-            acc0[1][i] = fmaf(w0, t0.y, acc0[1][i]);
-            acc1[1][i] = fmaf(w1, t1.y, acc1[1][i]);
-          } else {
-            acc0[0][i] = fmaf(w0, wrow[kr], acc0[0][i]);
-            acc1[0][i] = fmaf(w1, wrow[kr + 1], acc1[0][i]);
-          }
-        }
+        for (int jj = 0; jj < nj; ++jj)
+          add(*reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]),
+              reinterpret_cast<const vec*>(lds.win + jj * PL * WS));
+      } else {
+        for (int jj = 0; jj < nj; ++jj)
+          if (__builtin_amdgcn_readfirstlane(lds.par[js + jj].flag))
+            add(*reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]),
+                reinterpret_cast<const vec*>(lds.win + jj * PL * WS));
       }
     }
   }
-  if (col >= n) return;
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
     const int row = r0 + ty + 8 * i;
-    if (row >= n) continue;
-    out0[(size_t)row * n + col] = acc0[0][i] + acc1[0][i];
-    if constexpr (SL == 2) out1[(size_t)row * n + col] = acc0[1][i] + acc1[1][i];
+#pragma unroll
+    for (int z = 0; z < PL; ++z) {
+      const SSPlane pl = ss_rt_plane(kind, z);
+      // tiles cover the rows (and, with the mirror, the columns) up to the middle; a pixel
+      // that is its own image is stored once
+      const int mr = pl.turn ? 1 : 0, mc = pl.turn != pl.mirror ? 1 : 0;
+      if (slice0 + pl.slice >= nslices || row >= n || col >= n) continue;
+      if (kind == SS_PLANES_QUAD ? 2 * row + mr > n - 1 || 2 * col + mc > n - 1
+                                 : (kind == SS_PLANES_PAIR || kind == SS_RT_TURN) && 2 * row + mr > n - 1)
+        continue;
+      const int zr = mr ? n - 1 - row : row, zc = mc ? n - 1 - col : col;
+      if (zr == 0 || zr == n - 1 || zc == 0 || zc == n - 1) continue;  // ss_rtp_border's
+      out[(size_t)pl.slice * out_slice + (size_t)zr * n + zc] = acc[i][z];
+    }
   }
 }
 
 // Blocks per CU the compiler must fit (registers): eight 256-thread blocks (8 waves per
-// SIMD, 64 VGPRs) for single-slice tiles of up to 4 rows per thread, whose register need
-// is near 64 (2048^2 x 1500: 2.66 -> 2.57 ms); slice pairs would spill under that bound.
-#ifndef RTP_BLOCKS_SMALL
-#define RTP_BLOCKS_SMALL 8
-#endif
-#define RTP_MIN_BLOCKS(ROWS, SL) ((ROWS) <= 4 && (SL) == 1 ? RTP_BLOCKS_SMALL : 1)
+// SIMD, 64 VGPRs) for one-plane tiles of up to 4 rows per thread, whose register need is
+// near 64; the planes need more.
+#define RTP_MIN_BLOCKS(ROWS, PL) ((ROWS) <= 4 && (PL) == 1 ? 8 : ((ROWS) <= 4 ? 4 : 1))
 
-// slices slice0 + blockIdx.z * SL .. + SL - 1
-template <int ROWS, int STAGE, int SL>
-__global__ __launch_bounds__(256, RTP_MIN_BLOCKS(ROWS, SL)) void k_radon_transpose_px(SSDevPlan p, const float* __restrict__ qT, int j0, int j1,
-                                                            int slice0, float* __restrict__ out) {
-  __shared__ SSRtpLds<STAGE, SL> lds;
-  const size_t slice = (size_t)slice0 + (size_t)blockIdx.z * SL;
-  const size_t sino = (size_t)p.g.nangles * p.g.nrays, img = (size_t)p.g.n * p.g.n;
-  // the pre-scaled copy holds slice pairs interleaved in the pairs' own space
-  ss_rtp_item<ROWS, STAGE, SL>(p, qT + slice * sino, j0, j1, blockIdx.x * BP_TILE_W, blockIdx.y * 8 * ROWS,
-                               out + slice * img, out + (slice + SL - 1) * img, lds);
+// Blocks [0, nborder): the border segments (4 sides x ceil(n / 32)) of each RTP_EDGE_SLICES
+// slices and angle group; then the tiles, tile fastest, then z = group * ngroups + g: planes
+// group `group` over the g-th of ngroups equal parts of the angles [j0, j1).  With ngroups > 1
+// the parts' partial images go to out[slice][g][n][n], for k_bp_groups_finish.
+template <int ROWS, int STAGE, int PL>
+__global__ __launch_bounds__(256, RTP_MIN_BLOCKS(ROWS, PL)) void k_radon_transpose_px(
+    SSDevPlan p, const float* __restrict__ planes, int kind, int nslices, int j0, int j1, int ngroups, int nborder,
+    int cols, int rows, float* __restrict__ out) {
+  __shared__ SSRtpLds<STAGE> lds;
+  const size_t img = (size_t)p.g.n * p.g.n;
+  const long long nj = j1 - j0;
+  int id = blockIdx.x;
+  if (id < nborder) {
+    const int segs = (p.g.n + 31) / 32, part = id / (4 * segs);
+    const int g = part % ngroups;
+    ss_rtp_border<STAGE>(p, planes, kind, nslices, j0 + (int)(g * nj / ngroups), j0 + (int)((g + 1) * nj / ngroups),
+                         id / segs % 4, id % segs, part / ngroups * RTP_EDGE_SLICES, ngroups, out + g * img, lds);
+    return;
+  }
+  id -= nborder;
+  const int z = id / (cols * rows), tile = id - z * (cols * rows);
+  const int ty = tile / cols, tx = tile - ty * cols;
+  const int group = z / ngroups, g = z - group * ngroups;
+  const int slice0 = group * ss_rt_slices(kind);
+  const int ja = j0 + (int)(g * nj / ngroups), jb = j0 + (int)((g + 1) * nj / ngroups);
+  ss_rtp_item<ROWS, STAGE, PL>(p, planes + (size_t)group * p.g.nangles * p.g.nrays * PL, kind, slice0, nslices, ja, jb,
+                               tx * BP_TILE_W, ty * 8 * ROWS, out + ((size_t)slice0 * ngroups + g) * img,
+                               ngroups * img, lds);
+}
+
+// The transpose's pre-scaled planes: out[group][a][r][z] = plane z's sinogram value at (a, r)
+// times its angle's Delta, for the angles j0 .. j1 - 1 (z >= PL: none).  Read from the
+// angle-major layout or (in_cols) from the (R, A) layout, which spares that its own
+// transposition pass.  A block moves 32 angles x 32 rays.
+template <int PL>
+__global__ __launch_bounds__(256) void k_rtp_planes(SSDevPlan p, const float* __restrict__ in, int in_cols, int kind,
+                                                    int nslices, int j0, int j1, float* __restrict__ out) {
+  __shared__ float T[PL][32][33];
+  typedef typename SSRtVec<PL>::type vec;
+  const int R = p.g.nrays, A = p.g.nangles;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int br = blockIdx.x * 32, ba = j0 + blockIdx.y * 32;
+#pragma unroll
+  for (int z = 0; z < PL; ++z) {
+    const SSPlane pl = ss_rt_plane(kind, z);
+    const size_t slice = (size_t)min((int)blockIdx.z * ss_rt_slices(kind) + pl.slice, nslices - 1);
+    const float* src = in + slice * A * R;
+#pragma unroll
+    for (int yy = ty; yy < 32; yy += 8) {
+      // tx runs along the input's contiguous direction
+      const int a = ba + (in_cols ? tx : yy), r = br + (in_cols ? yy : tx);
+      float v = 0.f;
+      if (a < j1 && r < R) {
+        const SSBpMirror m = pl.mirror ? ss_bp_mirror(a, A) : SSBpMirror{a, false};
+        const int rz = pl.turn != m.flip ? R - 1 - r : r;
+        v = src[in_cols ? (size_t)rz * A + m.row : (size_t)m.row * R + rz] * p.angles[m.row].delta;
+        // irregular rays (k_radon_transpose_fixup adds them) have the range (0, -2)
+        if (p.nirregular && p.bounds[(size_t)m.row * R + rz].y == -2) v = 0.f;
+      }
+      T[z][in_cols ? tx : yy][in_cols ? yy : tx] = v;  // [angle][ray]
+    }
+  }
+  __syncthreads();
+  vec* dst = reinterpret_cast<vec*>(out) + (size_t)blockIdx.z * A * R;
+#pragma unroll
+  for (int yy = ty; yy < 32; yy += 8) {
+    const int a = ba + yy, r = br + tx;
+    if (a >= j1 || r >= R) continue;
+    vec v;
+    if constexpr (PL == 1) {
+      v = T[0][yy][tx];
+    } else {
+#pragma unroll
+      for (int z = 0; z < PL; ++z) v[z] = T[z][yy][tx];
+    }
+    dst[(size_t)a * R + r] = v;
+  }
 }
 
 // LDS a block may use on the current device (gfx950: 160 KiB, also assumed if the query
@@ -2523,73 +2655,95 @@ static int ss_rt_lines(int n, int sl) {
   return 0;
 }
 
-// The pixel-driven transpose's pre-scaled rays: in[slice][a][r] * Delta_a for the angles
-// j0 .. j1 - 1; slices 2i, 2i + 1 (i < pairs) interleaved in their own space,
-// out[2i][a][r][2], the others as they are
-__global__ __launch_bounds__(256) void k_rtp_scale(SSDevPlan p, const float* __restrict__ in, int j0, int j1,
-                                                   int pairs, float* __restrict__ out) {
-  const int R = p.g.nrays;
-  const size_t slice = blockIdx.z;
-  const int a = j0 + blockIdx.y;
-  if (a >= j1) return;
-  const size_t sino = (size_t)p.g.nangles * R;
-  const size_t row = slice * sino + (size_t)a * R;
-  const float d = p.angles[a].delta;
-  const bool paired = slice < 2 * (size_t)pairs;
-  float* __restrict__ dst = paired ? out + (slice & ~(size_t)1) * sino + (size_t)a * R * 2 + (slice & 1) : out + row;
-  const int step = paired ? 2 : 1;
-  for (int r = blockIdx.x * 256 + threadIdx.x; r < R; r += gridDim.x * 256) dst[(size_t)r * step] = in[row + r] * d;
+// Planes of a pixel-driven transpose over angles [j0, j1) of nslices slices.  Every plane's
+// arithmetic is the same in each of them, so a slice's result does not depend on what it is
+// launched with.
+static int ss_rt_kind(const SSDevPlan& p, int j0, int j1, int nslices) {
+  if (4 * (p.rt_window + 4) > 2 * kSSBpStage[p.rt_variant]) return SS_RT_ONE;  // a window of four does not fit
+  if ((p.rt_sym & 2) && j0 == 0 && j1 == p.g.nangles) return SS_PLANES_QUAD;
+  if (p.rt_sym & 1) return nslices >= 2 ? SS_PLANES_PAIR : SS_RT_TURN;
+  return nslices >= 3 ? SS_PLANES_SLICES : (nslices == 2 ? SS_RT_TWO : SS_RT_ONE);
 }
 
-size_t ss_radon_transpose_scratch(const SSDevPlan& p, int nslices) {
-  return p.rt_angles > 0 ? sizeof(float) * (size_t)nslices * p.g.nangles * p.g.nrays
-                         : sizeof(float) * (size_t)nslices * p.g.n * p.g.n;
+static dim3 ss_rt_grid(const SSDevPlan& p, int kind) {
+  const int n = p.g.n, th = 8 * kSSBpRows[p.rt_variant];
+  const int cols = kind == SS_PLANES_QUAD ? (n + 1) / 2 : n;
+  const int rows = kind == SS_PLANES_QUAD || kind == SS_PLANES_PAIR || kind == SS_RT_TURN ? (n + 1) / 2 : n;
+  return dim3((cols + BP_TILE_W - 1) / BP_TILE_W, (rows + th - 1) / th);
 }
 
-hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int j0, int j1, int nslices,
+// Angle groups, by the backprojection's rule.  Up to SS_RT_SAME_SLICES slices take one
+// slice's groups (of the form that launch has), so that their sums have the same order.
+static int ss_rt_groups(const SSDevPlan& p, int j0, int j1, int nslices) {
+  const int kind = ss_rt_kind(p, j0, j1, nslices);
+  const int one = nslices <= SS_RT_SAME_SLICES ? ss_rt_kind(p, j0, j1, 1) : kind;
+  const dim3 grid = ss_rt_grid(p, one);
+  const long long tiles = (long long)grid.x * grid.y *
+                          (nslices <= SS_RT_SAME_SLICES ? 1 : (nslices + ss_rt_slices(kind) - 1) / ss_rt_slices(kind));
+  return ss_angle_groups(tiles, j1 - j0);
+}
+
+static size_t ss_rt_planes_floats(const SSDevPlan& p, int kind, int nslices) {
+  const int per = ss_rt_slices(kind);
+  return (size_t)((nslices + per - 1) / per) * p.g.nangles * p.g.nrays * ss_rt_planes(kind);
+}
+
+size_t ss_radon_transpose_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
+  const size_t img = (size_t)nslices * p.g.n * p.g.n;
+  if (p.rt_angles <= 0) return sizeof(float) * img;
+  const int kind = ss_rt_kind(p, j0, j1, nslices), G = ss_rt_groups(p, j0, j1, nslices);
+  return sizeof(float) * (((ss_rt_planes_floats(p, kind, nslices) + 3) & ~(size_t)3) + (G > 1 ? G * img : 0));
+}
+
+template <int PL>
+static hipError_t ss_launch_rtp(const SSDevPlan& p, const float* in, int in_cols, int kind, int j0, int j1,
+                                int nslices, float* out, float* scratch, hipStream_t stream) {
+  const int G = ss_rt_groups(p, j0, j1, nslices);
+  const int per = ss_rt_slices(kind), groups = (nslices + per - 1) / per;
+  float* planes = scratch;
+  float* part = scratch + ((ss_rt_planes_floats(p, kind, nslices) + 3) & ~(size_t)3);
+  hipLaunchKernelGGL(k_rtp_planes<PL>, dim3((p.g.nrays + 31) / 32, (j1 - j0 + 31) / 32, groups), dim3(256), 0, stream,
+                     p, in, in_cols, kind, nslices, j0, j1, planes);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const dim3 tiles = ss_rt_grid(p, kind);
+  const int nborder = 4 * ((p.g.n + 31) / 32) * ((nslices + RTP_EDGE_SLICES - 1) / RTP_EDGE_SLICES) * G;
+  const dim3 grid(nborder + tiles.x * tiles.y * groups * G);
+#define SS_RTP_LAUNCH(V, ROWS, STAGE)                                                                             \
+  case V:                                                                                                         \
+    hipLaunchKernelGGL((k_radon_transpose_px<ROWS, STAGE, PL>), grid, dim3(256), 0, stream, p, planes, kind,      \
+                       nslices, j0, j1, G, nborder, (int)tiles.x, (int)tiles.y, G > 1 ? part : out);              \
+    break;
+  switch (p.rt_variant) {
+    SS_BP_FOR_VARIANTS(SS_RTP_LAUNCH)
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef SS_RTP_LAUNCH
+  e = hipGetLastError();
+  if (e != hipSuccess || G == 1) return e;
+  const size_t img = (size_t)p.g.n * p.g.n;
+  hipLaunchKernelGGL(k_bp_groups_finish<SS_BP_PLAIN>, dim3((unsigned)((img + 255) / 256), nslices), dim3(256), 0,
+                     stream, part, G, p.g.n, 1.0f, out, SSEmUpdateArgs{nullptr, nullptr});
+  return hipGetLastError();
+}
+
+hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int in_cols, int j0, int j1, int nslices,
                                      float* out, float* scratch, hipStream_t stream) {
   const int n = p.g.n;
   if (p.rt_angles > 0) {  // the pixel-driven form (every angle's rays at least one cell apart)
-    if (!scratch) return hipErrorInvalidValue;
-    const int th = 8 * kSSBpRows[p.rt_variant];
-    // slices in pairs (a pair shares each pixel's geometry) when a pair's stage holds at
-    // least 8 angles, the last odd slice alone
-    const int pairs = (p.rt_angles / 2 >= 8) ? nslices / 2 : 0;
-    hipLaunchKernelGGL(k_rtp_scale, dim3((p.g.nrays + 255) / 256, j1 - j0, nslices), dim3(256), 0, stream, p, sinoT,
-                       j0, j1, pairs, scratch);
-    const hipError_t es = hipGetLastError();
-    if (es != hipSuccess) return es;
-    const float* scaled = scratch;
-    const int singles = nslices - 2 * pairs;
-    for (int part = 0; part < 2; ++part) {
-      const int count = part == 0 ? pairs : singles;
-      if (count == 0) continue;
-      dim3 grid((n + BP_TILE_W - 1) / BP_TILE_W, (n + th - 1) / th, count);
-      const int slice0 = part == 0 ? 0 : 2 * pairs;
-#define SS_RTP_LAUNCH(V, ROWS, STAGE)                                                                            \
-  case V:                                                                                                        \
-    if (part == 0)                                                                                               \
-      hipLaunchKernelGGL((k_radon_transpose_px<ROWS, STAGE, 2>), grid, dim3(256), 0, stream, p, scaled, j0, j1, \
-                         slice0, out);                                                                           \
-    else                                                                                                         \
-      hipLaunchKernelGGL((k_radon_transpose_px<ROWS, STAGE, 1>), grid, dim3(256), 0, stream, p, scaled, j0, j1, \
-                         slice0, out);                                                                           \
-    break;
-      switch (p.rt_variant) {
-        SS_BP_FOR_VARIANTS(SS_RTP_LAUNCH)
-        default:
-          return hipErrorInvalidValue;
-      }
-#undef SS_RTP_LAUNCH
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-    }
-    const hipError_t e = hipGetLastError();
+    if (!scratch || j1 <= j0) return hipErrorInvalidValue;
+    const int kind = ss_rt_kind(p, j0, j1, nslices);
+    const int pl = ss_rt_planes(kind);
+    const hipError_t e = pl == 4   ? ss_launch_rtp<4>(p, sinoT, in_cols, kind, j0, j1, nslices, out, scratch, stream)
+                         : pl == 2 ? ss_launch_rtp<2>(p, sinoT, in_cols, kind, j0, j1, nslices, out, scratch, stream)
+                                   : ss_launch_rtp<1>(p, sinoT, in_cols, kind, j0, j1, nslices, out, scratch, stream);
     if (e != hipSuccess || p.nirregular == 0) return e;
-    hipLaunchKernelGGL(k_radon_transpose_fixup, dim3(p.nirregular, nslices), dim3(256), 0, stream, p, sinoT, j0, j1,
-                       out);
+    hipLaunchKernelGGL(k_radon_transpose_fixup, dim3(p.nirregular, nslices), dim3(256), 0, stream, p, sinoT, in_cols,
+                       j0, j1, out);
     return hipGetLastError();
   }
+  if (in_cols) return hipErrorInvalidValue;  // the line form reads the angle-major layout
   // several slices per wave where the image is small enough for their lines to leave
   // room for many waves per CU: four for n <= 512, two for n <= 1024 (8 KiB per wave);
   // the remaining slices go in pairs, then alone
@@ -2627,7 +2781,7 @@ hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int
   hipLaunchKernelGGL(k_transpose_add, dim3(t, t, nslices), dim3(256), 0, stream, scratch, out, n);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.nirregular == 0) return e;
-  hipLaunchKernelGGL(k_radon_transpose_fixup, dim3(p.nirregular, nslices), dim3(256), 0, stream, p, sinoT, j0, j1,
+  hipLaunchKernelGGL(k_radon_transpose_fixup, dim3(p.nirregular, nslices), dim3(256), 0, stream, p, sinoT, 0, j0, j1,
                      out);
   return hipGetLastError();
 }

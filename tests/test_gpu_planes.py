@@ -62,7 +62,6 @@ def test_radon_planes(n, R, A, sc):
     enough slices that the launch takes the planes undivided."""
     import torch
     from pyraft_amd.device import Plan
-    from pyraft_amd.raftypes import libraft  # noqa: F401  (the library under test)
     p = Plan(n, R, A, sino_corners=sc)
     blocks = ((R + 127) // 128) * ((A // 2 + 8) // 8)
     many = min(-(-1024 // blocks), 1200) * 4 + 1  # odd, past SS_RADON_SLAB_BLOCKS in every form
@@ -93,3 +92,31 @@ def test_mesh_radon_planes(n, R, A, slices):
     idx = np.arange(slices) % 4
     got = p.radon(torch.from_numpy(x).cuda()[torch.from_numpy(idx).cuda()]).cpu().numpy()
     assert _rel(got, ref[idx]) <= REL and _rel(got[-1], ref[idx[-1]]) <= REL
+
+
+@pytest.mark.parametrize("n,R,A,sc", GEO)
+def test_transpose_planes(n, R, A, sc):
+    """Both layouts, whole and partial ranges, every tile variant, and slice counts on both
+    sides of the one-slice summation order."""
+    import torch
+    from pyraft_amd.device import Plan
+    y = np.random.default_rng(3 * n + R).random((3, R, A)).astype(np.float32)
+    ref = np.stack([O.radon_transpose(v.astype(np.float64), n, **_geo(sc)) for v in y])
+    j0, j1 = A // 3, max(A // 3 + 1, A - 1)
+    part = np.zeros_like(y, dtype=np.float64)
+    part[:, :, j0:j1] = y[:, :, j0:j1]
+    pref = np.stack([O.radon_transpose(v, n, **_geo(sc)) for v in part])
+    p = Plan(n, R, A, sino_corners=sc)
+    ys = torch.from_numpy(y).cuda()
+    for s in (1, 2, 3, 11):
+        print("transpose planes", n, R, A, sc, "slices", s, flush=True)
+        idx = torch.arange(s, device="cuda") % 3
+        own, pown = ref[np.arange(s) % 3], pref[np.arange(s) % 3]
+        got = p.radon_transpose(ys[idx]).cpu().numpy()
+        assert _rel(got, own) <= REL and _rel(got[-1], own[-1]) <= REL, s
+        am = ys[idx].transpose(-1, -2).contiguous()
+        assert np.array_equal(p.radon_transpose(am, angle_major=True).cpu().numpy(), got), s
+        if np.linalg.norm(pref) > 0:
+            assert _rel(p.radon_transpose(ys[idx], angles=(j0, j1)).cpu().numpy(), pown) <= REL, s
+    v, times = p.tune_transpose(1, reps=1, force=True)
+    assert v == -1 or _rel(p.radon_transpose(ys[0]).cpu().numpy(), ref[0]) <= REL
