@@ -37,10 +37,13 @@ struct raft_dda_plan {
   float* d_row_scale = nullptr;  // [A] lmax of the gather angles
   int kmax = 0;
   int gather_ws = 0;  // segment length of the two-candidate gather, 0 when it does not apply
+  int planes_ws = 0;  // window of the gather in planes, 0 when it does not apply
+  int sym = 0;        // DDA_SYM_*
   double* d_weights = nullptr;  // R^T 1 in FP64, built on first use
   std::mutex weights_mutex;
   SSDdaTransposePlan tplan() const {
-    return SSDdaTransposePlan{d_angles, d_gather, (int)h_gather.size(), kmax, gather_ws, d_straight,
+    return SSDdaTransposePlan{d_angles, d_gather, (int)h_gather.size(), kmax, gather_ws,
+                              planes_ws, sym, d_straight,
                               (int)h_straight.size(), d_ranges, d_row_scale, d_walk, (int)h_walk.size()};
   }
   ~raft_dda_plan() {
@@ -241,6 +244,23 @@ void set_trapezoid(const SSDdaGeom& g, const SSDdaGatherAngle& ga, SSDdaAngle& a
   a.fixed = 1;
 }
 
+// DDA_SYM_* of the geometry: positions (in pixels and rays) and directions agree within
+// FP64 rounding, the sets of exact-geometry angles are each other's mirrors
+int symmetry(const SSDdaGeom& g, const std::vector<SSDdaAngle>& angles) {
+  const double tol = 1e-11;
+  const int A = (int)angles.size();
+  const double ex = fabs((2.0 * g.ox + (g.cols - 1) * g.hx) / g.hx), ey = fabs((2.0 * g.oy + (g.lines - 1) * g.hy) / g.hy);
+  const double et = fabs((2.0 * g.t0 + (g.nrays - 1) * g.dt) / g.dt);
+  if (!(ex <= tol * g.cols && ey <= tol * g.lines && et <= tol * g.nrays)) return 0;
+  int sym = DDA_SYM_TURN | DDA_SYM_MIRROR;
+  for (int a = 0; a < A; ++a) {
+    const SSDdaAngle &x = angles[a], &y = angles[A - 1 - a];
+    if (x.fixed != y.fixed) return DDA_SYM_TURN;
+    if (x.fixed && !(fabs(x.c + y.c) <= 1e-14 && fabs(x.s - y.s) <= 1e-14)) return DDA_SYM_TURN;
+  }
+  return sym;
+}
+
 int check_dda(const raft_dda_plan* p, int nslices) {
   if (!p) return ss_set_error(RAFT_SS_EINVAL, "null plan");
   if (nslices < 1 || nslices > 65535)
@@ -260,9 +280,10 @@ int ensure_weights(raft_dda_plan* p, hipStream_t stream) {
   double* w = nullptr;
   HIP_TRY(hipMalloc(&w, sizeof(double) * npix));
   DevBuf sinoT, acc, accT;
-  hipError_t e = sinoT.alloc(sizeof(float) * (size_t)(p->g.nrays + 4) * p->g.nangles, stream);
-  if (e == hipSuccess) e = acc.alloc(sizeof(double) * npix, stream);
-  if (e == hipSuccess) e = accT.alloc(sizeof(double) * npix, stream);
+  const SSDdaTransposeScratch sb = dda_transpose_scratch(p->g, p->tplan(), true, 1, sizeof(double));
+  hipError_t e = sinoT.alloc(sb.sino, stream);
+  if (e == hipSuccess) e = acc.alloc(sb.acc, stream);
+  if (e == hipSuccess) e = accT.alloc(sb.accT, stream);
   if (e == hipSuccess)
     e = dda_launch_transpose<double, double>(p->g, p->tplan(), sinoT.as<float>(), true, sinoT.as<float>(),
                                              acc.as<double>(), accT.as<double>(), nullptr, w, 1, stream);
@@ -279,13 +300,13 @@ int ensure_weights(raft_dda_plan* p, hipStream_t stream) {
 template <typename T, typename Out>
 int transpose_into(const raft_dda_plan* p, const float* sino, const double* w, Out* out, int nslices,
                    hipStream_t stream) {
-  const size_t n = (size_t)p->g.lines * p->g.cols * nslices;
   DevBuf sinoT, acc, accT;
-  HIP_TRY(sinoT.alloc(sizeof(float) * (size_t)(p->g.nrays + 4) * p->g.nangles * nslices, stream));
-  HIP_TRY(acc.alloc(sizeof(T) * n, stream));
-  HIP_TRY(accT.alloc(sizeof(T) * n, stream));
-  HIP_TRY((dda_launch_transpose<T, Out>(p->g, p->tplan(), sino, false, sinoT.as<float>(), acc.as<T>(), accT.as<T>(),
-                                        w, out, nslices, stream)));
+  const SSDdaTransposeScratch sb = dda_transpose_scratch(p->g, p->tplan(), false, nslices, sizeof(T));
+  HIP_TRY(sinoT.alloc(sb.sino, stream));
+  HIP_TRY(acc.alloc(sb.acc, stream));
+  if (sb.accT) HIP_TRY(accT.alloc(sb.accT, stream));
+  HIP_TRY((dda_launch_transpose<T, Out>(p->g, p->tplan(), sino, false, sinoT.as<float>(), acc.p, accT.as<T>(), w, out,
+                                        nslices, stream)));
   return 0;
 }
 
@@ -352,13 +373,16 @@ extern "C" int raft_dda_plan_create(raft_dda_plan** out, int lines, int cols, in
     }
   }
   std::vector<float> row_scale(nangles, 0.f);
-  int ws = 8;
+  int ws = 8, pws = 0;
   for (const SSDdaGatherAngle& ga : p->h_gather) {
     row_scale[ga.a] = (float)ga.lmax;
     p->kmax = std::max(p->kmax, ga.k);
     ws = std::max(ws, dda_gather2_ws(ga));
+    pws = std::max(pws, dda_gather_planes_ws(ga));
   }
   p->gather_ws = p->kmax <= 2 && ws <= DDA_G2_WSMAX ? ws : 0;
+  p->planes_ws = p->kmax <= 2 && pws <= DDA_GP_WSMAX && (long long)g.nrays * 16 <= 0x7fffffff ? pws : 0;
+  p->sym = symmetry(g, p->h_angles);
   HIP_TRY(hipMalloc(&p->d_row_scale, sizeof(float) * nangles));
   HIP_TRY(hipMemcpyAsync(p->d_row_scale, row_scale.data(), sizeof(float) * nangles, hipMemcpyHostToDevice, stream));
   HIP_TRY(hipMalloc(&p->d_angles, sizeof(SSDdaAngle) * nangles));
@@ -405,9 +429,11 @@ extern "C" int raft_dda_radon(const raft_dda_plan* p, const float* img, float* s
   if (rc) return rc;
   if (!img || !sino) return ss_set_error(RAFT_SS_EINVAL, "null buffer");
   hipStream_t stream = as_stream(stream_);
-  DevBuf pad;
-  HIP_TRY(pad.alloc(sizeof(float) * dda_radon_scratch_floats(p->g, nslices), stream));
-  HIP_TRY(dda_launch_radon(p->g, p->d_angles, img, pad.as<float>(), sino, nslices, stream));
+  DevBuf layout, part;
+  const SSDdaRadonForm form = dda_radon_form(p->g, p->tplan(), nslices);
+  HIP_TRY(layout.alloc(form.layout, stream));
+  if (form.part) HIP_TRY(part.alloc(form.part, stream));
+  HIP_TRY(dda_launch_radon(p->g, p->tplan(), img, layout.p, part.as<double>(), sino, nslices, stream));
   return 0;
 }
 

@@ -23,6 +23,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "ss_planes.h"
+
 #if defined(__HIPCC__)
 #define DDA_HD __host__ __device__
 #else
@@ -213,9 +215,7 @@ static inline DDA_HD SSDdaRay dda_ray_start(const SSDdaGeom& g, const SSDdaAngle
 
 // ---- launchers (dda_kernels.hip)
 
-// Radon: sino[slice][R][A] (overwritten) of img[slice][lines][cols]; pad
-// (dda_radon_scratch_floats) is scratch that the launcher fills with the image's padded
-// (line, column) and (column, line) layouts: DDA_PADW zeros either side of every line,
+// The one-ray Radon's scratch: the image's padded (line, column) and (column, line) layouts: DDA_PADW zeros either side of every line,
 // the line length rounded up to 4 floats (dda_pad_pitch).  The padding covers a whole
 // staged segment (DDA_WS_SEG) of a wave whose lowest ray lies left of the image while
 // another of its rays reaches in.
@@ -226,8 +226,6 @@ static inline DDA_HD int dda_pad_pitch(int ns) { return (ns + 2 * DDA_PADW + 3) 
 static inline size_t dda_radon_scratch_floats(const SSDdaGeom& g, int nslices) {
   return (size_t)nslices * ((size_t)g.lines * dda_pad_pitch(g.cols) + (size_t)g.cols * dda_pad_pitch(g.lines));
 }
-hipError_t dda_launch_radon(const SSDdaGeom& g, const SSDdaAngle* angles, const float* img, float* pad, float* sino,
-                            int nslices, hipStream_t stream);
 // The transpose's angles split into the pixel-driven set (gather table, ngather) and the
 // ray-traced set (walk list of sinogram columns, nwalk).
 // Two-candidate gather (k_dda_gather2): block of DDA_G2_COLS columns x 4 G lines (G
@@ -259,12 +257,35 @@ struct SSDdaStraight {
   double len;
 };
 
+// The gather in planes (k_dda_gather_planes): tiles of 32 x 8 DDA_GP_ROWS pixels, angles
+// staged DDA_GP_ANGLES at a time in windows of ws rays (dda_gather_planes_ws), DDA_GP_WSMAX at
+// most: two candidates per pixel mean |kx|, |ky| with |kx| + |ky| <= 2
+#define DDA_GP_ROWS 4
+#define DDA_GP_ANGLES 16
+#define DDA_GP_WSMAX 72
+// Blocks aimed at with angle groups (us at 512, 1024, 2048: 512^2 x 720 86, 79, 82;
+// 1024^2 x 721 195, 141, 146), and two groups for launches of up to two rounds of tiles, whose
+// last tiles end together then (2048^2 x 1500, 1024 tiles: one group 870, two 812)
+#define DDA_GP_BLOCKS 1024
+#define DDA_GP_PAIR_TILES 2048
+#define DDA_GP_MAXGROUPS 64
+static inline int dda_gather_planes_ws(const SSDdaGatherAngle& ga) {
+  const double span = 31 * fabs(ga.kx) + (8 * DDA_GP_ROWS - 1) * fabs(ga.ky);
+  return span < DDA_GP_WSMAX ? (int)ceil(span) + 5 : DDA_GP_WSMAX + 1;
+}
+// symmetries of a geometry (the detector's middle ray and the image's centre at the origin):
+// 1 half turn (x, y, t) -> (-x, -y, -t); 2 also mirror x -> -x, angle a -> A - 1 - a
+#define DDA_SYM_TURN 1
+#define DDA_SYM_MIRROR 2
+
 struct SSDdaTransposePlan {
   const SSDdaAngle* angles;
   const SSDdaGatherAngle* gather;
   int ngather;
   int kmax;                 // largest candidate count of the gather table
   int gather_ws;            // segment length of k_dda_gather2 (0: not usable)
+  int planes_ws;            // window of k_dda_gather_planes (0: not usable)
+  int sym;                  // DDA_SYM_*
   const SSDdaStraight* straight;  // straight angles (only when no angle is traced)
   int nstraight;
   const int* ranges;
@@ -273,12 +294,42 @@ struct SSDdaTransposePlan {
   int nwalk;
 };
 
-// out[slice] = R^T sino[slice] [/ w] (T: accumulator type of the ray-traced part, float or
-// double).  sinoT ([nslices][A][R + 4] floats), acc, accT ([nslices][lines*cols] T) are
-// scratch.  `ones`: R^T 1 for one slice (sino unused).
+// The Radon in planes (k_dda_radon_planes): zeros either side of a layout row
+#define DDA_RP_PAD 6
+// launches of few blocks divide the fast indices as the slant stack's (SS_PLANES_SLAB_BLOCKS),
+// into slabs of at least DDA_RP_MIN_ROWS (us at 32, 64, 128: 64^2 x 24 44, 30, 30; 512^2 x 720 82, 84,
+// 79; 1024^2 x 721 157, 158, 159)
+#define DDA_RP_MIN_ROWS 128
+// The form of a Radon launch: in planes (kind, nslab slabs of fast indices) or one ray per lane
+// (SS_PLANES_NONE); bytes of its image layouts and of its partial sums
+struct SSDdaRadonForm {
+  int kind, nslab;
+  size_t layout, part;
+};
+SSDdaRadonForm dda_radon_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, int nslices);
+// Radon: sino[slice][R][A] (overwritten) of img[slice][lines][cols]; layout and part are
+// scratch (dda_radon_form)
+hipError_t dda_launch_radon(const SSDdaGeom& g, const SSDdaTransposePlan& tp, const float* img, void* layout,
+                            double* part, float* sino, int nslices, hipStream_t stream);
+
+// The form the transpose's pixel-driven angles take: in planes (kind, ngroups angle groups) or
+// not (kind SS_PLANES_NONE)
+struct SSDdaGatherForm {
+  int kind, ngroups;
+};
+SSDdaGatherForm dda_gather_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, bool ones, int nslices);
+// bytes of the transpose's scratch: the sinogram copy, acc, and accT (T: see below)
+struct SSDdaTransposeScratch {
+  size_t sino, acc, accT;
+};
+SSDdaTransposeScratch dda_transpose_scratch(const SSDdaGeom& g, const SSDdaTransposePlan& tp, bool ones, int nslices,
+                                            size_t sizeof_t);
+
+// out[slice] = R^T sino[slice] [/ w] (T: accumulator type, float or double).  sinoT, acc and
+// accT are scratch (dda_transpose_scratch).  `ones`: R^T 1 for one slice (sino unused).
 template <typename T, typename Out>
 hipError_t dda_launch_transpose(const SSDdaGeom& g, const SSDdaTransposePlan& tp, const float* sino, bool ones,
-                                float* sinoT, T* acc, T* accT, const double* w, Out* out, int nslices,
+                                float* sinoT, void* acc, T* accT, const double* w, Out* out, int nslices,
                                 hipStream_t stream);
 hipError_t dda_launch_to_f32(const double* src, float* dst, size_t n, hipStream_t stream);
 

@@ -6,15 +6,21 @@
 // order (raft/raft_ddaiterator.c), so every ray visits the reference's pixels; taps
 // are FP32, the Radon's ray sums FP64.
 //
-//   k_dda_radon      gather: sino[r][a] = sum over the ray's pixels of f(pixel) * len
-//   k_dda_scatter    scatter: acc(pixel) += q * len with atomics (FP32 for R^T, FP64 for
-//                    the normalised backprojection and its weights R^T 1)
-//   k_dda_fold       out = acc + accT^T (optionally / weights) through an LDS tile
-//   k_dda_transpose_image  the column-major copy of the image the Radon reads for
-//                          angles whose fast axis is the column
+//   k_dda_radon_planes    Radon, four rays per lane on symmetric geometries and in stacks of
+//                         slices; k_dda_pad_planes its image layouts
+//   k_dda_radon           Radon, one ray per lane: sino[r][a] = sum over the ray's pixels of
+//                         f(pixel) * len; k_dda_pad_images its image layouts
+//   k_dda_gather_planes   transpose by pixels, four pixels per lane on the same geometries
+//   k_dda_gather2, k_dda_gather  transpose by pixels, one pixel per lane and line
+//   k_dda_scatter         transpose of traced angles: acc(pixel) += q * len with atomics (FP32 for
+//                         R^T, FP64 for the normalised backprojection and its weights R^T 1)
+//   k_dda_fold            the transpose's parts added, optionally / weights
 #include "dda_kernels.h"
+#include "ss_kernels.h"
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #define DDA_TILE 32
 
@@ -323,6 +329,410 @@ __global__ __launch_bounds__(256) void k_dda_radon(SSDdaGeom g, const SSDdaAngle
   if (lane_ok) sino[(slice * g.nrays + r) * g.nangles + ai] = (float)acc;
 }
 
+// ---------------------------------------------------------------- Radon in planes
+
+// The trapezoid form in planes.  k_dda_radon reads one 8-byte LDS pair and issues 13 VALU
+// instructions per fast index and ray.  Here a lane's tau and weights serve four rays
+// (SSPlane; the image, its half turn (ray R - 1 - r), its mirror x -> -x (angle A - 1 - a) and
+// the half turn of that, or slices), the layouts hold the planes' values of a pixel together
+// (16 bytes), and a block's 8 waves share one staged window (ss_planes_chunks).  Layout rows:
+// fast index k's pixels along the slow axis with DDA_RP_PAD zeros either side; the record of
+// slow index j is j + DDA_RP_PAD, and to the window code the rows are rows of an image of
+// ns + 2 DDA_RP_PAD - 2 cells.  A lane takes the fast indices where floor(tau) can be a
+// candidate inside the image, with an index of margin either side: tau moves by at most 2 per
+// index, so those samples lie within the padding, and their terms are zeros.  Sums are taken
+// in FP32 over at most 8 fast indices and those in FP64, as in k_dda_radon.
+// Per four updates: 6 VALU for tau, the address and the fraction, 5 for the weights, 8 FMAs,
+// two 16-byte reads.
+// 2048^2 x 1500: 2470 -> 805 us, the layouts' 34 us included; 1024^2 x 721 491 -> 160; 16 x 512^2 x 360
+// 660 -> 340; 256^2 x 180 80 -> 51.
+
+// Layouts: L[group][line][pc] and LT[group][column][pl] of img[slice][lines][cols], pc (pl) =
+// cols (lines) + 2 DDA_RP_PAD.  A block moves one 32 x 32 pixel tile; the first and last tile
+// of a row also write its padding.
+__global__ __launch_bounds__(256) void k_dda_pad_planes(int lines, int cols, int kind, int nslices,
+                                                        const float* __restrict__ img, ss_f32x4* __restrict__ L,
+                                                        ss_f32x4* __restrict__ LT) {
+  __shared__ float T[SS_PLANES][32][33];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32;
+  const int pc = cols + 2 * DDA_RP_PAD, pl = lines + 2 * DDA_RP_PAD;
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) {
+    const SSPlane p = ss_plane(kind, z);
+    const size_t slice = (size_t)min((int)blockIdx.z * ss_planes_slices(kind) + p.slice, nslices - 1);
+    const float* __restrict__ src = img + slice * lines * cols;
+#pragma unroll
+    for (int yy = ty; yy < 32; yy += 8) {
+      const int i = i0 + yy, j = j0 + tx;
+      const int si = p.turn ? lines - 1 - i : i, sj = p.turn != p.mirror ? cols - 1 - j : j;
+      T[z][yy][tx] = i < lines && j < cols ? src[(size_t)si * cols + sj] : 0.f;
+    }
+  }
+  __syncthreads();
+  ss_f32x4* __restrict__ o = L + (size_t)blockIdx.z * lines * pc;
+  ss_f32x4* __restrict__ oT = LT + (size_t)blockIdx.z * cols * pl;
+  const ss_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int yy = ty; yy < 32; yy += 8) {
+    const int i = i0 + yy, j = j0 + tx;
+    if (i < lines) {
+      ss_f32x4* __restrict__ row = o + (size_t)i * pc;
+      if (j < cols) row[j + DDA_RP_PAD] = ss_f32x4{T[0][yy][tx], T[1][yy][tx], T[2][yy][tx], T[3][yy][tx]};
+      if (blockIdx.x == 0 && tx < DDA_RP_PAD) row[tx] = zero;
+      if (j0 + 32 >= cols && tx < DDA_RP_PAD) row[cols + DDA_RP_PAD + tx] = zero;
+    }
+    const int jt = j0 + yy, it = i0 + tx;
+    if (jt < cols) {
+      ss_f32x4* __restrict__ row = oT + (size_t)jt * pl;
+      if (it < lines) row[it + DDA_RP_PAD] = ss_f32x4{T[0][tx][yy], T[1][tx][yy], T[2][tx][yy], T[3][tx][yy]};
+      if (blockIdx.y == 0 && tx < DDA_RP_PAD) row[tx] = zero;
+      if (i0 + 32 >= lines && tx < DDA_RP_PAD) row[lines + DDA_RP_PAD + tx] = zero;
+    }
+  }
+}
+
+// trapezoid terms of a wave's angle
+struct SSDdaTerms {
+  float c1, kz, pz, pz1;
+};
+
+// G fast indices s, s + 1, ... from the staged window; CHECK: an index at or beyond `end` or
+// outside the lane's range [lo, lo + span] reads the zero records
+template <int G, bool CHECK>
+__device__ __forceinline__ void dda_rp_group(const ss_f32x4* __restrict__ st, int s, int end, int64_t& u, int64_t step,
+                                             int lo, unsigned span, const SSDdaTerms& w, double (&tot)[SS_PLANES]) {
+  float part[SS_PLANES];
+  const unsigned stb = (unsigned)(size_t)(ss_lds_cell)st;
+#pragma unroll
+  for (int h = 0; h < G; h += 4) {  // four indices' reads in flight
+    ss_f32x4 a[4], b[4];
+    float fr[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      int idx = (int)(u >> 32);
+      if (CHECK) idx = s + h + g < end && (unsigned)(s + h + g - lo) <= span ? idx : PLANES_CAP;
+      fr[g] = (float)(uint32_t)u;
+      u += step;
+      __asm__ volatile("" : "+v"(u));  // one 64-bit add per index
+      const ss_lds_cell c = (ss_lds_cell)(size_t)(stb + ((unsigned)idx << 4));
+      a[g] = c[0];
+      b[g] = c[1];
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float z0 = __builtin_amdgcn_fmed3f(fmaf(-fabsf(w.c1 - fr[g]), w.kz, w.pz), 0.f, 1.f);
+      const float z1 = __builtin_amdgcn_fmed3f(fmaf(fr[g], w.kz, w.pz1), 0.f, 1.f);
+#pragma unroll
+      for (int z = 0; z < SS_PLANES; ++z) {
+        part[z] = h + g == 0 ? z0 * a[g][z] : fmaf(z0, a[g][z], part[z]);
+        part[z] = fmaf(z1, b[g][z], part[z]);
+      }
+    }
+  }
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) tot[z] += (double)part[z];
+}
+
+struct SSDdaRadonPlanes {
+  int kind, nslices;
+  int nangles, nrays;      // plane 0's angles and rays
+  SSPlanesOrder order;
+  int nslab, slab_rows;    // fast indices in slabs of slab_rows, each with its partial sums
+  const SSDdaStraight* straight;
+  int nstraight;           // straight angles: blocks of 64 rays, first in the launch
+  const int* walk;
+  int nwalk;               // traced angles: blocks of 512 rays, before those
+};
+
+// the layout of a slice's own plane in its group: rows of `pitch` records, a float every
+// SS_PLANES
+__device__ __forceinline__ const float* dda_rp_plane(const SSDdaRadonPlanes& rp, const ss_f32x4* __restrict__ lay,
+                                                     int slice, int nf, int pitch) {
+  const int per = ss_planes_slices(rp.kind);
+  const int z = rp.kind == SS_PLANES_PAIR ? 2 * (slice % 2) : slice % per;
+  return reinterpret_cast<const float*>(lay + (size_t)(slice / per) * nf * pitch) + z;
+}
+
+// a traced angle's rays, as k_dda_radon walks them, DDA_RP_MOVES moves at a time: their pixels
+// and lengths first, then the loads together (a move that adds nothing reads the layout's
+// first record, a zero), then the sums in order
+#define DDA_RP_MOVES 8
+__device__ __forceinline__ void dda_rp_walk(const SSDdaGeom& g, const SSDdaAngle* __restrict__ angles,
+                                            const SSDdaRadonPlanes& rp, const ss_f32x4* __restrict__ L,
+                                            const ss_f32x4* __restrict__ LT, int id, float* __restrict__ sino) {
+  const int nrb = (g.nrays + RADON_WAVES * SS_WAVE - 1) / (RADON_WAVES * SS_WAVE);
+  const int slice = id / (nrb * rp.nwalk);
+  id -= slice * (nrb * rp.nwalk);
+  const int ai = rp.walk[id / nrb], r = id % nrb * (RADON_WAVES * SS_WAVE) + threadIdx.x;
+  const SSDdaAngle& a = angles[ai];
+  const int nf = a.fast_i ? g.lines : g.cols, ns = a.fast_i ? g.cols : g.lines;
+  const int pitch = ns + 2 * DDA_RP_PAD;
+  const float* __restrict__ src = dda_rp_plane(rp, a.fast_i ? L : LT, slice, nf, pitch);
+  SSDdaRay ray = dda_ray_start(g, a, dda_ray_t(g, min(r, g.nrays - 1)));
+  bool alive = r < g.nrays && dda_inside(ray.f, ray.s, nf, ns);
+  int F = dda_wave_start(alive, ray.f, a.dfast);
+  double acc = 0.0;
+  // lanes start at most nf moves apart and then take at most nf + 1 moves each
+  for (int it = 0; it <= 2 * nf + 1; it += DDA_RP_MOVES) {
+    if (__ballot(alive) == 0) break;
+    // no lane's drift passes the pixel width in these moves (close to an axis, most): the same
+    // moves without their cases
+    double e = ray.e;
+#pragma unroll
+    for (int m = 0; m < DDA_RP_MOVES; ++m) e += a.e_step;
+    const int f_end = dda_step(ray.f, DDA_RP_MOVES * a.dfast);
+    const bool plain = ray.f == F && !ray.slow_next && (unsigned)f_end < (unsigned)nf && e <= a.e_cap;
+    if (__ballot(alive && !plain) == 0) {
+      const float* at = src + (alive ? (size_t)(ray.f * pitch + ray.s + DDA_RP_PAD) : 0) * SS_PLANES;
+      const ptrdiff_t step = alive ? (ptrdiff_t)a.dfast * pitch * SS_PLANES : 0;
+      float v[DDA_RP_MOVES];
+#pragma unroll
+      for (int m = 0; m < DDA_RP_MOVES; ++m) v[m] = at[m * step];
+#pragma unroll
+      for (int m = 0; m < DDA_RP_MOVES; ++m) acc = fma((double)v[m], m == 0 ? ray.len : a.len_full, acc);
+      if (alive) {
+        ray.f = f_end;
+        ray.e = e;
+        ray.len = a.len_full;
+      }
+      F += DDA_RP_MOVES * a.dfast;
+      continue;
+    }
+    int pix[2 * DDA_RP_MOVES];
+    double len[2 * DDA_RP_MOVES];
+#pragma unroll
+    for (int m = 0; m < DDA_RP_MOVES; ++m) {
+      pix[2 * m] = pix[2 * m + 1] = 0;
+      len[2 * m] = len[2 * m + 1] = 0.0;
+      if (alive && ray.f == F) {
+        pix[2 * m] = ray.f * pitch + ray.s + DDA_RP_PAD;
+        len[2 * m] = ray.len;
+        if (ray.slow_next) {
+          ray.s = dda_step(ray.s, a.dslow);
+          ray.len = a.len_full - ray.len;
+          ray.slow_next = 0;
+          alive = dda_inside(ray.f, ray.s, nf, ns);
+          if (alive) {
+            pix[2 * m + 1] = ray.f * pitch + ray.s + DDA_RP_PAD;
+            len[2 * m + 1] = ray.len;
+          }
+        }
+        if (alive) {
+          dda_fast_move(a, ray);
+          alive = dda_inside(ray.f, ray.s, nf, ns);
+        }
+      }
+      F += a.dfast;
+    }
+    float v[2 * DDA_RP_MOVES];
+#pragma unroll
+    for (int m = 0; m < 2 * DDA_RP_MOVES; ++m) v[m] = src[(size_t)pix[m] * SS_PLANES];
+#pragma unroll
+    for (int m = 0; m < 2 * DDA_RP_MOVES; ++m) acc = fma((double)v[m], len[m], acc);
+  }
+  if (r < g.nrays) sino[((size_t)slice * g.nrays + r) * g.nangles + ai] = (float)acc;
+}
+
+// a straight angle's rays: the block's waves sum an eighth of the fast indices each
+__device__ __forceinline__ void dda_rp_straight(const SSDdaGeom& g, const SSDdaAngle* __restrict__ angles,
+                                                const SSDdaRadonPlanes& rp, const ss_f32x4* __restrict__ L,
+                                                const ss_f32x4* __restrict__ LT, int id, double* red,
+                                                float* __restrict__ sino) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int nrb = (g.nrays + 63) / 64;
+  const int slice = id / (nrb * rp.nstraight);
+  id -= slice * (nrb * rp.nstraight);
+  const int ai = rp.straight[id / nrb].a, r = id % nrb * 64 + lane;
+  const SSDdaAngle& a = angles[ai];
+  const int nf = a.fast_i ? g.lines : g.cols, ns = a.fast_i ? g.cols : g.lines;
+  const int pitch = ns + 2 * DDA_RP_PAD;
+  const float* __restrict__ src = dda_rp_plane(rp, a.fast_i ? L : LT, slice, nf, pitch);
+  const SSDdaRay ray = dda_ray_start(g, a, dda_ray_t(g, min(r, g.nrays - 1)));
+  const bool in = dda_inside(ray.f, ray.s, nf, ns);
+  const int s = in ? ray.s : 0;
+  double sum = 0.0;
+  const int f0 = (int)((long long)nf * wv / RADON_WAVES), f1 = (int)((long long)nf * (wv + 1) / RADON_WAVES);
+#pragma unroll 8
+  for (int f = f0; f < f1; ++f) sum += (double)src[((size_t)f * pitch + s + DDA_RP_PAD) * SS_PLANES];
+  red[threadIdx.x] = sum;
+  __syncthreads();
+  if (wv != 0 || r >= g.nrays) return;
+  for (int w = 1; w < RADON_WAVES; ++w) sum += red[w * 64 + lane];
+  sino[((size_t)slice * g.nrays + r) * g.nangles + ai] = in ? (float)(sum * a.len_full) : 0.f;
+}
+
+// Blocks: the traced angles' and the straight angles' (all slices), then the planes' (order.blocks per
+// slab and group of planes).  PARTIAL: the slab's FP64 sums go to part[slice][slab][a][r].
+template <bool PARTIAL>
+__global__ __launch_bounds__(RADON_WAVES * SS_WAVE, PLANES_BLOCKS) void k_dda_radon_planes(
+    SSDdaGeom g, const SSDdaAngle* __restrict__ angles, SSDdaRadonPlanes rp, const ss_f32x4* __restrict__ L,
+    const ss_f32x4* __restrict__ LT, float* __restrict__ sino, double* __restrict__ part) {
+  __shared__ SSPlanesLds lds;
+  int id = blockIdx.x;
+  const int nwk = rp.nwalk * ((g.nrays + RADON_WAVES * SS_WAVE - 1) / (RADON_WAVES * SS_WAVE)) * rp.nslices;
+  if (id < nwk) {
+    dda_rp_walk(g, angles, rp, L, LT, id, sino);
+    return;
+  }
+  id -= nwk;
+  const int nst = rp.nstraight * ((g.nrays + 63) / 64) * rp.nslices;
+  if (id < nst) {
+    dda_rp_straight(g, angles, rp, L, LT, id, reinterpret_cast<double*>(lds.stage), sino);
+    return;
+  }
+  id -= nst;
+  const int2 at = ss_planes_place(rp.order, id % rp.order.blocks);
+  id /= rp.order.blocks;
+  const int slab = id % rp.nslab, group = id / rp.nslab;
+  if (at.y < 0) return;  // block-uniform
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = at.y * RADON_WAVES + wv, k = at.x * SS_WAVE + ss_plane_ray(lane);
+  const SSDdaAngle& a = angles[min(j, rp.nangles - 1)];
+  const bool active = j < rp.nangles && a.fixed;
+  const bool on = active && k < rp.nrays;
+  const int nf_a = a.fast_i ? g.lines : g.cols, ns_a = a.fast_i ? g.cols : g.lines;
+  const SSDdaTerms w{a.tr_c1, a.tr_kz, a.tr_pz, a.tr_pz1};
+  const int64_t beta = (int64_t)a.tr_dhi * ((int64_t)1 << 32) + a.tr_dlo;
+  // trajectory in Q32 records, less 1 (the window code's cells): a_k + s beta
+  int64_t a_k = 0;
+  int lo = 0x40000000, hi = -1;
+  if (on) {
+    const double x = fma(dda_ray_t(g, k), a.tr_inv, a.tr_off) - DDA_PADW;  // floor: the first candidate
+    const double v = fmin(fmax(x + (DDA_RP_PAD - 1), -1073741824.0), 1073741824.0), fv = floor(v);
+    a_k = (int64_t)fv * ((int64_t)1 << 32) + (int64_t)(uint32_t)((v - fv) * 4294967296.0);
+    const double ka = (-1.0 - x) / a.tr_d, kb = (ns_a - x) / a.tr_d;
+    const double kl = fmax(fmin(ka, kb), -1.0), kh = fmin(fmax(ka, kb), (double)nf_a);
+    if (kl <= kh) {  // false for NaN
+      lo = (int)fmax(0.0, floor(kl) - 1.0);
+      hi = (int)fmin(nf_a - 1.0, ceil(kh) + 1.0);
+    }
+  }
+  const bool any = lo <= hi;
+  const unsigned span = any ? (unsigned)(hi - lo) : 0u;
+  if (!any) lo = 0x40000000;
+  int ulo = any ? lo : 0x7fffffff, uhi = any ? hi : -1, clo = any ? lo : -0x7fffffff, chi = any ? hi : 0x7fffffff;
+  int64_t amin = any ? a_k : INT64_MAX, amax = any ? a_k : INT64_MIN;
+  for (int off = 32; off > 0; off >>= 1) {
+    ulo = min(ulo, __shfl_xor(ulo, off));
+    uhi = max(uhi, __shfl_xor(uhi, off));
+    clo = max(clo, __shfl_xor(clo, off));
+    chi = min(chi, __shfl_xor(chi, off));
+    amin = min(amin, (int64_t)__shfl_xor((long long)amin, off));
+    amax = max(amax, (int64_t)__shfl_xor((long long)amax, off));
+  }
+  ulo = ss_rfl(ulo);
+  uhi = ss_rfl(uhi);
+  clo = ss_rfl(clo);
+  chi = ss_rfl(chi);
+  const int branch = uhi < ulo ? -1 : (a.fast_i ? 0 : 1);
+  if (lane == 0) {
+    lds.wmeta[wv][0] = lds.wmeta[wv][3] = branch;
+    lds.wmeta[wv][1] = ulo;
+    lds.wmeta[wv][2] = uhi;
+    lds.wpar[wv][0] = amin;
+    lds.wpar[wv][1] = amax;
+    lds.wpar[wv][2] = beta;
+  }
+  if (threadIdx.x < 2) lds.stage[PLANES_CAP + threadIdx.x] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
+  double tot[SS_PLANES] = {0.0, 0.0, 0.0, 0.0};
+  for (int pass = 0; pass < 2; ++pass) {  // fast axis line, then column
+    __syncthreads();
+    if (lane == 0) lds.wmeta[wv][0] = branch == pass ? branch : -1;  // this pass's waves
+    __syncthreads();
+    int s_lo = 0x7fffffff, s_hi = -1;
+    for (int i = 0; i < RADON_WAVES; ++i)
+      if (lds.wmeta[i][0] >= 0) {
+        s_lo = min(s_lo, lds.wmeta[i][1]);
+        s_hi = max(s_hi, lds.wmeta[i][2]);
+      }
+    s_lo = max(ss_rfl(s_lo), slab * rp.slab_rows);
+    s_hi = min(ss_rfl(s_hi), (slab + 1) * rp.slab_rows - 1);
+    const bool mine = branch == pass;
+    const int nf = pass ? g.cols : g.lines, pitch = (pass ? g.lines : g.cols) + 2 * DDA_RP_PAD;
+    const ss_f32x4* lay = (pass ? LT : L) + (size_t)group * nf * pitch;
+    ss_planes_chunks(lds, lay, pitch, pitch - 2, s_lo, s_hi, wv, lane, [&](int s0, int s1, int rec0, int Wc, bool fits) {
+      const int ra = max(s0, ulo), rb = min(s1 - 1, uhi);
+      if (!mine || ra > rb || Wc <= 0) return;
+      const int64_t t = a_k + (int64_t)ra * beta;
+      if (fits) {
+        // high word: staged record index (cell + 1 - rec0) + (row - s0) * Wc
+        int64_t u = t + ((int64_t)(1 - rec0 + (ra - s0) * Wc) << 32);
+        int64_t step = beta + ((int64_t)Wc << 32);
+        if (!any) {
+          u = (int64_t)PLANES_CAP << 32;
+          step = 0;
+        }
+        int s = ra;
+        const int head = min(rb + 1, clo);
+        if (s < head) {
+          const int64_t u0 = u;
+          for (; s < head; s += 4) dda_rp_group<4, true>(lds.stage, s, head, u, step, lo, span, w, tot);
+          s = head;
+          u = u0 + (int64_t)(head - ra) * step;
+        }
+        const int mid = min(rb + 1, chi + 1);
+        for (; s + 8 <= mid; s += 8) dda_rp_group<8, false>(lds.stage, s, 0, u, step, lo, span, w, tot);
+        for (; s <= rb; s += 4) dda_rp_group<4, true>(lds.stage, s, rb + 1, u, step, lo, span, w, tot);
+      } else if (any) {  // the window does not fit the LDS: read the layout
+        int64_t u = t + ((int64_t)1 << 32);
+        for (int s = ra; s <= rb; ++s, u += beta) {
+          if ((unsigned)(s - lo) > span) continue;
+          const ss_f32x4* cell = lay + (size_t)s * pitch + (int)(u >> 32);
+          const ss_f32x4 q0 = cell[0], q1 = cell[1];
+          const float fr = (float)(uint32_t)u;
+          const float z0 = __builtin_amdgcn_fmed3f(fmaf(-fabsf(w.c1 - fr), w.kz, w.pz), 0.f, 1.f);
+          const float z1 = __builtin_amdgcn_fmed3f(fmaf(fr, w.kz, w.pz1), 0.f, 1.f);
+#pragma unroll
+          for (int z = 0; z < SS_PLANES; ++z) tot[z] += (double)fmaf(z1, q1[z], z0 * q0[z]);
+        }
+      }
+    });
+  }
+  if (!on) return;
+  const int R = g.nrays, A = g.nangles, slice0 = group * ss_planes_slices(rp.kind);
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) {
+    const SSPlane pl = ss_plane(rp.kind, z);
+    const int kz = pl.turn ? R - 1 - k : k, jz = pl.mirror ? A - 1 - j : j;
+    if (slice0 + pl.slice >= rp.nslices) continue;                     // a group past the last slice
+    if ((pl.turn && kz == k) || (pl.mirror && jz == j)) continue;     // its own half turn or mirror
+    const size_t slice = slice0 + pl.slice;
+    if (PARTIAL)
+      part[((slice * rp.nslab + slab) * A + jz) * R + kz] = tot[z];
+    else
+      sino[(slice * R + kz) * A + jz] = (float)(tot[z] * a.tr_lmax);
+  }
+}
+
+// sino[slice][r][a] = lmax times the sum, in order, of the slabs' partial sums (exact-geometry
+// angles).  A block moves 32 angles x 32 rays.
+__global__ __launch_bounds__(256) void k_dda_radon_finish(SSDdaGeom g, const SSDdaAngle* __restrict__ angles, int nslab,
+                                                          const double* __restrict__ part, float* __restrict__ sino) {
+  __shared__ float T[32][33];
+  const int R = g.nrays, A = g.nangles;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int r0 = blockIdx.x * 32, a0 = blockIdx.y * 32;
+  const size_t slice = blockIdx.z;
+  for (int yy = ty; yy < 32; yy += 8) {
+    const int a = a0 + yy, r = r0 + tx;
+    double sum = 0.0;
+    if (a < A && r < R && angles[a].fixed) {
+      const double* __restrict__ src = part + (slice * nslab * A + a) * R + r;
+#pragma unroll 4
+      for (int s = 0; s < nslab; ++s) sum += src[(size_t)s * A * R];
+      sum *= angles[a].tr_lmax;
+    }
+    T[yy][tx] = (float)sum;
+  }
+  __syncthreads();
+  for (int yy = ty; yy < 32; yy += 8) {
+    const int r = r0 + yy, a = a0 + tx;
+    if (a < A && r < R && angles[a].fixed) sino[(slice * R + r) * A + a] = T[tx][yy];
+  }
+}
+
 // ---------------------------------------------------------------- transpose (scatter)
 
 // acc: pixels of angles whose fast axis is the line ([lines][cols]); accT: the others
@@ -443,12 +853,6 @@ __global__ __launch_bounds__(256) void k_dda_gather(SSDdaGeom g, const SSDdaGath
 // [1, 6 + span] for span = (cols - 1)|kx| + (lines - 1)|ky| of the block (the FP32
 // fraction is within 1e-5 ray units of the FP64 value, so floor is off by at most one),
 // and ws >= span + 8.  Terms are summed in FP32 over a group, those sums in FP64.
-// s_waitcnt immediates (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt
-// 11:8; a counter at its maximum is not waited on)
-#define DDA_WAIT_VM0 0x0F70
-#define DDA_WAIT_LGKM0 0xC07F
-#define DDA_WAIT_VM_CHUNK (0x0F70 | (DDA_WS_ROWS / 2))  // vmcnt(DDA_WS_ROWS / 2), below 16
-typedef float dda_f2v __attribute__((ext_vector_type(2)));
 __device__ float dda_raw_load_f32(__amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset,
                                   int aux) __asm("llvm.amdgcn.raw.ptr.buffer.load.f32");
 
@@ -460,6 +864,7 @@ __device__ __forceinline__ int dda_floor_i32(float v) {
 
 #define DDA_G2_MISS (-0x7fffffff - 1)
 typedef __attribute__((address_space(3))) float dda_lds_float;
+typedef __attribute__((address_space(3))) const ss_f32x4* dda_lds_cell;
 
 template <typename T, int G>
 __global__ __launch_bounds__(256) void k_dda_gather2(SSDdaGeom g, const SSDdaGatherAngle* __restrict__ ga, int nga,
@@ -545,6 +950,164 @@ __global__ __launch_bounds__(256) void k_dda_gather2(SSDdaGeom g, const SSDdaGat
     if (i0 + rr < g.lines) out[(size_t)(i0 + rr) * g.cols + j] = T(tot[rr]);
 }
 
+// The two-candidate gather in planes.  k_dda_gather2 is bound by its LDS reads (one two-word
+// read per update) and by the floor, fraction and weights of every update, and launches of few
+// tiles walk all angles serially.  Here a pixel's ray coordinate rc - half, its candidates
+// and weights serve four values (SSPlane):
+//   SS_PLANES_QUAD    the pixel, its half turn (ray R - 1 - r), its mirror x -> -x (angle
+//                     A - 1 - a) and the half turn of that, tiles over a quarter of the image;
+//   SS_PLANES_PAIR    two slices and their half turns, tiles over half the image;
+//   SS_PLANES_SLICES  four slices.
+// sp[a][r] holds the planes' lmax-scaled values of a ray together (k_dda_rows_planes), copied
+// into LDS windows of ws rays by 16-byte buffer-to-LDS loads (rays off the detector read 0
+// through the range check); a lane reads a candidate's four values with one 16-byte read
+// (column order: ss_bp_column).  Geometry as in k_dda_gather2: per (thread, angle) FP64 gives
+// rc - half from the window's base and splits it; the thread's DDA_GP_ROWS consecutive lines
+// step from that fraction by ky in FP32.  Sums are taken in FP32 over DDA_GP_ANGLES angles,
+// those in FP64; with angle groups the groups' FP64 partial images are added by k_dda_fold.
+// Window: a tile's rc - half lies in [lo, hi] and its candidates in floor(lo) + 1 .. floor(hi) + 2;
+// the window holds floor(lo) .. floor(lo) + ws - 1, a ray of margin either side for rounding.
+//
+// Work per four updates: 7 VALU for the candidates and weights, 8 FMAs, two reads.
+// 1024^2 x 721, backprojection: 575 -> 141 us (this kernel 555 -> 112: VALU issue and LDS reads about
+// equal); 2048^2 x 1500 1670 -> 810; 16 x 512^2 x 360 430 -> 250; 256^2 x 180 136 -> 52.
+__global__ __launch_bounds__(256, 4) void k_dda_gather_planes(SSDdaGeom g, const SSDdaGatherAngle* __restrict__ ga,
+                                                              int nga, const ss_f32x4* __restrict__ planes, int kind,
+                                                              int nslices, int ws, int ngroups, int tcols, int trows,
+                                                              double* __restrict__ part) {
+  constexpr int ROWS = DDA_GP_ROWS, NA = DDA_GP_ANGLES, TH = 8 * ROWS;
+  __shared__ ss_f32x4 seg[NA * DDA_GP_WSMAX];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int z0 = blockIdx.x / (tcols * trows), tile = blockIdx.x - z0 * (tcols * trows);
+  const int group = z0 / ngroups, gi = z0 - group * ngroups;
+  const int r0 = tile / tcols * TH, c0 = tile % tcols * 32;
+  const int tx = ss_bp_column(tid), ty = (tid >> 5) * ROWS;
+  const int k0 = (int)((long long)gi * nga / ngroups), k1 = (int)((long long)(gi + 1) * nga / ngroups);
+  const ss_f32x4* __restrict__ sp = planes + (size_t)group * g.nangles * g.nrays;
+  const double txd = tx, tyd = ty;
+  double tot[ROWS][SS_PLANES];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+    for (int z = 0; z < SS_PLANES; ++z) tot[i][z] = 0.0;
+  for (int ka = k0; ka < k1; ka += 64) {
+    const int np = min(64, k1 - ka);
+    // angle ka + lane: rc - half at the tile's origin from the window's first ray, less 1
+    double o = 0.0;
+    int first = 0, row = 0;
+    bool meets = false;
+    if (lane < np) {
+      const SSDdaGatherAngle& A = ga[ka + lane];
+      const double v = fma((double)c0, A.kx, fma((double)r0, A.ky, A.k0h));
+      const double lo = v + fmin(0.0, 31 * A.kx) + fmin(0.0, (TH - 1) * A.ky);
+      const double hi = v + fmax(0.0, 31 * A.kx) + fmax(0.0, (TH - 1) * A.ky);
+      meets = hi >= -4.0 && lo <= g.nrays + 4.0;  // candidates floor(rc - half) + 1 and + 2
+      first = meets ? (int)floor(lo) : 0;
+      o = v - (first - 1);
+      row = A.a;
+    }
+    const unsigned long long near = __ballot(meets);
+    for (int ks = 0; ks < np; ks += NA) {
+      const int na = min(NA, np - ks);
+      __syncthreads();  // the previous windows are read
+      for (int t = wv; t < na; t += 4) {
+        if (!(near >> (ks + t) & 1)) continue;
+        const int a = __builtin_amdgcn_readlane(row, ks + t), base = __builtin_amdgcn_readlane(first, ks + t);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(sp + (size_t)a * g.nrays), (short)0, g.nrays * (int)sizeof(ss_f32x4), DDA_RSRC_DWORD3);
+        for (int m = 0; m < ws; m += 64) {
+          // the whole offset in the register: the range check sees a ray below 0 as out of range
+          int off = (base + m + lane) * (int)sizeof(ss_f32x4);
+          __asm__ volatile("" : "+v"(off));
+          if (m + lane < ws)  // active lanes write their record: stay in this window
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (dda_lds_ptr)(seg + t * DDA_GP_WSMAX + m), 16, off, 0, 0, 0);
+        }
+      }
+      __syncthreads();
+      float sum[ROWS][SS_PLANES];
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+        for (int z = 0; z < SS_PLANES; ++z) sum[i][z] = 0.f;
+      for (int t = 0; t < na; ++t) {
+        if (!(near >> (ks + t) & 1)) continue;
+        const SSDdaGatherAngle& A = ga[ka + ks + t];
+        const long long ob = __builtin_bit_cast(long long, o);
+        const double ot = __builtin_bit_cast(
+            double, ((long long)__builtin_amdgcn_readlane((int)(ob >> 32), ks + t) << 32) |
+                        (unsigned)__builtin_amdgcn_readlane((int)ob, ks + t));
+        const double v = fma(txd, A.kx, fma(tyd, A.ky, ot));
+        const double b = floor(v);
+        const float g0 = (float)(v - b);
+        // candidate floor(rc - half) + 1 is record floor(v) of the window
+        const dda_lds_cell q = (dda_lds_cell)(seg + t * DDA_GP_WSMAX + (int)b);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+          const float gr = i == 0 ? g0 : fmaf((float)i, A.kyf, g0);
+          const int fl = i == 0 ? 0 : dda_floor_i32(gr);
+          const float fr = i == 0 ? g0 : __builtin_amdgcn_fractf(gr);
+          const ss_f32x4 q0 = q[fl], q1 = q[fl + 1];
+          const float w0 = __builtin_amdgcn_fmed3f(fmaf(-fabsf(A.c1 - fr), A.kz, A.pz), 0.f, 1.f);
+          const float w1 = __builtin_amdgcn_fmed3f(fmaf(fr, A.kz, A.pz1), 0.f, 1.f);
+#pragma unroll
+          for (int z = 0; z < SS_PLANES; ++z) sum[i][z] = fmaf(w1, q1[z], fmaf(w0, q0[z], sum[i][z]));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+        for (int z = 0; z < SS_PLANES; ++z) tot[i][z] += (double)sum[i][z];
+    }
+  }
+  const size_t npix = (size_t)g.lines * g.cols;
+  const int slice0 = group * ss_planes_slices(kind);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int row = r0 + ty + i, col = c0 + tx;
+#pragma unroll
+    for (int z = 0; z < SS_PLANES; ++z) {
+      const SSPlane pl = ss_plane(kind, z);
+      const int mr = pl.turn ? 1 : 0, mc = pl.turn != pl.mirror ? 1 : 0;
+      if (slice0 + pl.slice >= nslices || row >= g.lines || col >= g.cols) continue;
+      // tiles reach the image's middle; a pixel that is its own image is stored once
+      if (kind != SS_PLANES_SLICES && 2 * row + mr > g.lines - 1) continue;
+      if (kind == SS_PLANES_QUAD && 2 * col + mc > g.cols - 1) continue;
+      const int zr = mr ? g.lines - 1 - row : row, zc = mc ? g.cols - 1 - col : col;
+      part[((size_t)(slice0 + pl.slice) * ngroups + gi) * npix + (size_t)zr * g.cols + zc] = tot[i][z];
+    }
+  }
+}
+
+// rows[group][a][r] = the planes' values sino[slice][r'][a'] * scale[a'] of ray r at angle a
+__global__ __launch_bounds__(256) void k_dda_rows_planes(int R, int A, int kind, int nslices,
+                                                         const float* __restrict__ sino,
+                                                         const float* __restrict__ scale, ss_f32x4* __restrict__ rows) {
+  __shared__ float T[SS_PLANES][32][33];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int br = blockIdx.x * 32, ba = blockIdx.y * 32;
+#pragma unroll
+  for (int z = 0; z < SS_PLANES; ++z) {
+    const SSPlane pl = ss_plane(kind, z);
+    const size_t slice = (size_t)min((int)blockIdx.z * ss_planes_slices(kind) + pl.slice, nslices - 1);
+    const float* __restrict__ src = sino + slice * (size_t)R * A;
+    const int a = ba + tx, az = pl.mirror ? A - 1 - a : a;
+    const float sc = a < A ? scale[az] : 0.f;
+#pragma unroll
+    for (int yy = ty; yy < 32; yy += 8) {
+      const int r = br + yy, rz = pl.turn ? R - 1 - r : r;
+      T[z][tx][yy] = a < A && r < R ? src[(size_t)rz * A + az] * sc : 0.f;
+    }
+  }
+  __syncthreads();
+  ss_f32x4* dst = rows + (size_t)blockIdx.z * A * R;
+#pragma unroll
+  for (int yy = ty; yy < 32; yy += 8) {
+    const int a = ba + yy, r = br + tx;
+    if (a < A && r < R) dst[(size_t)a * R + r] = ss_f32x4{T[0][yy][tx], T[1][yy][tx], T[2][yy][tx], T[3][yy][tx]};
+  }
+}
+
 // rows[slice][a][2 + r] = sino[slice][r][a] * scale[a], two zeros either side of each row
 __global__ __launch_bounds__(256) void k_dda_sino_rows(int R, int A, const float* __restrict__ sino,
                                                        const float* __restrict__ scale, float* __restrict__ rows) {
@@ -607,11 +1170,13 @@ __global__ __launch_bounds__(256) void k_dda_straight(SSDdaGeom g, const SSDdaSt
     vline[slice * g.lines + s] = T(sum);
 }
 
-// out[lines][cols] = acc[lines][cols] + accT[cols][lines]^T + vcol[cols] + vline[lines]
-// (accT, vcol, vline may be null), divided by w when given.
+// out[lines][cols] = acc[lines][cols] + more[lines][cols] + accT[cols][lines]^T + vcol[cols] +
+// vline[lines] (more, accT, vcol, vline may be null), divided by w when given.  acc: the sum, in order, of
+// ngroups partial images [slice][group][lines][cols] of type P.
 // Block (32, 8) handles a 32 x 32 tile; accT is read along its lines through LDS.
-template <typename T, typename Out>
-__global__ __launch_bounds__(256) void k_dda_fold(int lines, int cols, const T* __restrict__ acc,
+template <typename T, typename Out, typename P>
+__global__ __launch_bounds__(256) void k_dda_fold(int lines, int cols, const P* __restrict__ acc, int ngroups,
+                                                  const T* __restrict__ more,
                                                   const T* __restrict__ accT, const T* __restrict__ vcol,
                                                   const T* __restrict__ vline, const double* __restrict__ w,
                                                   Out* __restrict__ out) {
@@ -629,7 +1194,11 @@ __global__ __launch_bounds__(256) void k_dda_fold(int lines, int cols, const T* 
     const int i = i0 + ii, j = j0 + threadIdx.x;
     if (i < lines && j < cols) {
       const size_t p = (size_t)i * cols + j;
-      T v = acc[slice * npix + p] + tile[threadIdx.x][ii];
+      P sum = P(0);
+#pragma unroll 4
+      for (int k = 0; k < ngroups; ++k) sum += acc[(slice * ngroups + k) * npix + p];
+      T v = T(sum) + tile[threadIdx.x][ii];
+      if (more) v += more[slice * npix + p];
       if (vcol) v += vcol[slice * cols + j] + vline[slice * lines + i];
       out[slice * npix + p] = w ? Out((double)v / w[p]) : Out(v);
     }
@@ -684,10 +1253,81 @@ static dim3 dda_tiles(int lines, int cols, int nslices) {
   return dim3((cols + DDA_TILE - 1) / DDA_TILE, (lines + DDA_TILE - 1) / DDA_TILE, nslices);
 }
 
-hipError_t dda_launch_radon(const SSDdaGeom& g, const SSDdaAngle* angles, const float* img, float* pad, float* sino,
-                            int nslices, hipStream_t stream) {
-  float* img_pad = pad;
-  float* imgT_pad = pad + (size_t)nslices * g.lines * dda_pad_pitch(g.cols);
+static SSDdaRadonPlanes dda_radon_planes(const SSDdaGeom& g, const SSDdaTransposePlan& tp, int kind, int nslices) {
+  SSDdaRadonPlanes rp;
+  rp.kind = kind;
+  rp.nslices = nslices;
+  rp.nangles = kind == SS_PLANES_QUAD ? (g.nangles + 1) / 2 : g.nangles;
+  rp.nrays = kind == SS_PLANES_SLICES ? g.nrays : (g.nrays + 1) / 2;
+  rp.order = ss_planes_order(rp.nrays, rp.nangles);
+  const int nf = std::max(g.lines, g.cols);
+  const long long blocks = (long long)rp.order.blocks * ss_planes_groups(kind, nslices);
+  rp.nslab = ss_radon_slab_plan(nf, blocks, &rp.slab_rows,
+                                (int)std::min<long long>(SS_PLANES_SLAB_BLOCKS, blocks * (nf / DDA_RP_MIN_ROWS)));
+  rp.straight = tp.straight;
+  rp.nstraight = tp.nstraight;
+  rp.walk = tp.walk;
+  rp.nwalk = tp.nwalk;
+  return rp;
+}
+
+static long long dda_radon_planes_blocks(const SSDdaGeom& g, const SSDdaRadonPlanes& rp) {
+  const int wide = RADON_WAVES * SS_WAVE;
+  return (long long)rp.order.blocks * rp.nslab * ss_planes_groups(rp.kind, rp.nslices) +
+         ((long long)rp.nstraight * ((g.nrays + 63) / 64) + (long long)rp.nwalk * ((g.nrays + wide - 1) / wide)) *
+             rp.nslices;
+}
+
+SSDdaRadonForm dda_radon_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, int nslices) {
+  SSDdaRadonForm f{SS_PLANES_NONE, 1, 0, 0};
+  f.layout = sizeof(float) * dda_radon_scratch_floats(g, nslices);
+  if (tp.ngather == 0) return f;
+  // a traced ray's pixel offsets are ints
+  if ((long long)std::max(g.lines, g.cols) * (std::max(g.lines, g.cols) + 2 * DDA_RP_PAD) >= (1LL << 31)) return f;
+  int kind = SS_PLANES_NONE;
+  if (tp.sym & DDA_SYM_MIRROR)
+    kind = SS_PLANES_QUAD;
+  else if ((tp.sym & DDA_SYM_TURN) && nslices >= 2)
+    kind = SS_PLANES_PAIR;
+  else if (nslices >= 3)
+    kind = SS_PLANES_SLICES;
+  if (kind == SS_PLANES_NONE) return f;
+  const int groups = ss_planes_groups(kind, nslices);
+  const SSDdaRadonPlanes rp = dda_radon_planes(g, tp, kind, nslices);
+  if (dda_radon_planes_blocks(g, rp) > 0x7fffffffLL) return f;
+  f.kind = kind;
+  f.nslab = rp.nslab;
+  f.layout = sizeof(ss_f32x4) * (size_t)groups *
+             ((size_t)g.lines * (g.cols + 2 * DDA_RP_PAD) + (size_t)g.cols * (g.lines + 2 * DDA_RP_PAD));
+  f.part = rp.nslab > 1 ? sizeof(double) * (size_t)nslices * rp.nslab * g.nangles * g.nrays : 0;
+  return f;
+}
+
+hipError_t dda_launch_radon(const SSDdaGeom& g, const SSDdaTransposePlan& tp, const float* img, void* layout,
+                            double* part, float* sino, int nslices, hipStream_t stream) {
+  const SSDdaAngle* angles = tp.angles;
+  const SSDdaRadonForm form = dda_radon_form(g, tp, nslices);
+  if (form.kind != SS_PLANES_NONE) {
+    const int groups = ss_planes_groups(form.kind, nslices);
+    const SSDdaRadonPlanes rp = dda_radon_planes(g, tp, form.kind, nslices);
+    ss_f32x4* L = static_cast<ss_f32x4*>(layout);
+    ss_f32x4* LT = L + (size_t)groups * g.lines * (g.cols + 2 * DDA_RP_PAD);
+    hipLaunchKernelGGL(k_dda_pad_planes, dda_tiles(g.lines, g.cols, groups), dim3(256), 0, stream, g.lines, g.cols,
+                       form.kind, nslices, img, L, LT);
+    const unsigned blocks = (unsigned)dda_radon_planes_blocks(g, rp);
+    if (rp.nslab > 1) {
+      hipLaunchKernelGGL(k_dda_radon_planes<true>, dim3(blocks), dim3(RADON_WAVES * SS_WAVE), 0, stream, g, angles, rp,
+                         (const ss_f32x4*)L, (const ss_f32x4*)LT, sino, part);
+      hipLaunchKernelGGL(k_dda_radon_finish, dim3((g.nrays + 31) / 32, (g.nangles + 31) / 32, nslices), dim3(256), 0,
+                         stream, g, angles, rp.nslab, (const double*)part, sino);
+    } else {
+      hipLaunchKernelGGL(k_dda_radon_planes<false>, dim3(blocks), dim3(RADON_WAVES * SS_WAVE), 0, stream, g, angles, rp,
+                         (const ss_f32x4*)L, (const ss_f32x4*)LT, sino, part);
+    }
+    return hipGetLastError();
+  }
+  float* img_pad = static_cast<float*>(layout);
+  float* imgT_pad = img_pad + (size_t)nslices * g.lines * dda_pad_pitch(g.cols);
   hipLaunchKernelGGL(k_dda_pad_images, dda_tiles(g.lines, g.cols, nslices), dim3(DDA_TILE, 8), 0, stream, g.lines,
                      g.cols, img, img_pad, imgT_pad);
   hipLaunchKernelGGL(k_dda_radon, dim3((g.nrays + 255) / 256, g.nangles, nslices), dim3(256), 0, stream, g, angles,
@@ -695,12 +1335,64 @@ hipError_t dda_launch_radon(const SSDdaGeom& g, const SSDdaAngle* angles, const 
   return hipGetLastError();
 }
 
+static int dda_gp_cols(const SSDdaGeom& g, int kind) {
+  return ((kind == SS_PLANES_QUAD ? (g.cols + 1) / 2 : g.cols) + 31) / 32;
+}
+static int dda_gp_rows(const SSDdaGeom& g, int kind) {
+  return ((kind == SS_PLANES_SLICES ? g.lines : (g.lines + 1) / 2) + 8 * DDA_GP_ROWS - 1) / (8 * DDA_GP_ROWS);
+}
+
+SSDdaGatherForm dda_gather_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, bool ones, int nslices) {
+  SSDdaGatherForm f{SS_PLANES_NONE, 1};
+  if (ones || tp.ngather == 0 || tp.planes_ws <= 0) return f;
+  if (tp.sym & DDA_SYM_MIRROR)
+    f.kind = SS_PLANES_QUAD;
+  else if ((tp.sym & DDA_SYM_TURN) && nslices >= 2)
+    f.kind = SS_PLANES_PAIR;
+  else if (nslices >= 3)
+    f.kind = SS_PLANES_SLICES;
+  if (f.kind == SS_PLANES_NONE) return f;
+  const long long tiles = (long long)dda_gp_cols(g, f.kind) * dda_gp_rows(g, f.kind) * ss_planes_groups(f.kind, nslices);
+  if (tiles * DDA_GP_MAXGROUPS > 0x7fffffffLL) return SSDdaGatherForm{SS_PLANES_NONE, 1};
+  const long long want = std::max<long long>((DDA_GP_BLOCKS + tiles / 2) / tiles, tiles <= DDA_GP_PAIR_TILES ? 2 : 1);
+  f.ngroups = (int)std::min<long long>({DDA_GP_MAXGROUPS, want, (tp.ngather + DDA_GP_ANGLES - 1) / DDA_GP_ANGLES});
+  return f;
+}
+
+SSDdaTransposeScratch dda_transpose_scratch(const SSDdaGeom& g, const SSDdaTransposePlan& tp, bool ones, int nslices,
+                                            size_t sizeof_t) {
+  const size_t npix = (size_t)g.lines * g.cols, n = npix * nslices;
+  const SSDdaGatherForm f = dda_gather_form(g, tp, ones, nslices);
+  SSDdaTransposeScratch b;
+  if (f.kind != SS_PLANES_NONE) {
+    b.sino = sizeof(ss_f32x4) * (size_t)g.nrays * g.nangles * ss_planes_groups(f.kind, nslices);
+    b.acc = sizeof(double) * n * f.ngroups;
+    // the traced angles' two images, or the straight angles' vectors
+    b.accT = tp.nwalk > 0 ? 2 * sizeof_t * n : (tp.nstraight > 0 ? sizeof_t * (size_t)nslices * (g.lines + g.cols) : 0);
+  } else {
+    b.sino = sizeof(float) * (size_t)(g.nrays + 4) * g.nangles * nslices;
+    b.acc = b.accT = sizeof_t * n;
+  }
+  return b;
+}
+
 template <typename T, typename Out>
 hipError_t dda_launch_transpose(const SSDdaGeom& g, const SSDdaTransposePlan& tp, const float* sino, bool ones,
-                                float* sinoT, T* acc, T* accT, const double* w, Out* out, int nslices,
+                                float* sinoT, void* acc_, T* accT, const double* w, Out* out, int nslices,
                                 hipStream_t stream) {
   const size_t n = (size_t)g.lines * g.cols * nslices;
-  if (tp.ngather > 0) {
+  T* acc = static_cast<T*>(acc_);
+  const SSDdaGatherForm form = dda_gather_form(g, tp, ones, nslices);
+  if (form.kind != SS_PLANES_NONE) {
+    const int groups = ss_planes_groups(form.kind, nslices);
+    const int tc = dda_gp_cols(g, form.kind), tr = dda_gp_rows(g, form.kind);
+    ss_f32x4* rows = reinterpret_cast<ss_f32x4*>(sinoT);
+    hipLaunchKernelGGL(k_dda_rows_planes, dim3((g.nrays + 31) / 32, (g.nangles + 31) / 32, groups), dim3(256), 0,
+                       stream, g.nrays, g.nangles, form.kind, nslices, sino, tp.row_scale, rows);
+    hipLaunchKernelGGL(k_dda_gather_planes, dim3((unsigned)(tc * tr * groups * form.ngroups)), dim3(256), 0, stream, g,
+                       tp.gather, tp.ngather, (const ss_f32x4*)rows, form.kind, nslices, tp.planes_ws, form.ngroups,
+                       tc, tr, static_cast<double*>(acc_));
+  } else if (tp.ngather > 0) {
     if (!ones)  // angle-major, lmax-scaled, zero-padded copy of the sinogram
       hipLaunchKernelGGL(k_dda_sino_rows, dda_tiles(g.nrays, g.nangles, nslices), dim3(DDA_TILE, 8), 0, stream,
                          g.nrays, g.nangles, sino, tp.row_scale, sinoT);
@@ -727,7 +1419,8 @@ hipError_t dda_launch_transpose(const SSDdaGeom& g, const SSDdaTransposePlan& tp
     hipLaunchKernelGGL(k_dda_fill<T>, dim3(1024), dim3(256), 0, stream, acc, n);
   }
   if (tp.nwalk > 0) {
-    hipLaunchKernelGGL(k_dda_fill<T>, dim3(1024), dim3(256), 0, stream, accT, n);
+    if (form.kind != SS_PLANES_NONE) acc = accT + n;  // beside the gather's FP64 images
+    hipLaunchKernelGGL(k_dda_fill<T>, dim3(1024), dim3(256), 0, stream, accT, form.kind != SS_PLANES_NONE ? 2 * n : n);
     hipLaunchKernelGGL(k_dda_scatter<T>, dim3((g.nrays + 255) / 256, tp.nwalk, nslices), dim3(256), 0, stream, g,
                        tp.angles, tp.walk, sino, ones ? 1 : 0, acc, accT);
   }
@@ -741,9 +1434,14 @@ hipError_t dda_launch_transpose(const SSDdaGeom& g, const SSDdaTransposePlan& tp
     hipLaunchKernelGGL(k_dda_straight<T>, dim3((g.cols + g.lines + 255) / 256, nslices), dim3(256), 0, stream, g,
                        tp.straight, tp.nstraight, tp.ranges, sino, ones ? 1 : 0, vcol, vline);
   }
-  hipLaunchKernelGGL((k_dda_fold<T, Out>), dda_tiles(g.lines, g.cols, nslices), dim3(DDA_TILE, 8), 0, stream, g.lines,
-                     g.cols, (const T*)acc, (const T*)(tp.nwalk > 0 ? accT : nullptr), (const T*)vcol,
-                     (const T*)vline, w, out);
+  if (form.kind != SS_PLANES_NONE)
+    hipLaunchKernelGGL((k_dda_fold<T, Out, double>), dda_tiles(g.lines, g.cols, nslices), dim3(DDA_TILE, 8), 0, stream,
+                       g.lines, g.cols, (const double*)acc_, form.ngroups, (const T*)(tp.nwalk > 0 ? acc : nullptr),
+                       (const T*)(tp.nwalk > 0 ? accT : nullptr), (const T*)vcol, (const T*)vline, w, out);
+  else
+    hipLaunchKernelGGL((k_dda_fold<T, Out, T>), dda_tiles(g.lines, g.cols, nslices), dim3(DDA_TILE, 8), 0, stream,
+                       g.lines, g.cols, (const T*)acc, 1, (const T*)nullptr,
+                       (const T*)(tp.nwalk > 0 ? accT : nullptr), (const T*)vcol, (const T*)vline, w, out);
   return hipGetLastError();
 }
 
@@ -758,11 +1456,11 @@ hipError_t dda_launch_to_f32(const double* src, float* dst, size_t n, hipStream_
 }
 
 template hipError_t dda_launch_transpose<float, float>(const SSDdaGeom&, const SSDdaTransposePlan&, const float*,
-                                                      bool, float*, float*, float*, const double*, float*, int,
+                                                      bool, float*, void*, float*, const double*, float*, int,
                                                       hipStream_t);
 template hipError_t dda_launch_transpose<double, float>(const SSDdaGeom&, const SSDdaTransposePlan&, const float*,
-                                                       bool, float*, double*, double*, const double*, float*, int,
+                                                       bool, float*, void*, double*, const double*, float*, int,
                                                        hipStream_t);
 template hipError_t dda_launch_transpose<double, double>(const SSDdaGeom&, const SSDdaTransposePlan&, const float*,
-                                                        bool, float*, double*, double*, const double*, double*, int,
+                                                        bool, float*, void*, double*, const double*, double*, int,
                                                         hipStream_t);

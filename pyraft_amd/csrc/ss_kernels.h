@@ -13,6 +13,7 @@
 #include <stdint.h>
 
 #include "ss_geometry.h"
+#include "ss_planes.h"
 
 // Radon output modes; SS_OUT_PARTIAL: a row slab's partial ray sums (launches of few
 // blocks), which a finishing pass stores in one of the other modes
@@ -91,12 +92,6 @@ hipError_t ss_launch_plan_bounds(const SSGeom& g, const SSAngle* angles, int2* b
 hipError_t ss_launch_plan_wave_bounds(const SSGeom& g, const int2* bounds, int4* wbounds, hipStream_t stream);
 
 // ---- layouts
-// The Radon in planes (k_radon_planes): what the four planes of a launch are, the slices that
-// a group of planes covers, and the groups of a launch
-enum { SS_PLANES_NONE = 0, SS_PLANES_QUAD = 1, SS_PLANES_PAIR = 2, SS_PLANES_SLICES = 3 };
-static inline __host__ __device__ int ss_planes_slices(int kind) {
-  return kind == SS_PLANES_QUAD ? 1 : (kind == SS_PLANES_PAIR ? 2 : 4);
-}
 // the exact transpose's further forms: a slice and its half turn, two slices, one
 enum { SS_RT_TURN = 4, SS_RT_TWO = 5, SS_RT_ONE = 6 };
 static inline __host__ __device__ int ss_rt_slices(int kind) {
@@ -106,9 +101,6 @@ static inline __host__ __device__ int ss_rt_planes(int kind) {
   return kind <= SS_PLANES_SLICES ? 4 : (kind == SS_RT_ONE ? 1 : 2);
 }
 #define SS_RT_SAME_SLICES 8  // launches of up to this many slices sum in one slice's order
-static inline int ss_planes_groups(int kind, int nslices) {
-  return (nslices + ss_planes_slices(kind) - 1) / ss_planes_slices(kind);
-}
 // the gather layouts are built in square tiles of SS_GATHER_TILE records per direction;
 // records q = 0..n+1 of each row
 #define SS_GATHER_TILE 64
@@ -137,9 +129,6 @@ struct SSEmRatioArgs {
 // every (angle block, ray group) into slabs taken by separate blocks, which write partial
 // ray sums; a finishing pass adds them.  ss_radon_slab_plan: slab count (1: no division)
 // and rows per slab of an n x n image in a launch of `blocks` blocks.
-#ifndef RADON_WAVES
-#define RADON_WAVES 8  // angles (one per wave) of a Radon block
-#endif
 #define SS_RADON_SLAB_BLOCKS (8192 / RADON_WAVES)
 // the planes form (two blocks per CU): 1024^2 x 720, 384 blocks, 160 us undivided, 138 in four
 // slabs

@@ -13,7 +13,6 @@
 #include "ss_kernels.h"
 #include "ss_plan_logic.h"
 
-#define SS_WAVE 64
 #define SS_INV_FIX 2.3283064365386963e-10f  // 2^-32
 #define SS_FIX_ONE_I64 ((int64_t)1 << 32)    // one cell in Q32.32
 
@@ -287,16 +286,6 @@ __device__ __forceinline__ void ss_radon_store(const SSRadonView& p, int j, int 
 // rows into slabs taken by separate blocks instead (ss_radon_slab_plan).
 
 typedef float ss_f32x2 __attribute__((ext_vector_type(2)));
-typedef float ss_f32x4 __attribute__((ext_vector_type(4)));
-
-// Column of a lane in its 32-pixel tile row.  A 16-byte LDS read serves 16 lanes of a half
-// wave per pass, the lanes 0-3, 12-15, 20-27 and then the others; giving each of the two
-// sets 16 neighbouring columns keeps a pass within 16 neighbouring records, so that no two
-// of them share a bank (pixels are at most one ray apart).
-__device__ __forceinline__ int ss_bp_column(int lane) {
-  const int q = (lane >> 2) & 7;
-  return ((0x73261540 >> (4 * q)) & 7) * 4 + (lane & 3);
-}
 
 #define SS_RSRC_DWORD3 0x00020000  // gfx9 buffer word 3: 32-bit data format, no swizzle
 
@@ -321,12 +310,6 @@ struct SSRadonShape {
   static constexpr int CAP = SH == 0 ? 4096 : 4864;
   static constexpr int CHUNK = SH == 0 ? 32 : 40;
 };
-#ifndef RADON_ROW_ROUND
-#define RADON_ROW_ROUND 8  // chunk rows rounded down to a multiple of this where the window allows
-#endif
-
-#define RADON_TABLE SS_WAVE  // chunks per window table: one (chunk, wave) pair per thread
-
 template <int CAP>
 struct SSRadonLds {
   double red[RADON_WAVES];
@@ -336,18 +319,6 @@ struct SSRadonLds {
   int2 table[RADON_TABLE];       // per chunk of the super-chunk: first staged record, records per row
   __attribute__((aligned(16))) float2 stage[CAP + 2];  // chunk window; record CAP stays (0, 0)
 };
-
-typedef __attribute__((address_space(1))) const void* ss_global_cptr;
-typedef __attribute__((address_space(3))) void* ss_lds_ptr;
-
-// wave-uniform copies (scalar registers) of values the compiler cannot prove uniform
-__device__ __forceinline__ int ss_rfl(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t ss_rfl64(int64_t v) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-__device__ __forceinline__ float ss_rflf(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 
 // Direct sample reader: (row s, trajectory u) -> (lower tap, difference), where u is
 // the Q32.32 trajectory plus one cell, its high word the record index.
@@ -459,53 +430,6 @@ __device__ __forceinline__ void ss_radon_rows(const Rd& rd, int sa, int sb, int 
     }
     u += beta;
   }
-}
-
-// Window table of `nch` chunks of `rows` sample rows from row sc (the last chunk ends
-// at s_hi at the latest): for each chunk, the gather records [rec0, rec0 + Wc) of each
-// row that the block's waves read in its rows (Wc = 0: none).  Each thread takes one
-// (chunk, wave) pair, bounds the cells of that wave's rays over the chunk's rows at the
-// corners (the trajectory is affine in ray and row; valid samples have cells in
-// [-1, n-1]), and the RADON_WAVES lanes of a chunk take the union.  Returns the widest
-// Wc of the table (block-uniform); `pass` selects the reduction slots, so that a second
-// pass right after the first needs no barrier in between.
-template <bool PAIRS, class Lds>
-__device__ __forceinline__ int ss_radon_windows(Lds& lds, int pass, int sc, int rows, int nch, int s_hi, int n) {
-  const int t = threadIdx.x;
-  const int c = t / RADON_WAVES, w = t % RADON_WAVES;
-  int cmin = 0x7fffffff, cmax = -0x7fffffff;
-  if (c < nch) {
-    const int s0 = sc + c * rows, s1 = min(s0 + rows, s_hi + 1);
-    const int ra = max(s0, lds.wmeta[w][1]), rb = min(s1 - 1, lds.wmeta[w][2]);
-    if (lds.wmeta[w][0] >= 0 && ra <= rb) {
-      const int64_t beta = lds.wpar[w][2];
-      const int64_t c00 = lds.wpar[w][0] + (int64_t)ra * beta;
-      const int64_t c10 = lds.wpar[w][1] + (int64_t)ra * beta;
-      const int64_t ds = (int64_t)(rb - ra) * beta;
-      const int m0 = (int)(c00 >> 32), m1 = (int)(c10 >> 32);
-      const int m2 = (int)((c00 + ds) >> 32), m3 = (int)((c10 + ds) >> 32);
-      cmin = max(min(min(m0, m1), min(m2, m3)), -1);
-      cmax = min(max(max(m0, m1), max(m2, m3)), n - 1);
-    }
-  }
-  for (int off = 1; off < RADON_WAVES; off <<= 1) {
-    cmin = min(cmin, __shfl_xor(cmin, off));
-    cmax = max(cmax, __shfl_xor(cmax, off));
-  }
-  // pair records: cells c_lo..c_hi need records c_lo+1..c_hi+1; rec0 is even so that rows of
-  // the window start 16-byte aligned in the layout (even pitch) and in LDS (even Wc).  Plane
-  // cells (16 bytes each): c_lo+1..c_hi+2, the upper tap being the next cell
-  const int rec0 = PAIRS ? (cmin + 1) & ~1 : cmin + 1;
-  int wc = 0;
-  if (cmax >= cmin) wc = PAIRS ? ((cmax + 2 - rec0) + 1) & ~1 : cmax + 3 - rec0;
-  if (c >= nch) wc = 0;
-  if (c < nch && w == 0) lds.table[c] = make_int2(rec0, wc);
-  for (int off = 32; off > 0; off >>= 1) wc = max(wc, __shfl_xor(wc, off));
-  if ((t & (SS_WAVE - 1)) == 0) lds.wred[pass][t / SS_WAVE] = wc;
-  __syncthreads();
-  int wmax = 0;
-  for (int i = 0; i < RADON_WAVES; ++i) wmax = max(wmax, lds.wred[pass][i]);
-  return ss_rfl(wmax);
 }
 
 // One block's work: rays [grp*64, grp*64+64) of the RADON_WAVES angles starting at
@@ -759,24 +683,6 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE) void k_radon(SSDevPlan p, co
 // once.  Irregular rays have empty ranges here and go to k_radon_fixup.
 // =====================================================================================
 
-#define SS_PLANES 4
-
-// plane z of a launch: its slice within the group, whether it is the half turn of its image
-// and whether the mirror
-struct SSPlane {
-  int slice;
-  bool turn, mirror;
-};
-__device__ __host__ __forceinline__ SSPlane ss_plane(int kind, int z) {
-  if (kind == SS_PLANES_QUAD) return SSPlane{0, (z & 1) != 0, (z & 2) != 0};
-  if (kind == SS_PLANES_PAIR) return SSPlane{z >> 1, (z & 1) != 0, false};
-  return SSPlane{z, false, false};
-}
-
-// Ray of a lane within its group of 64: a 16-byte LDS read serves the lanes 0-3, 12-15,
-// 20-27 of a half wave in one pass and the others in the next; each set gets 16 neighbours.
-__device__ __forceinline__ int ss_plane_ray(int lane) { return (lane & 32) + ss_bp_column(lane); }
-
 // Layout row r of B (image rows) and row c of A (image columns), cells q in [0, n + 1]:
 //   LB[r][q] = (G_0, .., G_3)(r, q - 1),  LA[c][q] = (G_0, .., G_3)(q - 1, c)
 // with G_z plane z's image and 0 outside.  A block moves one 32 x 32 pixel tile.
@@ -819,24 +725,6 @@ __global__ __launch_bounds__(256) void k_gather_planes(const float* __restrict__
     }
   }
 }
-
-// staged cells per block and sample rows per chunk at most: two 512-thread blocks per CU
-#ifndef PLANES_CAP
-#define PLANES_CAP 4864
-#define PLANES_CHUNK 40
-#define PLANES_BLOCKS 2
-#endif
-
-struct SSPlanesLds {
-  double red[RADON_WAVES];
-  int64_t wpar[RADON_WAVES][3];  // as SSRadonLds
-  int wmeta[RADON_WAVES][4];
-  int wred[2][RADON_WAVES];
-  int2 table[RADON_TABLE];
-  alignas(16) ss_f32x4 stage[PLANES_CAP + 2];  // chunk window; cells CAP, CAP + 1 stay 0
-};
-
-typedef __attribute__((address_space(3))) const ss_f32x4* ss_lds_cell;
 
 // the sample range of a lane's ray on each plane, in the sample order of plane 0's ray
 struct SSPlaneRanges {
@@ -1014,81 +902,45 @@ __device__ __forceinline__ void ss_planes_item(const SSRadonView& p, const ss_f3
     s_hi = min(ss_rfl(s_hi), row_hi - 1);
     const bool mine = branch == pass;
     const ss_f32x4* lay = pass ? lA : lB;
-    int64_t t0 = s_lo <= s_hi ? a_k + (int64_t)s_lo * beta : 0;
-    for (int sc = s_lo; sc <= s_hi;) {  // block-uniform; super-chunks as in ss_radon_item
-      int rows = PLANES_CHUNK;
-      int nch = min(RADON_TABLE, (s_hi - sc + rows) / rows);
-      const int wmax = ss_radon_windows<false>(lds, 0, sc, rows, nch, s_hi, n);
-      if (wmax * rows > PLANES_CAP) {
-        int r2 = PLANES_CAP / wmax;
-        if (r2 >= RADON_ROW_ROUND) r2 = r2 / RADON_ROW_ROUND * RADON_ROW_ROUND;
-        rows = max(r2, 1);
-        nch = min(RADON_TABLE, (s_hi - sc + rows) / rows);
-        (void)ss_radon_windows<false>(lds, 1, sc, rows, nch, s_hi, n);
-      }
-      const int64_t chunk_step = (int64_t)rows * beta;
-      for (int c = 0; c < nch; ++c) {
-        const int s0 = sc + c * rows, s1 = min(s0 + rows, s_hi + 1);
-        const int2 tw = lds.table[c];
-        const int rec0 = ss_rfl(tw.x), Wc = ss_rfl(tw.y);
-        const bool fits = Wc > 0 && (s1 - s0) * Wc <= PLANES_CAP;  // block-uniform
-        if (c > 0) __syncthreads();  // every wave is done with the previous chunk
+    ss_planes_chunks(lds, lay, pitch, n, s_lo, s_hi, wv, lane, [&](int s0, int s1, int rec0, int Wc, bool fits) {
+      const int ra2 = max(s0, ulo), rb2 = min(s1 - 1, uhi);
+      if (mine && ra2 <= rb2 && Wc > 0) {
+        const int64_t t = a_k + (int64_t)ra2 * beta;
+        float acc[SS_PLANES] = {0.f, 0.f, 0.f, 0.f};  // the chunk's sum
         if (fits) {
-          const ss_f32x4* src0 = lay + (size_t)(s0 + wv) * pitch + rec0 + lane;
-          for (int seg = 0; seg < Wc; seg += SS_WAVE) {
-            if (seg + lane < Wc) {
-              const ss_f32x4* src = src0 + seg;
-              ss_f32x4* dst = lds.stage + wv * Wc + seg;
-              for (int r = wv; r < s1 - s0; r += RADON_WAVES) {
-                __builtin_amdgcn_global_load_lds((ss_global_cptr)src, (ss_lds_ptr)dst, 16, 0, 0);
-                src += (size_t)RADON_WAVES * pitch;
-                dst += RADON_WAVES * Wc;
+          // high word: staged cell index (cell + 1 - rec0) + (row - s0) * Wc
+          int64_t u = t + ((int64_t)(1 - rec0 + (ra2 - s0) * Wc) << 32);
+          int64_t step = beta + ((int64_t)Wc << 32);
+          if (!any) {
+            u = (int64_t)PLANES_CAP << 32;
+            step = 0;
+          }
+          if (own_wave)
+            ss_planes_rows<true>(lds.stage, ra2, rb2 + 1, clo, chi + 1, u, step, rg, acc);
+          else
+            ss_planes_rows<false>(lds.stage, ra2, rb2 + 1, clo, chi + 1, u, step, rg, acc);
+        } else if (any) {  // the window does not fit the LDS: read the layout
+          int64_t u = t + ((int64_t)1 << 32);
+          for (int s = ra2; s <= rb2; ++s, u += beta) {
+            int keep = 0;
+#pragma unroll
+            for (int z = 0; z < SS_PLANES; ++z) keep |= ((unsigned)(s - rg.lo[z]) <= rg.span[z]) << z;
+            if (keep) {
+              const ss_f32x4* cell = lay + (size_t)s * pitch + (int)(u >> 32);
+              const ss_f32x4 a = cell[0], b = cell[1];
+              const float w = (float)(uint32_t)u, w1 = 4294967296.f - w;
+#pragma unroll
+              for (int z = 0; z < SS_PLANES; ++z) {
+                const float v = fmaf(w, b[z], w1 * a[z]);
+                acc[z] += keep >> z & 1 ? v : 0.f;
               }
             }
           }
         }
-        __syncthreads();  // window staged
-        const int ra2 = max(s0, ulo), rb2 = min(s1 - 1, uhi);
-        if (mine && ra2 <= rb2 && Wc > 0) {
-          const int64_t t = t0 + (int64_t)(ra2 - s0) * beta;
-          float acc[SS_PLANES] = {0.f, 0.f, 0.f, 0.f};  // the chunk's sum
-          if (fits) {
-            // high word: staged cell index (cell + 1 - rec0) + (row - s0) * Wc
-            int64_t u = t + ((int64_t)(1 - rec0 + (ra2 - s0) * Wc) << 32);
-            int64_t step = beta + ((int64_t)Wc << 32);
-            if (!any) {
-              u = (int64_t)PLANES_CAP << 32;
-              step = 0;
-            }
-            if (own_wave)
-              ss_planes_rows<true>(lds.stage, ra2, rb2 + 1, clo, chi + 1, u, step, rg, acc);
-            else
-              ss_planes_rows<false>(lds.stage, ra2, rb2 + 1, clo, chi + 1, u, step, rg, acc);
-          } else if (any) {  // the window does not fit the LDS: read the layout
-            int64_t u = t + ((int64_t)1 << 32);
-            for (int s = ra2; s <= rb2; ++s, u += beta) {
-              int keep = 0;
 #pragma unroll
-              for (int z = 0; z < SS_PLANES; ++z) keep |= ((unsigned)(s - rg.lo[z]) <= rg.span[z]) << z;
-              if (keep) {
-                const ss_f32x4* cell = lay + (size_t)s * pitch + (int)(u >> 32);
-                const ss_f32x4 a = cell[0], b = cell[1];
-                const float w = (float)(uint32_t)u, w1 = 4294967296.f - w;
-#pragma unroll
-                for (int z = 0; z < SS_PLANES; ++z) {
-                  const float v = fmaf(w, b[z], w1 * a[z]);
-                  acc[z] += keep >> z & 1 ? v : 0.f;
-                }
-              }
-            }
-          }
-#pragma unroll
-          for (int z = 0; z < SS_PLANES; ++z) tot[z] += acc[z];
-        }
-        t0 += chunk_step;
+        for (int z = 0; z < SS_PLANES; ++z) tot[z] += acc[z];
       }
-      sc += nch * rows;
-    }
+    });
   }
   double ll = 0.0;
   if (on) {
@@ -1116,27 +968,6 @@ __device__ __forceinline__ void ss_planes_item(const SSRadonView& p, const ss_f3
   }
 }
 
-// Order of a planes launch's blocks: consecutive blocks go to the 8 XCDs in turn, each with an
-// L2 of its own.  A unit is a ray group's angle blocks [c yc, (c + 1) yc); the units, from the
-// long rays at the detector's centre to the short ones at its edge, are dealt to the XCDs
-// there and back, so that each XCD gets the same mix and walks one strip of the image with
-// slowly turning angles at a time.
-struct SSPlanesOrder {
-  int g, y;       // ray groups, angle blocks
-  int c, yc;      // units per ray group (g c a multiple of 16), angle blocks per unit
-  int blocks;     // blocks launched; those past a group's angle blocks have no work
-};
-static SSPlanesOrder ss_planes_order(int nrays, int nangles) {
-  SSPlanesOrder o;
-  o.g = (nrays + SS_WAVE - 1) / SS_WAVE;
-  o.y = (nangles + RADON_WAVES - 1) / RADON_WAVES;
-  o.c = 1;
-  while (o.g * o.c % 16) o.c *= 2;
-  o.yc = (o.y + o.c - 1) / o.c;
-  o.blocks = o.g * o.c * o.yc;
-  return o;
-}
-
 // blockIdx.z = group * nslab + z.  The block's rays and angles come from `order`, over plane
 // 0's angles [j0, jd1) and rays [0, nrays); partial sums are laid out over [j0, j1).
 template <int MODE>
@@ -1147,24 +978,20 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE, PLANES_BLOCKS) void k_radon_
   __shared__ SSPlanesLds lds;
   const int z = (int)(blockIdx.z % (unsigned)nslab);
   const int group = (int)(blockIdx.z / (unsigned)nslab);
-  const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
-  const int deal = turn / order.yc;
-  const int unit = deal * 8 + (deal & 1 ? 7 - xcd : xcd);
-  const int grp = order.g - 1 - unit / order.c;
-  const int ablk = unit % order.c * order.yc + turn % order.yc;
+  const int2 at = ss_planes_place(order, blockIdx.x);
+  const int grp = at.x, ablk = at.y;
   const size_t lay = (size_t)group * p.g.n * p.g.pitch;
   const int slice0 = group * ss_planes_slices(kind);
   const size_t per = (size_t)(j1 - j0) * p.g.nrays;
   double* slot = nullptr;
   if (MODE == SS_OUT_EM_RATIO) slot = em.ll_partials + (size_t)group * gridDim.x + blockIdx.x;
-  if (ablk >= order.y) {  // block-uniform
+  if (ablk < 0) {  // block-uniform
     if (MODE == SS_OUT_EM_RATIO && threadIdx.x == 0) *slot = 0.0;
     return;
   }
   float* po = MODE == SS_OUT_PARTIAL ? part + ((size_t)slice0 * nslab + z) * per : nullptr;
   ss_planes_item<MODE>(ss_radon_view(p), lA + lay, lB + lay, kind, slice0, nslices, j0, jd1, j0, j1 - j0, nrays,
-                       grp, ablk,
-                       z * slab_rows, min(p.g.n, (z + 1) * slab_rows), out, em.meas, slot, po,
+                       grp, ablk, z * slab_rows, min(p.g.n, (z + 1) * slab_rows), out, em.meas, slot, po,
                        (size_t)nslab * per, lds);
 }
 
@@ -1311,8 +1138,12 @@ hipError_t ss_launch_gather_planes(const SSDevPlan& p, const float* image, float
   return hipGetLastError();
 }
 
+static SSPlanesOrder ss_planes_order(const SSDevPlan& p, int j0, int j1) {
+  return ss_planes_order(ss_planes_rays(p), ss_planes_j1(p, j1) - j0);
+}
+
 long long ss_planes_blocks(const SSDevPlan& p, int j0, int j1, int nslices) {
-  return (long long)ss_planes_order(ss_planes_rays(p), ss_planes_j1(p, j1) - j0).blocks *
+  return (long long)ss_planes_order(p, j0, j1).blocks *
          ss_planes_groups(p.radon_planes, nslices);
 }
 
@@ -1341,7 +1172,7 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
   dim3 block(RADON_WAVES * SS_WAVE);
   int partial_base;
   const int jd1 = ss_planes_j1(p, j1), half = ss_planes_rays(p);
-  const SSPlanesOrder order = ss_planes_order(half, jd1 - j0);
+  const SSPlanesOrder order = ss_planes_order(p, j0, j1);
   if (p.radon_planes) grid = dim3(order.blocks, 1, ss_planes_groups(p.radon_planes, nslices) * nslab);
   // the main pass in the plan's form: planes, or block shape 0 or 1
 #define SS_RADON_LAUNCH(MODE, OUTP, PARTP, NSLAB, ROWS, EM)                                                        \

@@ -1,6 +1,7 @@
 """Symmetric geometries, where one ray coordinate serves several pixels or rays: against the
 FP64 oracle at the edges of the form (odd and even sides, bins and angles, tiles and
 windows that end inside the image, the grids that only one of the symmetries fits)."""
+import ctypes
 import math
 
 import numpy as np
@@ -120,3 +121,63 @@ def test_transpose_planes(n, R, A, sc):
             assert _rel(p.radon_transpose(ys[idx], angles=(j0, j1)).cpu().numpy(), pown) <= REL, s
     v, times = p.tune_transpose(1, reps=1, force=True)
     assert v == -1 or _rel(p.radon_transpose(ys[0]).cpu().numpy(), ref[0]) <= REL
+
+
+# (image shape, R, A, image corners, sinogram corners, slices): both symmetries, the half turn
+# alone, none (stacks of slices; one or two slices take the one-ray kernels), rectangular
+# images, detectors narrower and wider than the image
+IC = (-1.0, 1.0, 1.0, -1.0)
+LINE_GEO = [
+    ((2, 2), 2, 2, IC, (0.0, 1.0, PI, -1.0), 1), ((5, 5), 7, 4, IC, (0.0, 1.0, PI, -1.0), 3),
+    ((31, 31), 33, 9, IC, (0.0, 1.0, PI, -1.0), 1), ((32, 32), 64, 17, IC, (0.0, 1.0, PI, -1.0), 2),
+    ((33, 33), 31, 16, IC, (0.0, 1.0, PI, -1.0), 1), ((64, 64), 63, 65, IC, (0.0, 0.7, PI, -0.7), 5),
+    ((65, 65), 80, 40, IC, (0.0, 1.42, PI, -1.42), 1), ((97, 97), 97, 129, IC, (0.0, 1.0, PI, -1.0), 1),
+    ((130, 130), 131, 48, IC, (0.0, 1.0, PI, -1.0), 1), ((66, 66), 90, 35, IC, (0.1, 1.0, 2.9, -1.0), 4),
+    ((67, 67), 65, 33, IC, (0.0, 1.0, PI / 2 - 0.1, -1.0), 2), ((67, 67), 65, 33, IC, (0.0, 1.0, PI / 2 - 0.1, -1.0), 1),
+    ((64, 64), 64, 30, IC, (0.0, 1.03, PI, -0.97), 6), ((65, 65), 65, 30, IC, (0.0, 1.03, PI, -0.97), 3),
+    ((64, 64), 70, 30, IC, (0.0, 1.03, PI, -0.97), 1), ((41, 81), 90, 50, (-1.0, 0.5, 1.0, -0.5), (0.0, 1.1, PI, -1.1), 3),
+    ((96, 50), 100, 41, (-0.49, 0.95, 0.49, -0.95), (0.0, 1.1, PI, -1.1), 1), ((160, 160), 41, 37, IC, (0.0, 0.2, PI, -0.2), 1),
+]
+
+
+def _line_matrix(shape, R, A, ic, sc):
+    """(ray, pixel, length) of the line traversal as the plan defines it, traced on the host"""
+    from pyraft_amd.raftypes import libraft
+    d4 = ctypes.c_double * 4
+    cap = 2 * sum(shape) + 8
+    ij, ln = np.zeros((cap, 2), np.int32), np.zeros(cap)
+    ray, pix, val = [], [], []
+    for a in range(A):
+        for r in range(R):
+            k = libraft.raft_dda_host_ray(shape[0], shape[1], R, A, d4(*ic), d4(*sc), a, r,
+                                          ij.ctypes.data_as(ctypes.POINTER(ctypes.c_int)),
+                                          ln.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), cap)
+            assert 0 <= k <= cap
+            ray.append(np.full(k, r * A + a))
+            pix.append(ij[:k, 0] * shape[1] + ij[:k, 1])
+            val.append(ln[:k].copy())
+    return np.concatenate(ray), np.concatenate(pix), np.concatenate(val)
+
+
+@pytest.mark.parametrize("shape,R,A,ic,sc,S", LINE_GEO)
+def test_line_planes(shape, R, A, ic, sc, S):
+    import torch
+    from pyraft_amd.device import DdaPlan
+    print("line", shape, R, A, sc, S, flush=True)
+    ray, pix, val = _line_matrix(shape, R, A, ic, sc)
+    rng = np.random.default_rng(R + A)
+    s = rng.random((S, R, A)).astype(np.float32)
+    p = DdaPlan(shape, R, A, ic, sc)
+    x = torch.from_numpy(s).cuda()
+    t, b = p.radon_transpose(x).cpu().numpy(), p.backprojection(x).cpu().numpy()
+    npix = shape[0] * shape[1]
+    f = rng.random((S,) + shape).astype(np.float32)
+    g = p.radon(torch.from_numpy(f).cuda()).cpu().numpy()
+    for i in range(S):
+        assert _rel(g[i].ravel(), np.bincount(ray, val * f[i].ravel().astype(np.float64)[pix], R * A)) <= REL
+    w = np.bincount(pix, val, npix).reshape(shape)
+    ok = w > 1e-6 * w.max()
+    for i in range(S):
+        ref = np.bincount(pix, val * s[i].ravel().astype(np.float64)[ray], npix).reshape(shape)
+        assert _rel(t[i], ref) <= REL
+        assert _rel(b[i][ok], ref[ok] / w[ok]) <= REL
