@@ -821,7 +821,7 @@ int ss_em_prepare(const raft_ss_plan* p, int nsubsets, int nslices, int niter, h
   L->rho_off = off;
   off += sizeof(float) * sino_sz;
   L->weights_off = off;
-  off += sizeof(float) * (size_t)nsubsets * img_sz;
+  off += sizeof(float) * (size_t)nsubsets * n * n;
   off = (off + 7) & ~(size_t)7;
   L->partials_off = off;
   off += sizeof(double) * (size_t)L->poff[nsubsets];
@@ -855,14 +855,7 @@ int ss_em_launch(const raft_ss_plan* p, const SSEmLaunch& L, const float* d_sino
   if (!d_ll) d_ll = reinterpret_cast<double*>(base + L.ll_off);
 
   HIP_TRY(ss_launch_sino_to_t(d_sino, measT, R, A, nslices, stream));
-  // W_b = BP_b(1) with the same backprojection kernel
-  HIP_TRY(ss_launch_fill(rhoT, 1.0f, sino_sz, stream));
-  SSEmUpdateArgs none{nullptr, nullptr};
-  for (int b = 0; b < S; ++b) {
-    const int j0 = (int)(((long long)b * A) / S), j1 = (int)(((long long)(b + 1) * A) / S);
-    HIP_TRY(ss_launch_backprojection(L.dpb, rhoT, j0, j1, nslices, SS_BP_PLAIN, weights + (size_t)b * img_sz, none,
-                                     bp_part, stream));
-  }
+  HIP_TRY(ss_launch_bp_weights(L.dp, S, weights, stream));
   for (int it = 0; it < niter; ++it) {
     for (int b = 0; b < S; ++b) {
       const int j0 = (int)(((long long)b * A) / S), j1 = (int)(((long long)(b + 1) * A) / S);
@@ -872,7 +865,7 @@ int ss_em_launch(const raft_ss_plan* p, const SSEmLaunch& L, const float* d_sino
       HIP_TRY(ss_launch_gather_layouts(L.dps[b], d_x, gA, gB, nslices, stream, need));
       SSEmRatioArgs ea{measT, partials + L.poff[b]};
       HIP_TRY(ss_launch_radon(L.dps[b], gA, gB, j0, j1, nslices, SS_OUT_EM_RATIO, rhoT, ea, slabs, stream));
-      SSEmUpdateArgs ua{d_x, weights + (size_t)b * img_sz};
+      SSEmUpdateArgs ua{d_x, weights + (size_t)b * n * n};
       HIP_TRY(ss_launch_backprojection(L.dpb, rhoT, j0, j1, nslices, SS_BP_EM_UPDATE, nullptr, ua, bp_part, stream));
     }
     HIP_TRY(ss_launch_sum_partials(partials, npartials, d_ll + it, stream));

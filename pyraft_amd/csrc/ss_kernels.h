@@ -154,8 +154,10 @@ int ss_radon_partials(const SSDevPlan& p, int j0, int j1, int nslices);
 // ---- backprojection (reads angle-major sinogram)
 struct SSEmUpdateArgs {
   float* x;            // image updated in place
-  const float* weight; // BP_b(1)
+  const float* weight; // BP_b(1), one image for all slices
 };
+// W_b = BP_b(1) of `nsubsets` subsets to out[b][n][n]
+hipError_t ss_launch_bp_weights(const SSDevPlan& p, int nsubsets, float* out, hipStream_t stream);
 // A launch may divide its angles into groups taken by separate blocks, at least
 // SS_BP_GROUP_ANGLES angles each; every group writes a partial image (unscaled sums) to
 // scratch and a finishing pass adds the groups in group order, scales by dtheta and stores
@@ -167,7 +169,8 @@ struct SSEmUpdateArgs {
 // launches (us with 1 / 4 / 8 / 16 / 32 groups, variant 0): 2048^2 x 1500 680 / 621 / 596 /
 // 630 / 734; 1448^2 x 720 288 / 195 / 179 / 184 / 251; 1024^2 x 720 285 / 145 / 104 / 102 /
 // 120; 768^2 x 500 203 / 105 / 65 / 57 / 66; 512^2 x 720 312 / 143 / 79 / 54 / 48; the rule
-// takes 8, 8, 12, 13, 24.
+// takes 8, 8, 12, 13, 24.  Below 2 the launch is not divided (94 angles of a 2048^2 image, G = 1.5:
+// 50 us undivided, 64 in two groups).
 // ss_bp_groups: the group count (1: no division); ss_bp_scratch: the bytes of the partial
 // images (0 when not divided).
 #define SS_BP_GROUP_SCALE 0.22

@@ -1262,15 +1262,47 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
 #define BP_TILE_W 32
 
 struct alignas(16) BPAngle {
-  float f0, b, c;  // read together with flag by one 16-byte LDS read
+  float f0, b, c;  // read together by one 16-byte LDS read
   int flag;        // 0 outside, 1 interior, 2 boundary
   int base;
-  int pad0, pad1, pad2;
+  float lo, hi;    // u of the pixels that are on the detector for certain
+  int pad;
 };
 
 __device__ __forceinline__ int ss_bp_exact_valid(const SSDevPlan& p, int j, int row, int col) {
   const SSAngle& a = p.angles[j];
   return ss_bp_sample_valid(p.g, a.cost, a.sint, row, col) ? 1 : 0;
+}
+
+// Pixels this near (in rays) to the first or last ray take the exact test: a tile's pixels have
+// u < W rays from its base, and its FP32 evaluation (the rounded origin, slopes times up to 63
+// pixels, two fused steps) is within W 2^-22 of the FP64 coordinate; four times that.  (At
+// 1e-3 for every tile one wave in ten took the test and waited for its loads.)
+__device__ __forceinline__ float ss_bp_edge(int W) { return (float)W * 9.5367431640625e-7f; }
+
+// Angle j on the tile [c0, c0 + 32) x [r0, r0 + th): its origin's ray coordinate from the base
+// ray, the slopes, and whether the tile lies on the detector
+__device__ __forceinline__ BPAngle ss_bp_params(const SSDevPlan& p, int j, int c0, int r0, int th) {
+  BPAngle q{0.f, 0.f, 0.f, 0, 0, 0.f, 0.f, 0};
+  const int R = p.g.nrays;
+  const SSAngle& a = p.angles[j];
+  const double U = a.bp_a + (double)c0 * a.bp_b + (double)r0 * a.bp_c;
+  const double ec = (double)(BP_TILE_W - 1) * a.bp_b, er = (double)(th - 1) * a.bp_c;
+  const double umin = U + fmin(0.0, ec) + fmin(0.0, er);
+  const double umax = U + fmax(0.0, ec) + fmax(0.0, er);
+  const double base = floor(umin) - 1.0;
+  q.f0 = (float)(U - base);
+  q.b = (float)a.bp_b;
+  q.c = (float)a.bp_c;
+  const double eps = 1e-6;
+  if (umax < -eps || umin >= (double)(R - 1) + eps)
+    q.flag = 0;
+  else if (umin >= eps && umax < (double)(R - 1) - eps)
+    q.flag = 1;
+  else
+    q.flag = 2;
+  q.base = (int)base;
+  return q;
 }
 
 template <int STAGE>
@@ -1404,6 +1436,9 @@ __device__ __forceinline__ bool ss_bp_plane_pixel(int z, int n, int row, int col
 //           pi - theta, pixel (r, n-1-c) has pixel (r, c)'s coordinate, and (n-1-r, c) its
 //           reverse; a window also holds the rows of that angle.  Tiles cover a quadrant.
 // Each pixel's range test is its own (a mirrored pixel re-evaluates its own FP64 expression).
+// The tiles that some angles end in set a short launch's time: 45 angles of a 1024^2 image 21 us
+// with a branch on each angle's flag and a test per pixel, 15 in the form below, 10 where no
+// angle ends in the image; 720 angles 97 / 95, 2048^2 x 1500 587 / 570.
 // VALU instructions per update in the loop: 5 / 3.5 / 2.75.
 template <int MODE, int ROWS, int STAGE, int PL>
 __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __restrict__ sl, int j0, int j1, int c0,
@@ -1427,7 +1462,7 @@ __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __re
     fty[i] = (float)(ty + 8 * i);
   }
   const float ftx = (float)tx;
-  const float lo_rel_eps = 1e-3f;
+  const float edge = ss_bp_edge(W);
 
   // Parameters of up to 64 angles at a time: lane l of every wave holds those of angle
   // ja + l, for as many whole stages as fit (in FP64: redone per stage they were 7% of the
@@ -1435,28 +1470,11 @@ __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __re
   const int JP = SS_WAVE / J * J;
   for (int ja = j0; ja < j1; ja += JP) {
     const int np = min(JP, j1 - ja);
-    BPAngle q{0.f, 0.f, 0.f, 0, 0, 0, 0, 0};
-    if (lane < np) {
-      const SSAngle& a = p.angles[ja + lane];
-      const double U = a.bp_a + (double)c0 * a.bp_b + (double)r0 * a.bp_c;
-      const double ec = (double)(BP_TILE_W - 1) * a.bp_b, er = (double)(TH - 1) * a.bp_c;
-      const double umin = U + fmin(0.0, ec) + fmin(0.0, er);
-      const double umax = U + fmax(0.0, ec) + fmax(0.0, er);
-      const double base = floor(umin) - 1.0;
-      q.f0 = (float)(U - base);
-      q.b = (float)a.bp_b;
-      q.c = (float)a.bp_c;
-      const double eps = 1e-6;
-      if (umax < -eps || umin >= (double)(R - 1) + eps)
-        q.flag = 0;
-      else if (umin >= eps && umax < (double)(R - 1) - eps)
-        q.flag = 1;
-      else
-        q.flag = 2;
-      q.base = (int)base;
-    }
+    BPAngle q{0.f, 0.f, 0.f, 0, 0, 0.f, 0.f, 0};
+    if (lane < np) q = ss_bp_params(p, ja + lane, c0, r0, TH);
     // the angles that are interior for this tile run without predicates
     const unsigned long long interior = __ballot(lane < np && q.flag == 1);
+    const unsigned long long ending = __ballot(lane < np && q.flag == 2);
     for (int js = 0; js < np; js += J) {
       const int jb = ja + js, nj = min(J, np - js);
       const bool mixed = __popcll(interior >> js & (~0ull >> (SS_WAVE - nj))) != nj;
@@ -1465,8 +1483,8 @@ __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __re
         lds.par[lane].f0 = q.f0;
         lds.par[lane].b = q.b;
         lds.par[lane].c = q.c;
-        lds.par[lane].flag = q.flag;
-        lds.par[lane].base = q.base;
+        lds.par[lane].lo = (float)(-q.base) + edge;
+        lds.par[lane].hi = (float)(R - 1 - q.base) - edge;
       }
       // base is at least one ray below the tile's lowest U, so every pixel has u >= 1 and
       // (int)u < W - 1
@@ -1487,46 +1505,70 @@ __device__ __forceinline__ void ss_bp_item(const SSDevPlan& p, const float* __re
       if (!mixed) {
 #pragma unroll 2
         for (int jj = 0; jj < nj; ++jj)
-          add(*reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]), lds.win + jj * RW * W);  // f0, b, c, flag
+          add(*reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]), lds.win + jj * RW * W);  // f0, b, c
       } else {
-        for (int jj = 0; jj < nj; ++jj) {
-          const ss_f32x4 par = *reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]);
-          const float2* wrow = lds.win + jj * RW * W;
-          const int flag = __builtin_amdgcn_readfirstlane(__float_as_int(par.w));
-          if (flag == 0) continue;
-          if (flag == 1) {
-            add(par, wrow);
-            continue;
+        // Some angles end in this tile or miss it.  By the scalar masks (a flag read per angle put
+        // two LDS latencies in a row before its updates): first the interior ones, then those that
+        // end here with per-pixel 0 <= m <= R-2 tests; two angles at a time.  Pixels within `edge`
+        // rays of an end are left out and take the reference's FP64 expression afterwards; most
+        // stages have none.
+        const unsigned long long mask = ~0ull >> (SS_WAVE - nj);
+        auto two = [&](unsigned long long m, auto&& one) {
+          while (m) {
+            const int j1 = __builtin_ctzll(m);
+            m &= m - 1;
+            if (m) {
+              const int j2 = __builtin_ctzll(m);
+              m &= m - 1;
+              one(j1);
+              one(j2);
+            } else {
+              one(j1);
+            }
           }
-          // boundary tile: per-pixel 0 <= m <= R-2 test; pixels within 1e-3 bins of an edge
-          // take the reference's FP64 expression.  The result is an integer mask applied by
-          // select, keeping the divergent region free of value phis.
-          const int base = lds.par[js + jj].base;
+        };
+        two(interior >> js & mask, [&](int jj) {
+          add(*reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]), lds.win + jj * RW * W);
+        });
+        bool near = false;
+        const unsigned long long ends = ending >> js & mask;
+        two(ends, [&](int jj) {
+          const ss_f32x4 par = *reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]);
+          const float lo = lds.par[js + jj].lo, hi = lds.par[js + jj].hi;
           const float t0 = fmaf(ftx, par.y, par.x);
-          const float lo_rel = (float)(-base), hi_rel = (float)(R - 1 - base);
-          int keep = 0;
 #pragma unroll
           for (int i = 0; i < ROWS; ++i) {
             const float u = fmaf(fty[i], par.z, t0);
-            const bool inside = (u > lo_rel + lo_rel_eps) && (u < hi_rel - lo_rel_eps);
-            const bool outside = (u < lo_rel - lo_rel_eps) || (u > hi_rel + lo_rel_eps);
-            int ok = inside ? (1 << PL) - 1 : 0;
-            if (!inside && !outside) {
-              const int jm = PL == 4 ? ss_bp_mirror(jb + jj, A).row : jb + jj;
+            const bool in = __builtin_amdgcn_fmed3f(u, lo, hi) == u;
+            near = near || (!in && __builtin_amdgcn_fmed3f(u, lo - 2.f * edge, hi + 2.f * edge) == u);
+            float val[PL];
+            ss_bp_lerp<PL, STAGE>(lds.win + jj * RW * W, u, val);
+#pragma unroll
+            for (int z = 0; z < PL; ++z) acc[i][z] += in ? val[z] : 0.f;
+          }
+        });
+        if (__ballot(near) != 0ull) {
+          for (unsigned long long m = ends; m; m &= m - 1) {
+            const int jj = __builtin_ctzll(m);
+            const ss_f32x4 par = *reinterpret_cast<const ss_f32x4*>(&lds.par[js + jj]);
+            const float lo = lds.par[js + jj].lo, hi = lds.par[js + jj].hi;
+            const float t0 = fmaf(ftx, par.y, par.x);
+            const int jm = PL == 4 ? ss_bp_mirror(jb + jj, A).row : jb + jj;
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i) {
+              const float u = fmaf(fty[i], par.z, t0);
+              if (__builtin_amdgcn_fmed3f(u, lo, hi) == u ||
+                  __builtin_amdgcn_fmed3f(u, lo - 2.f * edge, hi + 2.f * edge) != u)
+                continue;
+              float val[PL];
+              ss_bp_lerp<PL, STAGE>(lds.win + jj * RW * W, u, val);
+#pragma unroll
               for (int z = 0; z < PL; ++z) {
                 int zr, zc;
                 (void)ss_bp_plane_pixel<PL>(z, n, r0 + ty + 8 * i, col, &zr, &zc);
-                ok |= ss_bp_exact_valid(p, z >= 2 ? jm : jb + jj, zr, zc) << z;
+                acc[i][z] += ss_bp_exact_valid(p, z >= 2 ? jm : jb + jj, zr, zc) ? val[z] : 0.f;
               }
             }
-            keep |= ok << (PL * i);
-          }
-#pragma unroll
-          for (int i = 0; i < ROWS; ++i) {
-            float val[PL];
-            ss_bp_lerp<PL, STAGE>(wrow, fmaf(fty[i], par.z, t0), val);
-#pragma unroll
-            for (int z = 0; z < PL; ++z) acc[i][z] += ((keep >> (PL * i + z)) & 1) ? val[z] : 0.f;
           }
         }
       }
@@ -1575,7 +1617,84 @@ __global__ __launch_bounds__(256) void k_backprojection(SSDevPlan p, const float
   float* dst = MODE == SS_BP_PLAIN ? out + io : (MODE == SS_BP_PARTIAL ? out + (slice * ngroups + g) * per : nullptr);
   ss_bp_item<MODE, ROWS, STAGE, PL>(p, sinoT + so, ja, jb, blockIdx.x * BP_TILE_W, blockIdx.y * 8 * ROWS, dst,
                                 MODE == SS_BP_EM_UPDATE ? em.x + io : nullptr,
-                                MODE == SS_BP_EM_UPDATE ? em.weight + io : nullptr, lds);
+                                MODE == SS_BP_EM_UPDATE ? em.weight : nullptr, lds);
+}
+
+// The OSEM weights W_b = BP_b(1) of the subsets [b A / S, (b + 1) A / S), to out[b][n][n]: between
+// two rays the backprojection of ones adds 1, so a pixel's sum is the count of the subset's
+// angles whose ray coordinate lies on the detector, by the test of ss_bp_item.  A block takes
+// a 32 x 32 pixel tile (and subset b0 + blockIdx.z), a wave's lanes the flags of 64 angles at a
+// time: angles interior to the tile add to all its pixels at once, only those that end in it are
+// tested per pixel.  1024^2, 16 subsets of 45 angles: 365 us as 16 backprojections, 47 here (the
+// angles' FP64 terms and one wait for their loads per block).  SPLIT: launches of few tiles walk
+// their angles too long (226^2, one subset of 449, an iteration: 117 us, split 84), so a block takes 32 x 8
+// pixels, each of its waves all of them for a quarter of the angles.
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void k_bp_weights(SSDevPlan p, int S, int b0, float* __restrict__ out) {
+  const int n = p.g.n, R = p.g.nrays, A = p.g.nangles, b = b0 + blockIdx.z;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  constexpr int TH = SPLIT ? 8 : 32, STEP = SPLIT ? 2 : 8;  // tile rows, rows between a thread's pixels
+  const int tx = threadIdx.x & 31, ty = (SPLIT ? lane : (int)threadIdx.x) >> 5;
+  const int c0 = blockIdx.x * BP_TILE_W, r0 = blockIdx.y * TH;
+  const int col = c0 + tx;
+  int j0 = (int)((long long)b * A / S), j1 = (int)((long long)(b + 1) * A / S);
+  if (SPLIT) {
+    const int nj = j1 - j0;
+    j1 = j0 + (int)((wv + 1LL) * nj / 4);
+    j0 += (int)((long long)wv * nj / 4);
+  }
+  const float edge = ss_bp_edge(2 * p.bp_window);  // these tiles may be twice the plan's
+  int all = 0, count[4] = {0, 0, 0, 0};
+  for (int ja = j0; ja < j1; ja += SS_WAVE) {
+    const int np = min(SS_WAVE, j1 - ja);
+    const BPAngle q = lane < np ? ss_bp_params(p, ja + lane, c0, r0, TH) : BPAngle{0.f, 0.f, 0.f, 0, 0, 0.f, 0.f, 0};
+    all += __popcll(__ballot(q.flag == 1));
+    for (unsigned long long mixed = __ballot(q.flag == 2); mixed; mixed &= mixed - 1) {
+      const int jj = __builtin_ctzll(mixed);
+      const float f0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.f0), jj));
+      const float pb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.b), jj));
+      const float pc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.c), jj));
+      const int base = __builtin_amdgcn_readlane(q.base, jj);
+      const float t0 = fmaf((float)tx, pb, f0), lo = (float)(-base), hi = (float)(R - 1 - base);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float u = fmaf((float)(ty + STEP * i), pc, t0);
+        if (u > lo + edge && u < hi - edge)
+          ++count[i];
+        else if (!(u < lo - edge || u > hi + edge))
+          count[i] += ss_bp_exact_valid(p, ja + jj, r0 + ty + STEP * i, col);
+      }
+    }
+  }
+  const float dth = (float)p.g.dth;
+  if constexpr (SPLIT) {
+    __shared__ int part[4][TH * 32];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[wv][(ty + STEP * i) * 32 + tx] = all + count[i];
+    __syncthreads();
+    const int t = threadIdx.x, row = r0 + (t >> 5);
+    const int sum = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+    if (row < n && col < n) out[((size_t)b * n + row) * n + col] = (float)sum * dth;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = r0 + ty + STEP * i;
+      if (row < n && col < n) out[((size_t)b * n + row) * n + col] = (float)(all + count[i]) * dth;
+    }
+  }
+}
+
+hipError_t ss_launch_bp_weights(const SSDevPlan& p, int nsubsets, float* out, hipStream_t stream) {
+  const int t = (p.g.n + 31) / 32;
+  const bool split = (long long)t * t * nsubsets <= SS_BP_ROUND_BLOCKS;
+  for (int b0 = 0; b0 < nsubsets; b0 += 65535) {  // grid dimension limit
+    const dim3 grid(t, split ? (p.g.n + 7) / 8 : t, std::min(nsubsets - b0, 65535));
+    if (split)
+      hipLaunchKernelGGL(k_bp_weights<true>, grid, dim3(256), 0, stream, p, nsubsets, b0, out);
+    else
+      hipLaunchKernelGGL(k_bp_weights<false>, grid, dim3(256), 0, stream, p, nsubsets, b0, out);
+  }
+  return hipGetLastError();
 }
 
 // the groups' partial sums of each pixel added in group order, times dtheta, stored
@@ -1596,7 +1715,7 @@ __global__ __launch_bounds__(256) void k_bp_groups_finish(const float* __restric
   if (MODE == SS_BP_PLAIN) {
     out[o] = bp;
   } else {
-    const float wgt = em.weight[o];
+    const float wgt = em.weight[idx];
     const float x = em.x[o];
     em.x[o] = wgt > 0.f ? x * bp / wgt : x;
   }
@@ -1622,7 +1741,8 @@ int ss_bp_tiles(int n, int variant, int planes) {
 static int ss_angle_groups(long long tiles, int nj) {
   if (tiles <= 0 || nj < 2 * SS_BP_GROUP_ANGLES) return 1;
   const double g = SS_BP_GROUP_SCALE * sqrt((double)SS_BP_ROUND_BLOCKS * nj / (double)tiles);
-  return (int)std::max(1.0, std::min(floor(g + 0.5), (double)(nj / SS_BP_GROUP_ANGLES)));
+  if (g < 2.0) return 1;  // two groups cost more than they even out (SS_BP_GROUP_SCALE)
+  return (int)std::min(floor(g + 0.5), (double)(nj / SS_BP_GROUP_ANGLES));
 }
 
 int ss_bp_groups(const SSDevPlan& p, int j0, int j1, int nslices) {

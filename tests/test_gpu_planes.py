@@ -181,3 +181,30 @@ def test_line_planes(shape, R, A, ic, sc, S):
         ref = np.bincount(pix, val * s[i].ravel().astype(np.float64)[ray], npix).reshape(shape)
         assert _rel(t[i], ref) <= REL
         assert _rel(b[i][ok], ref[ok] / w[ok]) <= REL
+
+
+@pytest.mark.parametrize("n,R,A,sc,S", [(2, 3, 1, (0.0, 1.0, PI, -1.0), 1), (31, 33, 7, (0.0, 1.0, PI, -1.0), 3),
+                                        (33, 31, 70, (0.0, 1.0, 2 * PI, -1.0), 1), (64, 65, 150, (0.0, 0.6, PI, -0.6), 2),
+                                        (65, 64, 24, (0.0, 1.03, PI, -0.97), 24), (97, 150, 66, (0.0, 1.42, 2.0, -1.42), 5)])
+def test_osem_weights(n, R, A, sc, S):
+    """One pass of the subsets: the update by the weights against the same steps made with the
+    projectors, two slices."""
+    import torch
+    from pyraft_amd.device import Plan
+    print("osem weights", n, R, A, sc, S, flush=True)
+    rng = np.random.default_rng(n + R + A)
+    y = torch.from_numpy((5 + rng.random((2, R, A))).astype(np.float32)).cuda()
+    p = Plan(n, R, A, sino_corners=sc)
+    got = p.em(y, 1, S).cpu().numpy()
+    x = np.ones((2, n, n))
+    for b in range(S):
+        j0, j1 = b * A // S, (b + 1) * A // S
+        on = np.zeros((R, A))
+        on[:, j0:j1] = 1.0
+        w = O.backprojection(on, n, **_geo(sc))
+        for i in range(2):
+            f = O.radon(x[i], R, A, **_geo(sc))
+            rho = np.where((f > 0) & (on > 0), y[i].cpu().numpy() / np.where(f > 0, f, 1.0), 0.0)
+            bp = O.backprojection(rho, n, **_geo(sc))
+            x[i] = np.where(w > 0, x[i] * bp / np.where(w > 0, w, 1.0), x[i])
+    assert _rel(got, x) <= REL
