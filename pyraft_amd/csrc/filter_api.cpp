@@ -34,15 +34,14 @@ std::vector<double> ramp_bins(int R, double cutoff, double dt) {
 void toeplitz_taps(int R, double cutoff, double dt, float* taps) {
   const int Z = 2 * R - 1;
   const std::vector<double> ramp = ramp_bins(R, cutoff, dt);
-  std::vector<double> H(R), ct(Z);
-  for (int k = 0; k < R; ++k) H[k] = k < (int)ramp.size() ? ramp[k] / Z : 1.0;
+  std::vector<double> H(R), ct(Z), K(R);
+  for (int k = 0; k < R; ++k) H[k] = (k > 0 ? 2.0 : 1.0) * (k < (int)ramp.size() ? ramp[k] / Z : 1.0);
   for (int j = 0; j < Z; ++j) ct[j] = cos(2.0 * M_PI * (double)j / Z);
+  ss_cosine_sums(H.data(), R, ct.data(), Z, K.data(), R);
   taps[0] = 0.f;
   for (int d = 0; d < R; ++d) {
-    double acc = H[0];
-    for (int k = 1; k < R; ++k) acc += 2.0 * H[k] * ct[((long long)k * d) % Z];
-    taps[R + d] = (float)acc;  // K is even in d
-    taps[R - d] = (float)acc;
+    taps[R + d] = (float)K[d];  // K is even in d
+    taps[R - d] = (float)K[d];
   }
 }
 

@@ -153,6 +153,8 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 void ss_report_legacy(const char* fn, int rc);
 
 // FP32 circular-convolution kernel of the numpy FBP filters (kind RAFT_SS_FILTER_*)
+// out[m] = a[0] + sum over 0 < f < n of a[f] ct[(f m) mod Z], in the order of f, for m < count
+void ss_cosine_sums(const double* a, int n, const double* ct, int Z, double* out, int count);
 void ss_filter_kernel(int R, double tmin, double tmax, int kind, double param, float* g);
 
 // ------------------------------------------------------------------ host <-> raft_image staging

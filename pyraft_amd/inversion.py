@@ -52,7 +52,7 @@ def fbp_gpu(*args):
     img_size = int(args[1]) if len(args) > 1 else rays
     sc = _corners(s)
     plan = Plan(img_size, rays, angles)
-    rows = _to_device(numpy.asarray(s, dtype=numpy.float32).T)
+    rows = _to_device(s).t().contiguous()  # transposed on the device: strided host copies are slow
     g = torch.from_numpy(ramp_kernel(rays, sc[3], sc[1])).cuda()
     filt = filter_rows(rows, g)
     return plan.backprojection(filt, angle_major=True).cpu().numpy()
