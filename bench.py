@@ -111,8 +111,8 @@ def roofline_of(kernel, updates, seconds, traffic, traffic_src, counters=None):
 
 def _profile_name_matches(key, kernel):
     """A profile key ("name/work-items") names `kernel`; a kernel given without its last
-    template arguments ("k_radon<1>") matches every instantiation that extends it
-    ("k_radon<1, 1>": the Radon's block shape is picked per launch)."""
+    template arguments ("k_backprojection<0, 4, 2048>") matches every instantiation that
+    extends it ("k_backprojection<0, 4, 2048, 4>": the planes are picked per launch)."""
     name = key.split("/")[0]
     return name == kernel or (kernel.endswith(">") and name.startswith(kernel[:-1] + ", "))
 
@@ -779,7 +779,7 @@ def main():
     torch.cuda.synchronize()
     transpose_ms = e0.elapsed_time(e1) / 3
 
-    dominant = ("k_backprojection<0, %d, %d>" % (bp_rows, bp_stage)) if t_bp >= t_radon else "k_radon<1>"
+    dominant = ("k_backprojection<0, %d, %d>" % (bp_rows, bp_stage)) if t_bp >= t_radon else "k_radon_planes<1>"
     t_dom = max(t_bp, t_radon)
     traffic, traffic_src = measured_traffic(dominant)
     roofline = roofline_of(dominant, upd, t_dom, traffic, traffic_src, measured_counters(dominant))

@@ -14,9 +14,10 @@ extern "C" {
 #endif
 #pragma GCC visibility push(default)
 
-/* Bytes of the library's static device scratch array: two gather layouts of one
- * 2048 x 2048 slice (2 * 2048 * 2064 * 8 bytes) plus the row-slab partial sums of a
- * divided launch.  Every GPU the library is loaded on holds this array until the
+/* The workspace limit: two gather layouts of one 2048 x 2048 slice (2 * 2048 * 2064 * 8
+ * bytes) plus the row-slab partial sums of a divided launch, in the form with one ray per
+ * lane.  The library's static device scratch array is twice as large (the form with four
+ * rays per lane keeps 16-byte cells); every GPU the library is loaded on holds it until the
  * process ends. */
 #define RAFT_SS_NOALLOC_SCRATCH_BYTES (72u * 1024u * 1024u)
 

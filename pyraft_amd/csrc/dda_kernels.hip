@@ -1253,6 +1253,14 @@ static dim3 dda_tiles(int lines, int cols, int nslices) {
   return dim3((cols + DDA_TILE - 1) / DDA_TILE, (lines + DDA_TILE - 1) / DDA_TILE, nslices);
 }
 
+// The planes a launch takes
+static int dda_planes_kind(const SSDdaTransposePlan& tp, int nslices) {
+  if (ss_planes_stack(nslices)) return SS_PLANES_SLICES;
+  if (tp.sym & DDA_SYM_MIRROR) return SS_PLANES_QUAD;
+  if ((tp.sym & DDA_SYM_TURN) && nslices >= 2) return SS_PLANES_PAIR;
+  return nslices >= 3 ? SS_PLANES_SLICES : SS_PLANES_NONE;
+}
+
 static SSDdaRadonPlanes dda_radon_planes(const SSDdaGeom& g, const SSDdaTransposePlan& tp, int kind, int nslices) {
   SSDdaRadonPlanes rp;
   rp.kind = kind;
@@ -1284,13 +1292,7 @@ SSDdaRadonForm dda_radon_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, 
   if (tp.ngather == 0) return f;
   // a traced ray's pixel offsets are ints
   if ((long long)std::max(g.lines, g.cols) * (std::max(g.lines, g.cols) + 2 * DDA_RP_PAD) >= (1LL << 31)) return f;
-  int kind = SS_PLANES_NONE;
-  if (tp.sym & DDA_SYM_MIRROR)
-    kind = SS_PLANES_QUAD;
-  else if ((tp.sym & DDA_SYM_TURN) && nslices >= 2)
-    kind = SS_PLANES_PAIR;
-  else if (nslices >= 3)
-    kind = SS_PLANES_SLICES;
+  const int kind = dda_planes_kind(tp, nslices);
   if (kind == SS_PLANES_NONE) return f;
   const int groups = ss_planes_groups(kind, nslices);
   const SSDdaRadonPlanes rp = dda_radon_planes(g, tp, kind, nslices);
@@ -1345,12 +1347,7 @@ static int dda_gp_rows(const SSDdaGeom& g, int kind) {
 SSDdaGatherForm dda_gather_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, bool ones, int nslices) {
   SSDdaGatherForm f{SS_PLANES_NONE, 1};
   if (ones || tp.ngather == 0 || tp.planes_ws <= 0) return f;
-  if (tp.sym & DDA_SYM_MIRROR)
-    f.kind = SS_PLANES_QUAD;
-  else if ((tp.sym & DDA_SYM_TURN) && nslices >= 2)
-    f.kind = SS_PLANES_PAIR;
-  else if (nslices >= 3)
-    f.kind = SS_PLANES_SLICES;
+  f.kind = dda_planes_kind(tp, nslices);
   if (f.kind == SS_PLANES_NONE) return f;
   const long long tiles = (long long)dda_gp_cols(g, f.kind) * dda_gp_rows(g, f.kind) * ss_planes_groups(f.kind, nslices);
   if (tiles * DDA_GP_MAXGROUPS > 0x7fffffffLL) return SSDdaGatherForm{SS_PLANES_NONE, 1};

@@ -100,7 +100,6 @@ static inline __host__ __device__ int ss_rt_slices(int kind) {
 static inline __host__ __device__ int ss_rt_planes(int kind) {
   return kind <= SS_PLANES_SLICES ? 4 : (kind == SS_RT_ONE ? 1 : 2);
 }
-#define SS_RT_SAME_SLICES 8  // launches of up to this many slices sum in one slice's order
 // the gather layouts are built in square tiles of SS_GATHER_TILE records per direction;
 // records q = 0..n+1 of each row
 #define SS_GATHER_TILE 64

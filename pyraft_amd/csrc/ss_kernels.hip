@@ -2611,6 +2611,7 @@ static int ss_rt_lines(int n, int sl) {
 // launched with.
 static int ss_rt_kind(const SSDevPlan& p, int j0, int j1, int nslices) {
   if (4 * (p.rt_window + 4) > 2 * kSSBpStage[p.rt_variant]) return SS_RT_ONE;  // a window of four does not fit
+  if (ss_planes_stack(nslices)) return SS_PLANES_SLICES;
   if ((p.rt_sym & 2) && j0 == 0 && j1 == p.g.nangles) return SS_PLANES_QUAD;
   if (p.rt_sym & 1) return nslices >= 2 ? SS_PLANES_PAIR : SS_RT_TURN;
   return nslices >= 3 ? SS_PLANES_SLICES : (nslices == 2 ? SS_RT_TWO : SS_RT_ONE);
@@ -2623,14 +2624,14 @@ static dim3 ss_rt_grid(const SSDevPlan& p, int kind) {
   return dim3((cols + BP_TILE_W - 1) / BP_TILE_W, (rows + th - 1) / th);
 }
 
-// Angle groups, by the backprojection's rule.  Up to SS_RT_SAME_SLICES slices take one
+// Angle groups, by the backprojection's rule.  Up to SS_PLANES_STACK slices take one
 // slice's groups (of the form that launch has), so that their sums have the same order.
 static int ss_rt_groups(const SSDevPlan& p, int j0, int j1, int nslices) {
   const int kind = ss_rt_kind(p, j0, j1, nslices);
-  const int one = nslices <= SS_RT_SAME_SLICES ? ss_rt_kind(p, j0, j1, 1) : kind;
+  const int one = nslices <= SS_PLANES_STACK ? ss_rt_kind(p, j0, j1, 1) : kind;
   const dim3 grid = ss_rt_grid(p, one);
   const long long tiles = (long long)grid.x * grid.y *
-                          (nslices <= SS_RT_SAME_SLICES ? 1 : (nslices + ss_rt_slices(kind) - 1) / ss_rt_slices(kind));
+                          (nslices <= SS_PLANES_STACK ? 1 : (nslices + ss_rt_slices(kind) - 1) / ss_rt_slices(kind));
   return ss_angle_groups(tiles, j1 - j0);
 }
 

@@ -51,10 +51,18 @@ extern "C" int raft_ss_radon_noalloc(const raft_ss_plan* p, const float* d_image
   // the plan's slab choice when an earlier call made one (this entry never times)
   hipStream_t stream = as_stream(stream_);
   if ((rc = ss_plan_radon_rows(p, j0, j1, nslices, stream, false, &dp))) return rc;
+  // the limit counts the one-ray form's workspace in any form; the array holds twice that
+  SSDevPlan one = dp;
+  if (dp.radon_planes) {
+    one.radon_planes = SS_PLANES_NONE;
+    one.radon_slab_rows = one.radon_shape = 0;
+    if (2 * ss_radon_layout_bytes(dp, nslices) + ss_radon_scratch(dp, j0, j1, nslices) >
+        2 * (size_t)RAFT_SS_NOALLOC_SCRATCH_BYTES)
+      dp = one;
+  }
   const size_t layout = ss_radon_layout_bytes(dp, nslices) / sizeof(float2);
   const size_t layout_bytes = 2 * layout * sizeof(float2);
-  // the limit counts the one-ray layouts in any form
-  const size_t need = 16 * (size_t)nslices * p->g.n * p->g.pitch + ss_radon_scratch(dp, j0, j1, nslices);
+  const size_t need = 2 * ss_radon_layout_bytes(one, nslices) + ss_radon_scratch(one, j0, j1, nslices);
   if (need > (size_t)RAFT_SS_NOALLOC_SCRATCH_BYTES)
     return ss_set_error(RAFT_SS_EINVAL,
                         "radon_noalloc: %d slice(s) of %d x %d need %zu bytes of workspace, more than the %zu of "

@@ -208,3 +208,21 @@ def test_osem_weights(n, R, A, sc, S):
             bp = O.backprojection(rho, n, **_geo(sc))
             x[i] = np.where(w > 0, x[i] * bp / np.where(w > 0, w, 1.0), x[i])
     assert _rel(got, x) <= REL
+
+
+@pytest.mark.parametrize("n,A,S", [(2048, 60, 1), (2048, 9, 1), (700, 90, 6), (200, 40, 16)])
+def test_noalloc_planes(n, A, S):
+    """The allocation-free Radon on a plan without earlier choices: sizes that its limit admits
+    by the one-ray form's workspace."""
+    import torch
+    from pyraft_amd.device import Plan, current_stream_handle
+    from pyraft_amd.raftypes import libraft
+    print("radon_noalloc", n, A, S, flush=True)
+    p = Plan(n, n, A)
+    x = torch.rand(S, n, n, device="cuda")
+    out = torch.empty(S, A, n, device="cuda")
+    rc = libraft.raft_ss_radon_noalloc(p.handle, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()), 1, 0,
+                                       A, S, current_stream_handle(x.device))
+    assert rc == 0, libraft.raft_ss_last_error()
+    ref = p.radon(x, angle_major=True)
+    assert _rel(out.cpu().numpy(), ref.cpu().numpy().astype(np.float64)) <= 1e-6
