@@ -166,6 +166,12 @@ int raft_ss_plan_host_bounds_mesh(int n, const double *img_corners, int nrays, c
 int raft_ss_plan_host_info(int n, int nrays, int nangles, const double *img_corners, const double *sino_corners,
                            int *info);
 
+/* values that one ray coordinate serves in the Radon of angles [j0, j1) of nslices slices,
+ * computed on the host for a plan with `nirregular` irregular rays: 0 one ray, 1 the image, its
+ * half turn and their mirrors, 2 two slices and their half turns, 3 four slices */
+int raft_ss_plan_host_radon_planes(int n, int nrays, int nangles, const double *img_corners,
+                                   const double *sino_corners, int nirregular, int j0, int j1, int nslices);
+
 /* backprojection staging of every kernel variant computed on the host:
  * windows[v] = rays staged per angle, per_stage[v] = angles per LDS stage (0 when the
  * window does not fit variant v); arrays of RAFT_SS_BP_NVARIANTS ints */

@@ -503,6 +503,22 @@ extern "C" int raft_ss_plan_host_info(int n, int nrays, int nangles, const doubl
   return 0;
 }
 
+extern "C" int raft_ss_plan_host_radon_planes(int n, int nrays, int nangles, const double* img_corners,
+                                              const double* sino_corners, int nirregular, int j0, int j1,
+                                              int nslices) {
+  if (!img_corners || !sino_corners) return set_error(RAFT_SS_EINVAL, "null argument");
+  SSGeom g = make_geom(n, nrays, nangles, img_corners, sino_corners);
+  std::vector<SSAngle> angles;
+  int ndeg = 0;
+  if (n < 2 || nrays < 2 || nangles < 1) return validate_geom(g, angles);
+  build_angles(g, angles, &ndeg);
+  int rc = validate_geom(g, angles);
+  if (rc) return rc;
+  bool turn = false, mirror = false;
+  radon_symmetry(g, angles, &turn, &mirror);
+  return ss_radon_planes_kind(turn, mirror, nirregular, j0 == 0 && j1 == nangles, nslices);
+}
+
 // Host-side backprojection staging of every kernel variant (no device needed):
 // windows[v] = staged rays per angle, per_stage[v] = angles per stage (0: the window
 // does not fit the variant's LDS stage).

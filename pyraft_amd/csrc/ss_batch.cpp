@@ -367,12 +367,8 @@ int ss_plan_range_variant(raft_ss_plan* p, int j0, int j1, hipStream_t stream, i
   return 0;
 }
 
-// The planes that a Radon launch can take (k_radon_planes)
 static int ss_plan_planes(const raft_ss_plan* p, int j0, int j1, int nslices) {
-  if (ss_planes_stack(nslices)) return SS_PLANES_SLICES;
-  if (p->radon_mirror && j0 == 0 && j1 == p->g.nangles) return SS_PLANES_QUAD;
-  if (p->radon_turn && nslices >= 2) return SS_PLANES_PAIR;
-  return nslices >= 3 ? SS_PLANES_SLICES : SS_PLANES_NONE;
+  return ss_radon_planes_kind(p->radon_turn, p->radon_mirror, p->nirregular, j0 == 0 && j1 == p->g.nangles, nslices);
 }
 
 int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipStream_t stream, bool may_time,

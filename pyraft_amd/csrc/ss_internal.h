@@ -68,6 +68,16 @@ int ss_em_launch(const raft_ss_plan* p, const SSEmLaunch& L, const float* d_sino
 int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipStream_t stream, bool may_time,
                        SSDevPlan* dp);
 
+// The planes that a Radon launch can take (k_radon_planes).  None with irregular rays: they are
+// added by k_radon_fixup, which reads the one-ray layouts.
+static inline int ss_radon_planes_kind(bool turn, bool mirror, int nirregular, bool whole_range, int nslices) {
+  if (nirregular > 0) return SS_PLANES_NONE;
+  if (ss_planes_stack(nslices)) return SS_PLANES_SLICES;
+  if (mirror && whole_range) return SS_PLANES_QUAD;
+  if (turn && nslices >= 2) return SS_PLANES_PAIR;
+  return nslices >= 3 ? SS_PLANES_SLICES : SS_PLANES_NONE;
+}
+
 struct raft_ss_plan {
   int device = 0;
   SSGeom g{};

@@ -680,7 +680,7 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE) void k_radon(SSDevPlan p, co
 //
 // Every plane's ray keeps its own exact sample range, delta and output; rays computed twice
 // (the middle ray of an odd detector, theta = 0 and pi/2, slices past the last) are stored
-// once.  Irregular rays have empty ranges here and go to k_radon_fixup.
+// once.  Plans with irregular rays don't take this form (ss_radon_planes_kind).
 // =====================================================================================
 
 // Layout row r of B (image rows) and row c of A (image columns), cells q in [0, n + 1]:
@@ -1156,7 +1156,7 @@ size_t ss_radon_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
 int ss_radon_partials(const SSDevPlan& p, int j0, int j1, int nslices) {
   int rows;
   const int nslab = ss_radon_slabs(p, j0, j1, nslices, &rows);
-  if (nslab == 1 && p.radon_planes) return (int)ss_planes_blocks(p, j0, j1, nslices) + p.nirregular * nslices;
+  if (nslab == 1 && p.radon_planes) return (int)ss_planes_blocks(p, j0, j1, nslices);
   const int main = nslab > 1 ? ss_radon_finish_blocks(j1 - j0, p.g.nrays)
                              : p.nwaves * ((j1 - j0 + RADON_WAVES - 1) / RADON_WAVES);
   return (main + p.nirregular) * nslices;

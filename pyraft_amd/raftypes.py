@@ -142,6 +142,7 @@ _decl("raft_ss_plan_wave_bounds", [_vp, ctypes.POINTER(_i)], _i)
 _decl("raft_ss_plan_host_bounds", [_i, _i, _i, _d4, _d4, ctypes.POINTER(_i),
                                    ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(_i)], _i)
 _decl("raft_ss_plan_host_info", [_i, _i, _i, _d4, _d4, ctypes.POINTER(_i)], _i)
+_decl("raft_ss_plan_host_radon_planes", [_i, _i, _i, _d4, _d4, _i, _i, _i, _i], _i)
 _decl("raft_dda_plan_create", [ctypes.POINTER(_vp), _i, _i, _i, _i, _d4, _d4, _vp], _i)
 _decl("raft_dda_plan_destroy", [_vp], _i)
 _decl("raft_dda_plan_info", [_vp, ctypes.POINTER(_i), _i], _i)
@@ -354,6 +355,7 @@ EXPORTED_SYMBOLS = (
     "raft_backprojection_slantstack_gpu", "raft_em_gpu", "raft_image_phantom_fromdesc",
     "raft_radon_fromdesc", "raft_radon_transpose_slantstack", "raft_ss_legacy_status", "raft_ss_last_error", "raft_ss_version", "raft_ss_plan_create",
     "raft_ss_plan_destroy", "raft_ss_plan_info", "raft_ss_plan_bounds", "raft_ss_plan_wave_bounds", "raft_ss_plan_host_bounds", "raft_ss_plan_host_info",
+    "raft_ss_plan_host_radon_planes",
     "raft_ss_radon", "raft_ss_radon_range", "raft_ss_radon_noalloc", "raft_ss_backprojection", "raft_ss_backprojection_range",
     "raft_ss_radon_transpose", "raft_ss_radon_transpose_range", "raft_ss_fbp_filter", "raft_ss_fbp",
     "raft_ss_em", "raft_ss_phantom", "raft_ss_ramp_kernel", "raft_ss_filter_rows",

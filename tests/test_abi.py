@@ -257,3 +257,17 @@ def test_invalid_geometry_reports_error(lib):
                                       np.zeros((4, 16, 2), np.int32).ctypes.data_as(ctypes.POINTER(ctypes.c_int)),
                                       None, None)
     assert rc == -1 and b"zero-extent" in lib.raft_ss_last_error()
+
+
+@pytest.mark.parametrize("sc,whole,slices,kind", [
+    (DEF_SC, True, 1, 1), (DEF_SC, True, 8, 1), (DEF_SC, True, 12, 3), (DEF_SC, False, 1, 0), (DEF_SC, False, 2, 2),
+    ((0.0, 1.0, 2.0, -1.0), True, 5, 2), ((0.0, 1.03, math.pi, -0.97), True, 2, 0),
+    ((0.0, 1.03, math.pi, -0.97), True, 3, 3)])
+def test_radon_planes_without_irregular_rays_only(lib, sc, whole, slices, kind):
+    """Irregular rays are added from the one-ray layouts, so their plans take no planes."""
+    def form(nirregular):
+        return lib.raft_ss_plan_host_radon_planes(64, 64, 40, (ctypes.c_double * 4)(*DEF_IC),
+                                                  (ctypes.c_double * 4)(*sc), nirregular, 0, 40 if whole else 39,
+                                                  slices)
+    assert form(0) == kind
+    assert form(1) == 0 and form(7) == 0
