@@ -671,7 +671,7 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE) void k_radon(SSDevPlan p, co
 // The layouts hold the planes' values of a cell together (16 bytes), so one 16-byte LDS
 // read gives the lower taps and another the upper taps of all four; the lanes of a read
 // pass hold 16 neighbouring rays (ss_plane_ray), which keeps its conflicts two-way.  Per
-// four updates: 4 VALU for the trajectory, address and the two weights, 8 FMAs, two reads
+// four updates: 5 VALU for the trajectory, address and the two weights, 8 FMAs, two reads
 // (16 updates per CU-clock at any stride).  Sums are taken in FP32 over 8 samples, those over
 // a chunk's rows and those over the ray: 1e-7 from the 64-bit sums at 2048^2 x 1500 (one
 // running sum per ray: 6e-7).  2048^2 x 1500: 1.07 -> 0.78 ms, the layouts' 27 us included; the
@@ -739,7 +739,7 @@ template <int G, bool CHECK, bool OWN>
 __device__ __forceinline__ void ss_planes_group(const ss_f32x4* __restrict__ st, int s, int end, int64_t& u,
                                                 int64_t step, const SSPlaneRanges& rg, float (&acc)[SS_PLANES]) {
   float part[SS_PLANES];
-  const unsigned stb = (unsigned)(size_t)(ss_lds_cell)st;
+  const unsigned stb = ss_rfl((int)(unsigned)(size_t)(ss_lds_cell)st);
 #pragma unroll
   for (int h = 0; h < G; h += 4) {  // four samples' reads in flight
     ss_f32x4 a[4], b[4];
@@ -759,17 +759,21 @@ __device__ __forceinline__ void ss_planes_group(const ss_f32x4* __restrict__ st,
           idx = t < end && (unsigned)(t - rg.lo[0]) <= rg.span[0] ? idx : PLANES_CAP;
         }
       }
-      w[g] = (float)(uint32_t)u;
+      // weights in [0, 1]: left at 2^32 they would overflow sums from 8e28 on
+      w[g] = (float)(uint32_t)u * SS_INV_FIX;
       u += step;
       __asm__ volatile("" : "+v"(u));  // one 64-bit add per sample
-      // one byte address for both cells (the second in the read's offset field)
-      const ss_lds_cell c = (ss_lds_cell)(size_t)(stb + ((unsigned)idx << 4));
+      // one byte address for both cells (the second in the read's offset field): stb + 16 idx, by
+      // hand, as the compiler takes it out of u's words in three instructions
+      unsigned at;
+      __asm__("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at) : "v"(idx), "s"(stb));
+      const ss_lds_cell c = (ss_lds_cell)(size_t)at;
       a[g] = c[0];
       b[g] = c[1];
     }
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const float w1 = 4294967296.f - w[g];
+      const float w1 = 1.f - w[g];
 #pragma unroll
       for (int z = 0; z < SS_PLANES; ++z) {
         float lo = a[g][z], hi = b[g][z];
@@ -928,7 +932,7 @@ __device__ __forceinline__ void ss_planes_item(const SSRadonView& p, const ss_f3
             if (keep) {
               const ss_f32x4* cell = lay + (size_t)s * pitch + (int)(u >> 32);
               const ss_f32x4 a = cell[0], b = cell[1];
-              const float w = (float)(uint32_t)u, w1 = 4294967296.f - w;
+              const float w = (float)(uint32_t)u * SS_INV_FIX, w1 = 1.f - w;
 #pragma unroll
               for (int z = 0; z < SS_PLANES; ++z) {
                 const float v = fmaf(w, b[z], w1 * a[z]);
@@ -952,7 +956,7 @@ __device__ __forceinline__ void ss_planes_item(const SSRadonView& p, const ss_f3
       if (slice0 + pl.slice >= nslices) continue;     // a group past the last slice
       if (pl.turn && kz == k) continue;               // the middle ray, its own half turn
       if (pl.mirror && (j == 0 || jz == j)) continue;  // angles that are their own mirror
-      const float sum = tot[z] * SS_INV_FIX;
+      const float sum = tot[z];
       const size_t so = (size_t)(slice0 + pl.slice) * A * R;
       if (MODE == SS_OUT_PARTIAL) {
         part_out[(size_t)pl.slice * part_slice + (size_t)(jz - jpart) * R + kz] = sum;

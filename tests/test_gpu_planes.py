@@ -226,3 +226,21 @@ def test_noalloc_planes(n, A, S):
     assert rc == 0, libraft.raft_ss_last_error()
     ref = p.radon(x, angle_major=True)
     assert _rel(out.cpu().numpy(), ref.cpu().numpy().astype(np.float64)) <= 1e-6
+
+
+@pytest.mark.parametrize("sc,S", [((0.0, 1.0, PI, -1.0), 6), ((0.0, 1.0, 2.0, -1.0), 6),
+                                  ((0.0, 1.03, PI, -0.97), 8)])
+def test_radon_large_values(sc, S):
+    """Ray sums near the end of FP32's range stay finite: a block of 1e36 (the sums below 1e38) in
+    every kind of planes, launches that take them undivided."""
+    import torch
+    from pyraft_amd.device import Plan
+    n, R, A = 512, 512, 720
+    x = np.zeros((n, n), np.float32)
+    x[200:280, 220:340] = 1e36
+    ref = O.radon(x.astype(np.float64), R, A, **_geo(sc))
+    assert 1e35 < np.abs(ref).max() < 1e38
+    got = Plan(n, R, A, sino_corners=sc).radon(torch.from_numpy(x).cuda().expand(S, n, n).contiguous()).cpu().numpy()
+    assert np.isfinite(got).all()
+    for i in (0, 1, S - 1):
+        assert _rel(got[i], ref) <= REL
