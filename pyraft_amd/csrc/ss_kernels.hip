@@ -2335,14 +2335,16 @@ __device__ __forceinline__ void ss_rtp_border(const SSDevPlan& p, const float* _
         const float u0 = fmaf(-f, q.gs, (float)pix), u1 = u0 + q.gs;
         const int2* rng = p.bounds + (size_t)(ja + jj) * R;
         const int sline = q.branch_a ? col : row;  // the candidates' sample line
+        // every other u near the line reads the range (testing |u - top| < eps instead left out
+        // the float below top - eps, which rounds down at some n)
         bool in0 = q.flag == 1 && u0 >= eps && u0 < top - eps, in1 = q.flag == 1 && u1 >= eps && u1 < top - eps;
-        if ((q.flag == 2 || fabsf(u0) < eps || fabsf(u0 - top) < eps) && (unsigned)k < (unsigned)R) {
+        if (!in0 && (q.flag == 2 || (u0 > -eps && u0 < top + eps)) && (unsigned)k < (unsigned)R) {
           const int2 b = rng[k];
-          in0 = in0 || (sline >= b.x && sline <= b.y);
+          in0 = sline >= b.x && sline <= b.y;
         }
-        if ((q.flag == 2 || fabsf(u1) < eps || fabsf(u1 - top) < eps) && (unsigned)(k + 1) < (unsigned)R) {
+        if (!in1 && (q.flag == 2 || (u1 > -eps && u1 < top + eps)) && (unsigned)(k + 1) < (unsigned)R) {
           const int2 b = rng[k + 1];
-          in1 = in1 || (sline >= b.x && sline <= b.y);
+          in1 = sline >= b.x && sline <= b.y;
         }
         w0 = in0 ? w0 : 0.f;
         w1 = in1 ? w1 : 0.f;

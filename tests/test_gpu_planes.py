@@ -244,3 +244,20 @@ def test_radon_large_values(sc, S):
     assert np.isfinite(got).all()
     for i in (0, 1, S - 1):
         assert _rel(got[i], ref) <= REL
+
+
+@pytest.mark.parametrize("n,A,sc,S", [(512, 720, (0.0, 1.0, PI, -1.0), 1), (512, 720, (0.0, 1.0, PI, -1.0), 5),
+                                      (363, 400, (0.0, 1.0, 2.0, -1.0), 2), (256, 1500, (0.0, 1.0, 2.0, -1.0), 1),
+                                      (393, 500, (0.0, 1.0, PI, -1.0), 1)])
+def test_transpose_border_pixels(n, A, sc, S):
+    """Every pixel, also of the first and last rows and columns: at these sides the float below
+    top - eps, where a border candidate's position decides without its range, rounds down, and
+    some candidates lie on it.  FP32 weights are within 2e-5 of the exact ones; a sample left
+    out is 1e-3 of a pixel's sum and more."""
+    import torch
+    from pyraft_amd.device import Plan
+    y = (1.0 + np.random.default_rng(n).random((n, A))).astype(np.float32)
+    ref = O.radon_transpose(y.astype(np.float64), n, **_geo(sc))
+    got = Plan(n, n, A, sino_corners=sc).radon_transpose(torch.from_numpy(y).cuda().expand(S, n, A).contiguous())
+    for v in got.cpu().numpy():
+        assert np.abs(v - ref).max() <= 2e-5 * np.sqrt(np.mean(ref * ref))
