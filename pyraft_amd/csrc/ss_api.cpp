@@ -309,6 +309,12 @@ static int plan_create(raft_ss_plan** out, int n, int nrays, int nangles, const 
 
   const SSGeom& g = p->g;
   p->nwaves = (nrays + 63) / 64;
+  double spread = 0.0;
+  for (int j = 0; j < nangles; ++j) {
+    const SSAngle &a = p->h_angles[j], &b = p->h_angles[std::min(j + RADON_WAVES - 1, nangles - 1)];
+    spread += fabs(atan2(b.sint * a.cost - b.cost * a.sint, b.cost * a.cost + b.sint * a.sint));
+  }
+  p->angle_spread = spread / nangles;
   if (!p->mesh) {
     p->half_turn = half_turn_symmetric(g, p->h_angles);
     p->mirror = mirror_symmetric(g, p->h_angles);

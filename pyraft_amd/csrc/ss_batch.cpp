@@ -121,7 +121,7 @@ std::map<std::string, TuneEntry> g_tune;
 // A file of another format is ignored and a line that does not parse is skipped (that
 // geometry is timed again).  After each new choice the file is written whole to a
 // temporary name and renamed over the old one.  Callers hold g_tune_mu.
-const char* const kTuneFormat = "pyraft_amd tuning cache 4: backprojection variants x6 in planes, angle groups, radon shapes and planes";
+const char* const kTuneFormat = "pyraft_amd tuning cache 5: backprojection variants x6 in planes, angle groups, radon shapes, planes";
 bool g_tune_loaded = false;
 
 std::string tune_cache_path() {
@@ -371,6 +371,13 @@ static int ss_plan_planes(const raft_ss_plan* p, int j0, int j1, int nslices) {
   return ss_radon_planes_kind(p->radon_turn, p->radon_mirror, p->nirregular, j0 == 0 && j1 == p->g.nangles, nslices);
 }
 
+// Updates (image side x rays x angles x slices) from which the Radon's planes are tried.  Below,
+// a launch lasts as long as its latencies, which the planes' fewer and longer blocks add to: over
+// 1000 launches of 64^2 to 1448^2 they took 1.1 to 1.2 times the one-ray form's time below 2^24
+// updates and never less than 0.9 of it, around 2^24 to 2^27 between 1.5 and 0.6 of it, from 2^28
+// on 0.9 on average.
+static constexpr double kPlanesUpdates = 16777216.0;
+
 int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipStream_t stream, bool may_time,
                        SSDevPlan* out) {
   out->radon_slab_rows = 0;
@@ -382,8 +389,7 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
     return 0;
   }
   if (j1 <= j0) return 0;
-  SSDevPlan dp = p->dev();
-  const int planes = ss_plan_planes(p, j0, j1, nslices);
+  const SSDevPlan dp = p->dev();
   int r0 = n;
   const bool divides = ss_radon_slabs(dp, j0, j1, nslices, &r0) > 1;
   const long long pk = ((long long)(j1 - j0) << 20) | (long long)std::min(nslices, (1 << 20) - 1);
@@ -397,12 +403,17 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
       return 0;
     }
   }
-  // a planes launch that fills the chip undivided wins without timing: 2048^2 x 1500 780 us
-  // against 1070 with one ray per trajectory, 1448^2 x 500 204 against 266, 16 x 512^2 x 720
-  // 495 against 595, 8 x 768^2 x 600 on a mesh 429 against 572
   SSDevPlan dpp = dp;
-  dpp.radon_planes = planes;
-  if (planes && ss_planes_blocks(dpp, j0, j1, nslices) >= SS_RADON_SLAB_BLOCKS) {
+  if ((double)n * p->g.nrays * (j1 - j0) * nslices >= kPlanesUpdates)
+    dpp.radon_planes = ss_plan_planes(p, j0, j1, nslices);
+  const int planes = dpp.radon_planes;
+  // A launch that the planes suit in every respect takes them without timing: blocks for the
+  // whole chip (ss_planes_suit), an image of 512^2 or more, and angles near enough that a block's
+  // eight share their windows.  2048^2 x 1500 780 us against 1070 with one ray per trajectory, 1448^2
+  // x 500 204 / 266, 512^2 x 720 on a wide detector, 5 slices, 213 / 266, 8 x 768^2 x 600 on a mesh 361 / 531.
+  // Where one of them fails, one ray can win: 9 x 789^2 x 180 (angles far apart) 308 / 292, 5 x
+  // 512^2 x 720 in groups of four slices 238 / 196, 9 x 182^2 x 720 104 / 94.
+  if (planes && n >= 512 && p->angle_spread <= 0.045 && ss_planes_suit(dpp, j0, j1, nslices)) {
     out->radon_slab_rows = n;
     out->radon_planes = planes;
     return 0;
@@ -410,44 +421,54 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
   if (!may_time) return 0;  // the rule, shape 0 (no lookups that allocate)
   // candidates (slab rows, shape | planes << 1); rows 0 is the default rule, which does not
   // divide here
-  std::vector<std::pair<int, int>> cand;
+  typedef std::vector<std::pair<int, int>> Cands;
+  Cands one, four;
+  if (divides) {
+    one = {{r0, 0}, {r0, 1}};
+    if (2 * r0 < n) one.push_back({2 * r0, 0});
+    if (r0 / 2 >= RADON_SLAB_ALIGN && (r0 / 2) % RADON_SLAB_ALIGN == 0) one.push_back({r0 / 2, 0});
+    one.push_back({n, 0});
+    one.push_back({n, 1});
+  } else {
+    one = {{0, 0}, {0, 1}};
+  }
   if (planes) {
     int rp = n;
     (void)ss_radon_slabs(dpp, j0, j1, nslices, &rp);
-    cand = {{rp, planes << 1}};
-    if (2 * rp < n) cand.push_back({2 * rp, planes << 1});
-    if (rp < n) cand.push_back({n, planes << 1});
-    cand.push_back({r0, 0});
-    cand.push_back({r0, 1});
-    if (divides && 2 * r0 < n) cand.push_back({2 * r0, 0});
-  } else if (divides) {
-    cand = {{r0, 0}, {r0, 1}};
-    if (2 * r0 < n) cand.push_back({2 * r0, 0});
-    if (r0 / 2 >= RADON_SLAB_ALIGN && (r0 / 2) % RADON_SLAB_ALIGN == 0) cand.push_back({r0 / 2, 0});
-    cand.push_back({n, 0});
-    cand.push_back({n, 1});
-  } else {
-    cand = {{0, 0}, {0, 1}};
+    four = {{rp, planes << 1}};
+    if (2 * rp < n) four.push_back({2 * rp, planes << 1});
+    if (rp < n) four.push_back({n, planes << 1});
   }
-  const std::string key = plan_key(p) + "|radon|range" + std::to_string(j1 - j0) + "|s" + std::to_string(nslices);
+  // cache entries: the one-ray candidate, and (planes) 0 for that or 1 + the planes' candidate
+  const std::string range = "|range" + std::to_string(j1 - j0) + "|s" + std::to_string(nslices);
+  const std::string key = plan_key(p) + "|radon" + range, key4 = plan_key(p) + "|planes" + range;
   // mesh plans are timed per plan but kept out of the shared cache: its key does not
   // name their t and theta tables
   const bool shared = !p->mesh;
   TuneEntry cached;
-  int chosen = -1;
-  if (shared && tune_find(key, &cached) && cached.variant >= 0 && cached.variant < (int)cand.size())
-    chosen = cached.variant;
-  if (chosen < 0) {
+  int chosen1 = -1, chosen4 = planes ? -1 : 0;
+  if (shared && planes && tune_find(key4, &cached) && cached.variant >= 0 && cached.variant <= (int)four.size())
+    chosen4 = cached.variant;
+  if (shared && chosen4 <= 0 && tune_find(key, &cached) && cached.variant >= 0 && cached.variant < (int)one.size())
+    chosen1 = cached.variant;
+  if (chosen4 < 0 || (chosen4 == 0 && chosen1 < 0)) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(stream, &cs));
     if (cs != hipStreamCaptureStatusNone) return 0;  // the rule, untimed
+    auto form = [&](const std::pair<int, int>& c) {
+      SSDevPlan d = dp;
+      d.radon_slab_rows = c.first;
+      d.radon_shape = c.second & 1;
+      d.radon_planes = c.second >> 1;
+      return d;
+    };
     size_t layout = 0, slab_bytes = 0;
-    for (const auto& c : cand) {
-      dp.radon_slab_rows = c.first;
-      dp.radon_planes = c.second >> 1;
-      layout = std::max(layout, ss_radon_layout_bytes(dp, nslices) / sizeof(float2));
-      slab_bytes = std::max(slab_bytes, ss_radon_scratch(dp, j0, j1, nslices));
-    }
+    for (const Cands* list : {&one, &four})
+      for (const auto& c : *list) {
+        const SSDevPlan d = form(c);
+        layout = std::max(layout, ss_radon_layout_bytes(d, nslices) / sizeof(float2));
+        slab_bytes = std::max(slab_bytes, ss_radon_scratch(d, j0, j1, nslices));
+      }
     const size_t img = (size_t)nslices * n * n, sino = (size_t)nslices * p->g.nrays * p->g.nangles;
     DevBuf ws;
     HIP_TRY(ws.alloc(2 * layout * sizeof(float2) + (img + sino) * sizeof(float) + slab_bytes, stream));
@@ -457,31 +478,52 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
     float* sout = x + img;
     float* slabs = sout + sino;
     HIP_TRY(ss_launch_fill(x, 1.0f, img, stream));
-    TuneEntry te;
-    for (int v = 0; v < SS_BP_NVARIANTS; ++v) te.times[v] = -1.0;
-    int best = 0, rc = 0;
-    for (int c = 0; c < (int)cand.size() && c < SS_BP_NVARIANTS; ++c) {
-      dp.radon_slab_rows = cand[c].first;
-      dp.radon_shape = cand[c].second & 1;
-      dp.radon_planes = cand[c].second >> 1;
+    // the forms' layouts differ: they count where both forms are timed
+    if (!planes) HIP_TRY(ss_launch_gather_layouts(dp, x, gA, gB, nslices, stream));
+    TuneEntry te1, te4;
+    for (int v = 0; v < SS_BP_NVARIANTS; ++v) te1.times[v] = te4.times[v] = -1.0;
+    auto time = [&](const std::pair<int, int>& c, double* us) -> int {
+      const SSDevPlan d = form(c);
       SSEmRatioArgs none{nullptr, nullptr};
       auto run = [&]() -> int {
-        HIP_TRY(ss_launch_gather_layouts(dp, x, gA, gB, nslices, stream));
-        HIP_TRY(ss_launch_radon(dp, gA, gB, j0, j1, nslices, SS_OUT_SINOT, sout, none, slabs, stream));
+        if (planes) HIP_TRY(ss_launch_gather_layouts(d, x, gA, gB, nslices, stream));
+        HIP_TRY(ss_launch_radon(d, gA, gB, j0, j1, nslices, SS_OUT_SINOT, sout, none, slabs, stream));
         return 0;
       };
-      if ((rc = time_best(run, 3, stream, &te.times[c]))) return rc;
-      if (te.times[c] < te.times[best]) best = c;
+      return time_best(run, 3, stream, us);
+    };
+    // the first candidate of each form, then the others of a form that is not 1.3 times slower
+    // (over the 1000 launches above that never lost against timing all)
+    int rc = 0;
+    double best1 = 1e300, best4 = 1e300;
+    int b1 = 0, b4 = 0;
+    if ((rc = time(one[0], &te1.times[0]))) return rc;
+    best1 = te1.times[0];
+    if (planes) {
+      if ((rc = time(four[0], &te4.times[1]))) return rc;
+      best4 = te4.times[1];
     }
-    te.variant = best;
-    if (shared) tune_store(key, te);
-    chosen = best;
+    const double first1 = best1, first4 = best4;
+    for (int c = 1; first4 <= 1.3 * first1 && c < (int)four.size(); ++c) {
+      if ((rc = time(four[c], &te4.times[1 + c]))) return rc;
+      if (te4.times[1 + c] < best4) best4 = te4.times[1 + c], b4 = c;
+    }
+    for (int c = 1; first1 <= 1.3 * first4 && c < (int)one.size(); ++c) {
+      if ((rc = time(one[c], &te1.times[c]))) return rc;
+      if (te1.times[c] < best1) best1 = te1.times[c], b1 = c;
+    }
+    te1.variant = chosen1 = b1;
+    te4.times[0] = best1;
+    te4.variant = chosen4 = best4 < best1 ? 1 + b4 : 0;
+    if (shared && planes) tune_store(key4, te4);
+    if (shared && chosen4 == 0) tune_store(key, te1);
   }
+  const std::pair<int, int>& c = chosen4 > 0 ? four[chosen4 - 1] : one[chosen1];
   std::lock_guard<std::mutex> lock(p->radon_mutex);
-  p->radon_rows[pk] = cand[chosen].first | (cand[chosen].second << 24);
-  out->radon_slab_rows = cand[chosen].first;
-  out->radon_shape = cand[chosen].second & 1;
-  out->radon_planes = cand[chosen].second >> 1;
+  p->radon_rows[pk] = c.first | (c.second << 24);
+  out->radon_slab_rows = c.first;
+  out->radon_shape = c.second & 1;
+  out->radon_planes = c.second >> 1;
   return 0;
 }
 

@@ -57,12 +57,13 @@ int ss_em_launch(const raft_ss_plan* p, const SSEmLaunch& L, const float* d_sino
                  int nslices, void* ws, double* d_ll, hipStream_t stream);
 // Launch choice of the plan's Radon over angle ranges of j1 - j0 angles on nslices slices:
 // the block shape and the sample rows per slab (SSDevPlan::radon_shape, radon_slab_rows),
-// set in *dp.  Candidates: both shapes without row slabs and, where the default rule
-// divides the launch, both shapes at the rule's slab rows and shape 0 at twice and half of
-// them.  The fastest is timed once per process (gather layouts built first, not timed)
-// and cached with the backprojection choices (mesh plans: per plan only, since the cache
-// key does not name their tables); no timing while `stream` is captured, and
-// with `may_time` false only the plan's earlier choice or the rule with shape 0 (no host
+// and, for large launches, the planes (SSDevPlan::radon_planes), set in *dp.  Candidates: both
+// shapes without row slabs and, where the default rule divides the launch, both shapes at the
+// rule's slab rows and shape 0 at twice and half of them; the planes with their rule's rows,
+// twice those and undivided.  The fastest is timed once per process (the gather layouts too
+// where the planes are among the candidates) and cached with the backprojection choices (mesh
+// plans: per plan only, since the cache key does not name their tables); no timing while
+// `stream` is captured, and with `may_time` false only the plan's earlier choice or the rule with shape 0 (no host
 // allocation).  Rows pinned by raft_ss_plan_set_radon_slab_rows apply to every launch,
 // with shape 0.
 int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipStream_t stream, bool may_time,
@@ -101,6 +102,7 @@ struct raft_ss_plan {
   // the grids map onto themselves under a half turn; and the angles under theta -> pi - theta
   bool half_turn = false, mirror = false;
   bool radon_turn = false, radon_mirror = false;  // the same of the Radon's samples (radon_symmetry)
+  double angle_spread = 0.0;  // mean angle between the first and the last of a Radon block's angles
   // angles per stage of the backprojection with `planes` planes (0: not available)
   int bp_stage_v(int v, int planes) const {
     if (!half_turn || (planes == 4 && !mirror) || bp_angles_v[v] <= 0) return 0;

@@ -116,6 +116,7 @@ hipError_t ss_launch_gather_planes(const SSDevPlan& p, const float* image, float
 // bytes of one layout (gatherA or gatherB) in the launch's form
 size_t ss_radon_layout_bytes(const SSDevPlan& p, int nslices);
 long long ss_planes_blocks(const SSDevPlan& p, int j0, int j1, int nslices);
+bool ss_planes_suit(const SSDevPlan& p, int j0, int j1, int nslices);
 hipError_t ss_launch_sino_to_t(const float* sino, float* sinoT, int R, int A, int nslices, hipStream_t stream);
 hipError_t ss_launch_t_to_sino(const float* sinoT, float* sino, int R, int A, int nslices, hipStream_t stream);
 

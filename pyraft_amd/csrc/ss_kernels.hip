@@ -1151,6 +1151,15 @@ long long ss_planes_blocks(const SSDevPlan& p, int j0, int j1, int nslices) {
          ss_planes_groups(p.radon_planes, nslices);
 }
 
+// Whether an undivided planes launch has blocks with work for the whole chip, at most one
+// launched block in nine without (SSPlanesOrder) and at most one plane in 17 empty
+bool ss_planes_suit(const SSDevPlan& p, int j0, int j1, int nslices) {
+  const SSPlanesOrder o = ss_planes_order(p, j0, j1);
+  const long long groups = ss_planes_groups(p.radon_planes, nslices), work = (long long)o.g * o.y;
+  return work * groups >= SS_RADON_SLAB_BLOCKS && 8LL * o.blocks <= 9 * work &&
+         16 * groups * ss_planes_slices(p.radon_planes) <= 17LL * nslices;
+}
+
 size_t ss_radon_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
   int rows;
   const int nslab = ss_radon_slabs(p, j0, j1, nslices, &rows);

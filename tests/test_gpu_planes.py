@@ -261,3 +261,34 @@ def test_transpose_border_pixels(n, A, sc, S):
     got = Plan(n, n, A, sino_corners=sc).radon_transpose(torch.from_numpy(y).cuda().expand(S, n, A).contiguous())
     for v in got.cpu().numpy():
         assert np.abs(v - ref).max() <= 2e-5 * np.sqrt(np.mean(ref * ref))
+
+
+CHOICES = r"""
+import sys
+sys.path.insert(0, %r)
+import torch
+from pyraft_amd.device import Plan
+for n, A in ((256, 180), (700, 300)):
+    Plan(n, n, A).radon(torch.rand((n, n), device="cuda"))
+torch.cuda.synchronize()
+"""
+
+
+def test_small_radon_keeps_its_candidates(tmp_path):
+    """Launches of less than 2^24 updates, where the planes never pay, choose (and time) among the
+    one-ray forms alone; larger ones add the planes to all of those."""
+    import json
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    path = tmp_path / "tune.json"
+    out = subprocess.run([sys.executable, "-c", CHOICES % root], env=dict(os.environ, PYRAFT_AMD_TUNE_CACHE=str(path)),
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    entries = json.loads(path.read_text())["entries"]
+    small = {k.split("|")[-3]: v for k, v in entries.items() if "|256|256|180|" in k}
+    large = {k.split("|")[-3]: v for k, v in entries.items() if "|700|700|300|" in k}
+    assert set(small) == {"radon"} and "planes" in large
+    assert sum(t > 0 for t in small["radon"]["times_us"]) == 5  # both shapes in 32-row slabs and whole, 64 rows
+    assert large["planes"]["times_us"][1] > 0 and large["planes"]["times_us"][0] > 0
