@@ -263,13 +263,16 @@ static int bp_variants(raft_ss_plan* p) {
                      p->bp_window_v[SS_BP_DEFAULT_VARIANT]);
   p->bp_variant = p->bp_angles_v[SS_BP_DEFAULT_VARIANT] > 0 ? SS_BP_DEFAULT_VARIANT : first;
   // small images start from the 2-rows-per-thread tiles (twice the blocks); the autotuner may
-  // still pick another variant.  One plane: fewer than 4 default tiles per CU.  With planes
-  // (and angle groups) the larger tile wins earlier: 4 planes measured 61 against 57 us at
-  // 768^2 x 500, 43 against 48-54 at 512^2 x 720, 18 against 21 at 256^2 x 180.
+  // still pick another variant.  One plane, or undivided planes: fewer than 4 default tiles per CU
+  // (789^2 x 40 with two planes 11.6 against 15.1 us).  With planes and angle groups the larger tile
+  // wins earlier: 4 planes measured 61 against 57 us at 768^2 x 500, 43 against 48-54 at 512^2 x
+  // 720, 18 against 21 at 256^2 x 180.
   const int kSmallVariant = 1;  // 2 pixel rows per thread, 2048 staged pairs
-  const int planes = ss_bp_planes(p->dev(SS_BP_DEFAULT_VARIANT), 0, p->g.nangles);
+  const SSDevPlan dp = p->dev(SS_BP_DEFAULT_VARIANT);
+  const int planes = ss_bp_launch_planes(dp, 0, p->g.nangles, 1);
+  const bool groups = planes > 1 && ss_bp_groups(dp, 0, p->g.nangles, 1) > 1;
   if (p->bp_variant == SS_BP_DEFAULT_VARIANT && kSSBpRows[kSmallVariant] == 2 && p->bp_angles_v[kSmallVariant] > 0 &&
-      ss_bp_tiles(p->g.n, SS_BP_DEFAULT_VARIANT, planes) * planes < (planes > 1 ? 512 : 1024))
+      ss_bp_tiles(p->g.n, SS_BP_DEFAULT_VARIANT, planes) * planes < (groups ? 512 : 1024))
     p->bp_variant = kSmallVariant;
   return 0;
 }

@@ -173,6 +173,21 @@ hipError_t ss_launch_bp_weights(const SSDevPlan& p, int nsubsets, float* out, hi
 // 50 us undivided, 64 in two groups).
 // ss_bp_groups: the group count (1: no division); ss_bp_scratch: the bytes of the partial
 // images (0 when not divided).
+//
+// Few angles: a group's second pass costs more than the groups even out, and an undivided block
+// of four planes waits longer per angle (0.24 us, with one or two planes 0.17).  Fewer than
+// SS_BP_SHORT_ANGLES, or with T >= SS_BP_SHORT_TILES tiles of 32 x 16 pixels (two planes) up to
+// SS_BP_SHORT_ANGLES + T / 8 and at most 160, launch undivided, with two planes in place of four
+// below SS_BP_SHORT_QUAD tiles of four (us, in groups with four planes / undivided with two / with
+// four: 512^2 x 24 13.0 / 10.0 / 10.0; 512^2 x 64 13.3 / 15.0 / 18.7; 789^2 x 40 18.7 / 11.6 / 13.8; 789^2 x 91
+// 24.1 / 20.3 / 23.7; 1024^2 x 128 31.6 / 29.3 / 34.2; 1024^2 x 180 35.5 / 38.9 / 43.7; 1448^2 x 40 26.7 / 20.6 /
+// 18.6).  In groups, four planes pay from SS_BP_QUAD_WORK tiles of four (32 x 16) x angles on (a
+// filtered backprojection, two / four planes: 135^2 x 47 16.5 / 17.7, 256^2 x 91 16.4 / 17.7, 256^2 x 128
+// 17.4 / 19.0, 256^2 x 180 19.3 / 18.6, 363^2 x 91 21.8 / 21.2).
+#define SS_BP_QUAD_WORK 5000
+#define SS_BP_SHORT_ANGLES 32
+#define SS_BP_SHORT_TILES 240
+#define SS_BP_SHORT_QUAD 512
 #define SS_BP_GROUP_SCALE 0.22
 #define SS_BP_ROUND_BLOCKS 1024
 #define SS_BP_GROUP_ANGLES 8
@@ -194,7 +209,9 @@ hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int
 // ---- batched forms (items: gather = SS_GATHER_TILE^2 tiles; radon = 64-ray groups x blocks of
 //      8 angles x row slabs; finish = 256 rays of an entry; fixup = irregular rays; bp = pixel
 //      tiles of the variant; transpose = 32x32 tiles)
+// planes that angles [j0, j1) admit, and those that a launch takes
 int ss_bp_planes(const SSDevPlan& p, int j0, int j1);
+int ss_bp_launch_planes(const SSDevPlan& p, int j0, int j1, int nslices);
 int ss_bp_tiles(int n, int variant, int planes);
 // gather tile side for a batch of images with sides n[0..count): SS_GATHER_TILE when the
 // batch has at least 1024 such tiles, else 32 (items are tiles of that side)

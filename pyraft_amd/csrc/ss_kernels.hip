@@ -1758,9 +1758,25 @@ static int ss_angle_groups(long long tiles, int nj) {
   return (int)std::min(floor(g + 0.5), (double)(nj / SS_BP_GROUP_ANGLES));
 }
 
+// Whether a backprojection has too few angles for its tiles to be divided (SS_BP_SHORT_*)
+static bool ss_bp_short(const SSDevPlan& p, int j0, int j1, int nslices) {
+  const long long tiles = (long long)ss_bp_tiles(p.g.n, 1, 2) * std::max(nslices, 1);  // 32 x 16 pixels, two planes
+  return j1 - j0 < SS_BP_SHORT_ANGLES ||
+         (tiles >= SS_BP_SHORT_TILES && j1 - j0 <= std::min(160LL, SS_BP_SHORT_ANGLES + tiles / 8));
+}
+
+int ss_bp_launch_planes(const SSDevPlan& p, int j0, int j1, int nslices) {
+  const int planes = ss_bp_planes(p, j0, j1), ns = std::max(nslices, 1);
+  if (planes < 4 || p.bp_pair <= 0) return planes;
+  const long long small = (long long)ss_bp_tiles(p.g.n, 1, 4) * ns, large = (long long)ss_bp_tiles(p.g.n, 0, 4) * ns;
+  if (small * (j1 - j0) < SS_BP_QUAD_WORK) return 2;
+  return ss_bp_short(p, j0, j1, nslices) && large < SS_BP_SHORT_QUAD ? 2 : 4;
+}
+
 int ss_bp_groups(const SSDevPlan& p, int j0, int j1, int nslices) {
-  return ss_angle_groups((long long)ss_bp_tiles(p.g.n, p.bp_variant, ss_bp_planes(p, j0, j1)) * std::max(nslices, 1),
-                         j1 - j0);
+  if (ss_bp_short(p, j0, j1, nslices)) return 1;
+  const int planes = ss_bp_launch_planes(p, j0, j1, nslices);
+  return ss_angle_groups((long long)ss_bp_tiles(p.g.n, p.bp_variant, planes) * std::max(nslices, 1), j1 - j0);
 }
 
 size_t ss_bp_scratch(const SSDevPlan& p, int j0, int j1, int nslices) {
@@ -1779,7 +1795,7 @@ hipError_t ss_launch_backprojection(const SSDevPlan& p, const float* sinoT, int 
   const int G = scratch ? ss_bp_groups(p, j0, j1, nslices) : 1;
   const int kmode = G > 1 ? SS_BP_PARTIAL : mode;
   float* kout = G > 1 ? scratch : out;
-  const int planes = ss_bp_planes(p, j0, j1);
+  const int planes = ss_bp_launch_planes(p, j0, j1, nslices);
   dim3 grid(ss_bp_tile_cols(n, planes), (ss_bp_rows(n, planes) + th - 1) / th, nslices * G);
 #define SS_BP_LAUNCH_PL(ROWS, STAGE, PL)                                                                          \
   do {                                                                                                            \

@@ -292,3 +292,24 @@ def test_small_radon_keeps_its_candidates(tmp_path):
     assert set(small) == {"radon"} and "planes" in large
     assert sum(t > 0 for t in small["radon"]["times_us"]) == 5  # both shapes in 32-row slabs and whole, 64 rows
     assert large["planes"]["times_us"][1] > 0 and large["planes"]["times_us"][0] > 0
+
+
+# one angle on either side of the line between undivided and divided launches: few angles at any
+# size, more where the tiles fill the chip; two planes and four
+@pytest.mark.parametrize("n,A,sc,groups", [
+    (40, 31, (0.0, 1.0, PI, -1.0), False), (40, 32, (0.0, 1.0, PI, -1.0), True),
+    (512, 64, (0.0, 1.0, PI, -1.0), False), (512, 65, (0.0, 1.0, PI, -1.0), True),
+    (789, 40, (0.0, 1.0, 2.0, -1.0), False), (789, 110, (0.0, 1.0, PI, -1.0), False),
+    (789, 111, (0.0, 1.0, PI, -1.0), True), (1448, 24, (0.0, 1.0, PI, -1.0), False),
+    (500, 60, (0.0, 1.03, PI, -0.97), False)])
+def test_backprojection_few_angles(n, A, sc, groups):
+    import torch
+    from pyraft_amd.device import Plan
+    s = np.random.default_rng(n + A).random((3, n, A)).astype(np.float32)
+    p = Plan(n, n, A, sino_corners=sc)
+    assert (p.info()["bp_groups"] > 1) == groups
+    got = p.backprojection(torch.from_numpy(s).cuda()).cpu().numpy()
+    one = p.backprojection(torch.from_numpy(s[0]).cuda()).cpu().numpy()
+    ref = O.backprojection(s[0].astype(np.float64), n, **_geo(sc))
+    assert _rel(one, ref) <= REL and _rel(got[0], ref) <= REL
+    assert _rel(got[2], O.backprojection(s[2].astype(np.float64), n, **_geo(sc))) <= REL
