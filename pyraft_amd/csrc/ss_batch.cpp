@@ -680,13 +680,13 @@ int build_launch(raft_ss_batch* b, BatchLaunch& L, int kind, int S, int bsub, in
     if (S > 0) subset_range(p.g.nangles, S, bsub, &j0, &j1);
     blocks += ss_radon_blocks(p.nwaves, j0, j1);
   }
-  // Planes of the backprojection's tiles: whole ranges as the per-plan launch takes them.
+  // Planes of the backprojection's tiles: whole ranges as a plan's launch of the slice takes them.
   // Subset ranges are short, so a block's time is latency and fewer blocks cost more than
   // the planes save: two planes from SS_BATCH_PAIR_TILES tiles on.  An OSEM call of 8
   // subsets: 12 slices of 261^2 to 1021^2 (4900 paired tiles) 1531 us with two planes and
   // 1650 with one, 2 slices of 556^2 x 1242 (650 tiles) 689 and 629.
   auto bp_planes = [&](const raft_ss_plan& p, int j0, int j1, bool pairs) {
-    if (mode == SS_BP_PLAIN && j0 == 0 && j1 == p.g.nangles) return ss_bp_planes(p.dev(v), j0, j1);
+    if (mode == SS_BP_PLAIN && j0 == 0 && j1 == p.g.nangles) return ss_bp_launch_planes(p.dev(v), j0, j1, 1);
     return pairs && p.bp_stage_v(v, 2) > 0 ? 2 : 1;
   };
   bool pairs = true;
@@ -1183,7 +1183,7 @@ extern "C" int raft_ss_batch_tune(raft_ss_batch* b, int reps, int flags, void* s
         sl.sino_off = b->sino_off[i];
         sl.lay_off = b->lay_off[i];
         SSBatchEntry e{(int)h.size(), 0, std::min(sl.p.g.nangles, 360), (int)total};
-        e.planes = ss_bp_planes(sl.p, e.j0, e.j1);
+        e.planes = ss_bp_launch_planes(sl.p, e.j0, e.j1, 1);
         h.push_back(sl);
         L.entries.push_back(e);
         total += ss_bp_tiles(sl.p.g.n, v, e.planes);
