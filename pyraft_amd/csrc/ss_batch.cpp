@@ -587,7 +587,19 @@ struct GraphEntry {
   hipGraphExec_t exec = nullptr;
 };
 
-constexpr long long SS_BATCH_PAIR_TILES = 2048;
+// Rules of a batch's backprojection, by its tiles of 32 x 16 pixels with two planes.  Over 232 batches
+// of 2 to 64 slices (64^2 to 1400^2, equal sides and sides spread over a factor of four), the mean time
+// of an OSEM call with subsets of 22 to 720 angles, one plane and 2-row tiles = 1, and of a
+// whole-range backprojection with 4 rows, 2 rows = 1:
+//   tiles           two planes: 2 rows   4 rows        whole range, 4 rows
+//   below 256       0.94 - 1.01          1.15 - 1.30   1.50
+//   256 - 511       0.94 - 1.00          1.12 - 1.23   1.51
+//   512 - 1023      0.88 - 0.97          1.01 - 1.10   1.45
+//   1024 - 4095     0.81 - 0.90          0.83 - 0.93   1.12
+//   4096 - 8191     0.78 - 0.87          0.75 - 0.85   0.92
+//   from 8192       0.79 - 0.85          0.74 - 0.81   0.82
+constexpr long long SS_BATCH_PAIR_TILES = 512;
+constexpr long long SS_BATCH_ROWS_TILES = 8192;  // 4-row tiles from here on
 
 int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
@@ -681,10 +693,8 @@ int build_launch(raft_ss_batch* b, BatchLaunch& L, int kind, int S, int bsub, in
     blocks += ss_radon_blocks(p.nwaves, j0, j1);
   }
   // Planes of the backprojection's tiles: whole ranges as a plan's launch of the slice takes them.
-  // Subset ranges are short, so a block's time is latency and fewer blocks cost more than
-  // the planes save: two planes from SS_BATCH_PAIR_TILES tiles on.  An OSEM call of 8
-  // subsets: 12 slices of 261^2 to 1021^2 (4900 paired tiles) 1531 us with two planes and
-  // 1650 with one, 2 slices of 556^2 x 1242 (650 tiles) 689 and 629.
+  // Subset ranges are short, so a block's time is latency, and a launch of few tiles is not
+  // shorter for having fewer: two planes from SS_BATCH_PAIR_TILES tiles on.
   auto bp_planes = [&](const raft_ss_plan& p, int j0, int j1, bool pairs) {
     if (mode == SS_BP_PLAIN && j0 == 0 && j1 == p.g.nangles) return ss_bp_launch_planes(p.dev(v), j0, j1, 1);
     return pairs && p.bp_stage_v(v, 2) > 0 ? 2 : 1;
@@ -873,6 +883,7 @@ extern "C" int raft_ss_batch_create(raft_ss_batch** out, int nslices, const int*
   b->img_off.resize(nslices);
   b->sino_off.resize(nslices);
   b->lay_off.resize(nslices);
+  long long tiles = 0;
   for (int i = 0; i < nslices; ++i) {
     const double* ic = img_corners ? img_corners + 4 * i : dic;
     const double* sc = sino_corners ? sino_corners + 4 * i : dsc;
@@ -887,12 +898,7 @@ extern "C" int raft_ss_batch_create(raft_ss_batch** out, int nslices, const int*
       it = by_geom.emplace(key, std::shared_ptr<raft_ss_plan>(p, raft_ss_plan_destroy)).first;
     }
     b->plans[i] = it->second;
-    // Batched launches have no angle groups, and their OSEM ranges are short: images of up to
-    // 1024^2 start from the 2-rows-per-thread tiles, twice the blocks (12 slices of 261^2 to
-    // 1021^2, 8 subsets: 1531 us an iteration against 1675 with 4 rows, whole-range
-    // backprojection 333 against 418); one variant for all is one launch for all.
-    const raft_ss_plan& pl = *it->second;
-    b->variant[i] = pl.half_turn && n[i] <= 1024 && pl.bp_angles_v[kBatchVariant] > 0 ? kBatchVariant : pl.bp_variant;
+    if (it->second->half_turn) tiles += ss_bp_tiles(n[i], kBatchVariant, 2);
     // 256-byte aligned slices in the packed buffers
     b->img_off[i] = b->img_total;
     b->img_total = align_up(b->img_total + (int64_t)n[i] * n[i], 64);
@@ -900,6 +906,12 @@ extern "C" int raft_ss_batch_create(raft_ss_batch** out, int nslices, const int*
     b->sino_total = align_up(b->sino_total + (int64_t)nrays[i] * nangles[i], 64);
     b->lay_off[i] = b->lay_total;
     b->lay_total = align_up(b->lay_total + (int64_t)n[i] * it->second->g.pitch, 32);
+  }
+  // one variant for all symmetric slices is one launch for all
+  const int v = tiles < SS_BATCH_ROWS_TILES ? kBatchVariant : SS_BP_DEFAULT_VARIANT;
+  for (int i = 0; i < nslices; ++i) {
+    const raft_ss_plan& pl = b->plan(i);
+    b->variant[i] = pl.half_turn && pl.bp_angles_v[v] > 0 ? v : pl.bp_variant;
   }
   b->gather_tile = ss_batch_gather_tile(n, nslices);
   *out = b.release();

@@ -246,3 +246,23 @@ def test_one_slice_batch_em_is_the_plan_em(torch_mod):
         assert [l[0] for l in gll] == own_ll
         junk = torch.randn(1 << 18, device="cuda")
         (junk * 2).sum().item()
+
+
+@pytest.mark.parametrize("sizes,angles,variant", [([256] * 7, 64, 1), ([256] * 8, 64, 1), ([1100, 1100], 20, 1),
+                                                  ([64] * 2049, 8, 0)])
+def test_batch_tiles_choose_the_variant(torch_mod, sizes, angles, variant):
+    """2-row tiles below 8192 of them whatever the images' sides, 4-row tiles from there on; an OSEM
+    call on either side of the 512 tiles from which subsets take two pixels per coordinate."""
+    torch = torch_mod
+    from pyraft_amd.batch import Batch
+    from pyraft_amd.device import Plan
+    b = Batch(sizes, nangles=[angles] * len(sizes))
+    assert {b.info(i)["bp_variant"] for i in range(len(sizes))} == {variant}
+    n = sizes[0]
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    sinos = [5.0 + torch.rand((n, angles), device="cuda", generator=gen) for _ in range(2)]
+    got = b.em(b.pack_sinos([sinos[i % 2] for i in range(len(sizes))]), 1, 2)
+    p = Plan(n, n, angles)
+    own = [p.em(s, 1, 2).cpu().numpy() for s in sinos]
+    for i in (0, 1, len(sizes) - 1):
+        assert rel_l2(b.image(got, i).cpu().numpy(), own[i % 2]) <= 1e-5, i
