@@ -1640,10 +1640,14 @@ __global__ __launch_bounds__(256) void k_backprojection(SSDevPlan p, const float
 // time: angles interior to the tile add to all its pixels at once, only those that end in it are
 // tested per pixel.  1024^2, 16 subsets of 45 angles: 365 us as 16 backprojections, 47 here (the
 // angles' FP64 terms and one wait for their loads per block).  SPLIT: launches of few tiles walk
-// their angles too long (226^2, one subset of 449, an iteration: 117 us, split 84), so a block takes 32 x 8
-// pixels, each of its waves all of them for a quarter of the angles.
-template <bool SPLIT>
-__global__ __launch_bounds__(256) void k_bp_weights(SSDevPlan p, int S, int b0, float* __restrict__ out) {
+// their angles too long (226^2, one subset of 449, an iteration: 117 us, split 84), so a block takes
+// 32 x 8 pixels and each of its SPLIT waves all of them for its part of the angles: 4, and for the
+// smallest launches 16 (one subset of 457 angles, many of them ending in a tile, 170^2: 37 us with
+// 4 waves, 14 with 16, 25 as a backprojection of ones; an OSEM call of 1024^2 x 457 in one subset 390
+// with 4, 417 with 16).
+template <int SPLIT>
+__global__ __launch_bounds__(SPLIT ? SPLIT * SS_WAVE : 256) void k_bp_weights(SSDevPlan p, int S, int b0,
+                                                                             float* __restrict__ out) {
   const int n = p.g.n, R = p.g.nrays, A = p.g.nangles, b = b0 + blockIdx.z;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   constexpr int TH = SPLIT ? 8 : 32, STEP = SPLIT ? 2 : 8;  // tile rows, rows between a thread's pixels
@@ -1653,8 +1657,8 @@ __global__ __launch_bounds__(256) void k_bp_weights(SSDevPlan p, int S, int b0, 
   int j0 = (int)((long long)b * A / S), j1 = (int)((long long)(b + 1) * A / S);
   if (SPLIT) {
     const int nj = j1 - j0;
-    j1 = j0 + (int)((wv + 1LL) * nj / 4);
-    j0 += (int)((long long)wv * nj / 4);
+    j1 = j0 + (int)((wv + 1LL) * nj / SPLIT);
+    j0 += (int)((long long)wv * nj / SPLIT);
   }
   const float edge = ss_bp_edge(2 * p.bp_window);  // these tiles may be twice the plan's
   int all = 0, count[4] = {0, 0, 0, 0};
@@ -1681,12 +1685,15 @@ __global__ __launch_bounds__(256) void k_bp_weights(SSDevPlan p, int S, int b0, 
   }
   const float dth = (float)p.g.dth;
   if constexpr (SPLIT) {
-    __shared__ int part[4][TH * 32];
+    __shared__ int part[SPLIT][TH * 32];
 #pragma unroll
     for (int i = 0; i < 4; ++i) part[wv][(ty + STEP * i) * 32 + tx] = all + count[i];
     __syncthreads();
     const int t = threadIdx.x, row = r0 + (t >> 5);
-    const int sum = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+    if (t >= TH * 32) return;
+    int sum = 0;
+#pragma unroll
+    for (int w = 0; w < SPLIT; ++w) sum += part[w][t];
     if (row < n && col < n) out[((size_t)b * n + row) * n + col] = (float)sum * dth;
   } else {
 #pragma unroll
@@ -1699,13 +1706,17 @@ __global__ __launch_bounds__(256) void k_bp_weights(SSDevPlan p, int S, int b0, 
 
 hipError_t ss_launch_bp_weights(const SSDevPlan& p, int nsubsets, float* out, hipStream_t stream) {
   const int t = (p.g.n + 31) / 32;
-  const bool split = (long long)t * t * nsubsets <= SS_BP_ROUND_BLOCKS;
+  const long long tiles = (long long)t * t * nsubsets;
+  const bool split = tiles <= SS_BP_ROUND_BLOCKS;
+  const bool wide = 2 * tiles <= SS_BP_ROUND_BLOCKS && p.g.nangles / nsubsets >= 128;  // 8 angles a wave
   for (int b0 = 0; b0 < nsubsets; b0 += 65535) {  // grid dimension limit
     const dim3 grid(t, split ? (p.g.n + 7) / 8 : t, std::min(nsubsets - b0, 65535));
-    if (split)
-      hipLaunchKernelGGL(k_bp_weights<true>, grid, dim3(256), 0, stream, p, nsubsets, b0, out);
+    if (wide)
+      hipLaunchKernelGGL(k_bp_weights<16>, grid, dim3(16 * SS_WAVE), 0, stream, p, nsubsets, b0, out);
+    else if (split)
+      hipLaunchKernelGGL(k_bp_weights<4>, grid, dim3(4 * SS_WAVE), 0, stream, p, nsubsets, b0, out);
     else
-      hipLaunchKernelGGL(k_bp_weights<false>, grid, dim3(256), 0, stream, p, nsubsets, b0, out);
+      hipLaunchKernelGGL(k_bp_weights<0>, grid, dim3(256), 0, stream, p, nsubsets, b0, out);
   }
   return hipGetLastError();
 }

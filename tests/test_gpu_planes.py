@@ -313,3 +313,10 @@ def test_backprojection_few_angles(n, A, sc, groups):
     ref = O.backprojection(s[0].astype(np.float64), n, **_geo(sc))
     assert _rel(one, ref) <= REL and _rel(got[0], ref) <= REL
     assert _rel(got[2], O.backprojection(s[2].astype(np.float64), n, **_geo(sc))) <= REL
+
+
+# subsets of at least 128 angles on few tiles: 16 waves a block, of 8, 9 and 65 angles each
+@pytest.mark.parametrize("n,R,A,sc,S", [(40, 41, 128, (0.0, 1.0, PI, -1.0), 1), (65, 64, 280, (0.0, 0.9, 2.0, -0.84), 2),
+                                        (33, 31, 1030, (0.0, 1.0, PI, -0.94), 1)])
+def test_osem_weights_many_angles(n, R, A, sc, S):
+    test_osem_weights(n, R, A, sc, S)
