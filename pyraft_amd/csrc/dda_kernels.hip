@@ -1296,7 +1296,7 @@ SSDdaRadonForm dda_radon_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp, 
   if (kind == SS_PLANES_NONE) return f;
   const int groups = ss_planes_groups(kind, nslices);
   const SSDdaRadonPlanes rp = dda_radon_planes(g, tp, kind, nslices);
-  if (dda_radon_planes_blocks(g, rp) > 0x7fffffffLL) return f;
+  if (dda_radon_planes_blocks(g, rp) * RADON_WAVES * SS_WAVE > SS_GRID_THREADS) return f;
   f.kind = kind;
   f.nslab = rp.nslab;
   f.layout = sizeof(ss_f32x4) * (size_t)groups *
@@ -1350,9 +1350,9 @@ SSDdaGatherForm dda_gather_form(const SSDdaGeom& g, const SSDdaTransposePlan& tp
   f.kind = dda_planes_kind(tp, nslices);
   if (f.kind == SS_PLANES_NONE) return f;
   const long long tiles = (long long)dda_gp_cols(g, f.kind) * dda_gp_rows(g, f.kind) * ss_planes_groups(f.kind, nslices);
-  if (tiles * DDA_GP_MAXGROUPS > 0x7fffffffLL) return SSDdaGatherForm{SS_PLANES_NONE, 1};
   const long long want = std::max<long long>((DDA_GP_BLOCKS + tiles / 2) / tiles, tiles <= DDA_GP_PAIR_TILES ? 2 : 1);
   f.ngroups = (int)std::min<long long>({DDA_GP_MAXGROUPS, want, (tp.ngather + DDA_GP_ANGLES - 1) / DDA_GP_ANGLES});
+  if (tiles * f.ngroups * 256 > SS_GRID_THREADS) return SSDdaGatherForm{SS_PLANES_NONE, 1};
   return f;
 }
 

@@ -9,6 +9,9 @@
 #define SS_PLANES 4
 #define SS_WAVE 64
 
+// Threads of a launch along one dimension at most; HIP cuts a longer one short without an error
+#define SS_GRID_THREADS 0xffffffffLL
+
 #ifndef RADON_WAVES
 #define RADON_WAVES 8  // angles (one per wave) of a Radon block
 #endif

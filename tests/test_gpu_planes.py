@@ -320,3 +320,19 @@ def test_backprojection_few_angles(n, A, sc, groups):
                                         (33, 31, 1030, (0.0, 1.0, PI, -0.94), 1)])
 def test_osem_weights_many_angles(n, R, A, sc, S):
     test_osem_weights(n, R, A, sc, S)
+
+
+def test_line_radon_many_slices():
+    """Straight angles' blocks of 65535 slices on a wide detector: with them the planes' launch
+    would have more threads than a grid dimension holds, so the one-ray form runs."""
+    import torch
+    from pyraft_amd.device import DdaPlan
+    S, R = 65535, 4096
+    print("line radon, %d slices, %d rays" % (S, R), flush=True)
+    p = DdaPlan(2, R, 4)
+    x = torch.rand((S, 2, 2), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    got = p.radon(x)
+    for i in (0, S // 2, S - 1):
+        own = p.radon(x[i:i + 1])[0]
+        assert float(own.abs().max()) > 0.1
+        assert float((got[i] - own).abs().max()) <= 1e-5 * float(own.abs().max()), i
