@@ -755,18 +755,23 @@ extern "C" int raft_ss_radon_transpose_range(const raft_ss_plan* p, const float*
   if (!d_image || !d_sino) return set_error(RAFT_SS_EINVAL, "null device pointer");
   hipStream_t stream = as_stream(stream_);
   const SSDevPlan dp = p->dev();
-  const float* sT = d_sino;
   const bool pixels = dp.rt_angles > 0;  // reads either layout
-  const size_t sino_floats = angle_major || pixels ? 0 : (size_t)nslices * p->g.nrays * p->g.nangles;
-  const size_t scratch = ss_radon_transpose_scratch(dp, j0, j1, nslices);
-  Scratch ws;
-  HIP_TRY(ws.alloc(sino_floats * sizeof(float) + scratch, stream));
-  if (sino_floats) {
-    HIP_TRY(ss_launch_sino_to_t(d_sino, ws.as<float>(), p->g.nrays, p->g.nangles, nslices, stream));
-    sT = ws.as<float>();
+  const int most = ss_radon_transpose_slices(dp, j0, j1, nslices);
+  for (int s0 = 0; s0 < nslices; s0 += most) {
+    const int ns = std::min(most, nslices - s0);
+    const float* sino = d_sino + (size_t)s0 * p->g.nrays * p->g.nangles;
+    const size_t sino_floats = angle_major || pixels ? 0 : (size_t)ns * p->g.nrays * p->g.nangles;
+    const size_t scratch = ss_radon_transpose_scratch(dp, j0, j1, ns);
+    Scratch ws;
+    HIP_TRY(ws.alloc(sino_floats * sizeof(float) + scratch, stream));
+    if (sino_floats) {
+      HIP_TRY(ss_launch_sino_to_t(sino, ws.as<float>(), p->g.nrays, p->g.nangles, ns, stream));
+      sino = ws.as<float>();
+    }
+    HIP_TRY(ss_launch_radon_transpose(dp, sino, !angle_major && pixels, j0, j1, ns,
+                                      d_image + (size_t)s0 * p->g.n * p->g.n,
+                                      scratch ? ws.as<float>() + sino_floats : nullptr, stream));
   }
-  HIP_TRY(ss_launch_radon_transpose(dp, sT, !angle_major && pixels, j0, j1, nslices, d_image,
-                                    scratch ? ws.as<float>() + sino_floats : nullptr, stream));
   return 0;
 }
 

@@ -406,6 +406,9 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
   SSDevPlan dpp = dp;
   if ((double)n * p->g.nrays * (j1 - j0) * nslices >= kPlanesUpdates)
     dpp.radon_planes = ss_plan_planes(p, j0, j1, nslices);
+  // their blocks fill one grid dimension
+  if (dpp.radon_planes && ss_planes_blocks(dpp, j0, j1, 1) * RADON_WAVES * SS_WAVE > SS_GRID_THREADS)
+    dpp.radon_planes = SS_PLANES_NONE;
   const int planes = dpp.radon_planes;
   // A launch that the planes suit in every respect takes them without timing: blocks for the
   // whole chip (ss_planes_suit), an image of 512^2 or more, and angles near enough that a block's

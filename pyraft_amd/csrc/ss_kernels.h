@@ -202,6 +202,8 @@ hipError_t ss_launch_backprojection(const SSDevPlan& p, const float* sinoT, int 
 // images; the line form's transposed n x n FP32 image per slice (where the lines of the angles
 // that walk image columns accumulate before k_transpose_add)
 size_t ss_radon_transpose_scratch(const SSDevPlan& p, int j0, int j1, int nslices);
+// slices that one launch takes at most: its blocks fill one grid dimension (SS_GRID_THREADS)
+int ss_radon_transpose_slices(const SSDevPlan& p, int j0, int j1, int nslices);
 // in_cols: sinoT is in the (R, A) layout (pixel-driven form only: p.rt_angles > 0)
 hipError_t ss_launch_radon_transpose(const SSDevPlan& p, const float* sinoT, int in_cols, int j0, int j1, int nslices,
                                      float* out, float* scratch, hipStream_t stream);

@@ -2689,6 +2689,23 @@ size_t ss_radon_transpose_scratch(const SSDevPlan& p, int j0, int j1, int nslice
   return sizeof(float) * (((ss_rt_planes_floats(p, kind, nslices) + 3) & ~(size_t)3) + (G > 1 ? G * img : 0));
 }
 
+// blocks of the border (k_radon_transpose_px), and all of them
+static long long ss_rt_border_blocks(const SSDevPlan& p, int nslices, int G) {
+  return 4LL * ((p.g.n + 31) / 32) * ((nslices + RTP_EDGE_SLICES - 1) / RTP_EDGE_SLICES) * G;
+}
+static long long ss_rt_blocks(const SSDevPlan& p, int j0, int j1, int nslices) {
+  const int kind = ss_rt_kind(p, j0, j1, nslices), G = ss_rt_groups(p, j0, j1, nslices), per = ss_rt_slices(kind);
+  const dim3 tiles = ss_rt_grid(p, kind);
+  return ss_rt_border_blocks(p, nslices, G) + (long long)tiles.x * tiles.y * ((nslices + per - 1) / per) * G;
+}
+
+int ss_radon_transpose_slices(const SSDevPlan& p, int j0, int j1, int nslices) {
+  if (p.rt_angles <= 0) return nslices;
+  int most = nslices;
+  while (most > SS_PLANES_STACK && ss_rt_blocks(p, j0, j1, most) * 256 > SS_GRID_THREADS) most = (most / 2 + 3) & ~3;
+  return most;
+}
+
 template <int PL>
 static hipError_t ss_launch_rtp(const SSDevPlan& p, const float* in, int in_cols, int kind, int j0, int j1,
                                 int nslices, float* out, float* scratch, hipStream_t stream) {
@@ -2701,7 +2718,7 @@ static hipError_t ss_launch_rtp(const SSDevPlan& p, const float* in, int in_cols
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const dim3 tiles = ss_rt_grid(p, kind);
-  const int nborder = 4 * ((p.g.n + 31) / 32) * ((nslices + RTP_EDGE_SLICES - 1) / RTP_EDGE_SLICES) * G;
+  const int nborder = (int)ss_rt_border_blocks(p, nslices, G);
   const dim3 grid(nborder + tiles.x * tiles.y * groups * G);
 #define SS_RTP_LAUNCH(V, ROWS, STAGE)                                                                             \
   case V:                                                                                                         \

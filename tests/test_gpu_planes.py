@@ -336,3 +336,18 @@ def test_line_radon_many_slices():
         own = p.radon(x[i:i + 1])[0]
         assert float(own.abs().max()) > 0.1
         assert float((got[i] - own).abs().max()) <= 1e-5 * float(own.abs().max()), i
+
+
+def test_transpose_many_slices():
+    """More slices than one launch's grid dimension holds blocks for."""
+    import torch
+    from pyraft_amd.device import Plan
+    S = 14000002
+    print("transpose, %d slices" % S, flush=True)
+    y = torch.rand((S, 2, 1), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    p = Plan(2, 2, 1)
+    got = p.radon_transpose(y)
+    for i in (0, S // 2, S - 1):
+        own = p.radon_transpose(y[i:i + 1])[0]
+        assert float(own.abs().max()) > 0.0
+        assert float((got[i] - own).abs().max()) <= 1e-5 * float(own.abs().max()), i
