@@ -351,3 +351,29 @@ def test_transpose_many_slices():
         own = p.radon_transpose(y[i:i + 1])[0]
         assert float(own.abs().max()) > 0.0
         assert float((got[i] - own).abs().max()) <= 1e-5 * float(own.abs().max()), i
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("sc,S", [((0.0, 1.0, PI, -1.0), 6), ((0.0, 1.0, 2.0, -1.0), 6), ((0.0, 1.03, PI, -0.97), 8),
+                                  ((0.0, 1.0, PI, -1.0), 12)])
+def test_slices_stay_apart(sc, S, bad):
+    """A slice of NaN or Inf next to others that share its trajectories, windows and pixels: the
+    others' bits don't change, forwards and backwards, and its own values are not finite."""
+    import torch
+    from pyraft_amd.device import DdaPlan, Plan
+    n, R, A = 512, 512, 720
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.rand((S, n, n), device="cuda", generator=gen)
+    y = torch.rand((S, R, A), device="cuda", generator=gen)
+    ops = []
+    for p in (Plan(n, R, A, sino_corners=sc), DdaPlan(n, R, A, sino_corners=sc)):
+        ops += [(p.radon, x), (p.radon_transpose, y), (p.backprojection, y)]
+    for k, (op, v) in enumerate(ops):
+        print("slices apart", sc, S, bad, k, flush=True)
+        clean = op(v)
+        w = v.clone()
+        w[1] = bad
+        got = op(w)
+        keep = [i for i in range(S) if i != 1]
+        assert torch.equal(got[keep], clean[keep]), k
+        assert not torch.isfinite(got[1][n // 2, n // 2])
