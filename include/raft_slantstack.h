@@ -309,7 +309,12 @@ int raft_ss_plan_tune_transpose(raft_ss_plan *plan, int nslices, int reps, int f
  * items of all slices, heaviest first), the layout kernels (gather layouts, sinogram
  * transposes) with one block per tile of every slice; and with
  * RAFT_SS_BATCH_GRAPH the whole call is captured once into a HIP graph and
- * replayed by a single graph launch on later calls with the same arguments. */
+ * replayed by a single graph launch on later calls with the same arguments.
+ *
+ * A batch's calls share its work buffers (layouts, sinogram copies, the OSEM weights
+ * BP_b(1), which depend on the geometry alone and are computed by the first OSEM call
+ * with their subset count): calls on different streams must be ordered by the caller, as
+ * on one stream. */
 typedef struct raft_ss_batch raft_ss_batch;
 #define RAFT_SS_BATCH_GRAPH 1
 /* img_corners / sino_corners: nslices x 4 doubles, or NULL for the defaults (image

@@ -10,7 +10,8 @@ into a HIP graph and replayed by one graph launch.
 Data live in packed float32 device buffers: slice i's image is the n_i x n_i block
 at ``img_off[i]`` and its sinogram the R_i x A_i block (or A_i x R_i, angle-major)
 at ``sino_off[i]``; ``pack_images`` / ``unpack_images`` and the sinogram
-equivalents convert from and to lists of tensors.
+equivalents convert from and to lists of tensors.  Calls of one ``Batch`` share its work
+buffers: on several streams, order them (``Stream.wait_stream``).
 """
 import ctypes
 

@@ -628,7 +628,7 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE, PLANES_BLOCKS) void k_dda_ra
   chi = ss_rfl(chi);
   const int branch = uhi < ulo ? -1 : (a.fast_i ? 0 : 1);
   if (lane == 0) {
-    lds.wmeta[wv][0] = lds.wmeta[wv][3] = branch;
+    lds.wmeta[wv][0] = branch;
     lds.wmeta[wv][1] = ulo;
     lds.wmeta[wv][2] = uhi;
     lds.wpar[wv][0] = amin;

@@ -314,7 +314,7 @@ template <int CAP>
 struct SSRadonLds {
   double red[RADON_WAVES];
   int64_t wpar[RADON_WAVES][3];  // per wave: lowest and highest trajectory offset of its rays, slope
-  int wmeta[RADON_WAVES][4];     // per wave: branch (-1: no samples), first row, last row
+  int wmeta[RADON_WAVES][3];     // per wave: branch (-1: no samples), first row, last row
   int wred[2][RADON_WAVES];      // per wave: widest window of a table pass (two passes in turn)
   int2 table[RADON_TABLE];       // per chunk of the super-chunk: first staged record, records per row
   __attribute__((aligned(16))) float2 stage[CAP + 2];  // chunk window; record CAP stays (0, 0)
@@ -659,8 +659,8 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE) void k_radon(SSDevPlan p, co
 // Radon in planes: four rays per trajectory
 //
 // The one-ray kernel above is bound by its LDS reads (8-byte records gamma = 1..1.41 cells
-// apart: two-way bank conflicts, 7.9 lane-reads per CU-clock where the stride exceeds ~1.05)
-// and issues 5 VALU instructions per update, three of them for the trajectory, its weight
+// apart; reads alone reach 13.7 lane-reads per CU-clock at 1 cell, 9.0 at 1.05 and, with two-way
+// bank conflicts, 7.9 from 1.1 on) and issues 5 VALU instructions per update, three of them for the trajectory, its weight
 // and the address.  Here a lane's trajectory serves four rays whose samples lie at the same
 // cell of four images, the planes:
 //   SS_PLANES_QUAD    on a grid symmetric about the rotation axis, over all angles of
@@ -672,11 +672,12 @@ __global__ __launch_bounds__(RADON_WAVES * SS_WAVE) void k_radon(SSDevPlan p, co
 // read gives the lower taps and another the upper taps of all four; the lanes of a read
 // pass hold 16 neighbouring rays (ss_plane_ray), which keeps its conflicts two-way.  Per
 // four updates: 5 VALU for the trajectory, address and the two weights, 8 FMAs, two reads
-// (16 updates per CU-clock at any stride).  Sums are taken in FP32 over 8 samples, those over
+// (such pairs of reads alone: 26 updates per CU-clock at a stride of 1, 18 at 1.05, 16 from 1.1 on;
+// in the order of the lanes 10.5 at 1.41).  Sums are taken in FP32 over 8 samples, those over
 // a chunk's rows and those over the ray: 1e-7 from the 64-bit sums at 2048^2 x 1500 (one
-// running sum per ray: 6e-7).  2048^2 x 1500: 1.07 -> 0.78 ms, the layouts' 27 us included; the
-// kernel issues VALU 0.85 and reads LDS 0.75 of the clocks a CU is busy, which is 0.85 of its
-// time (2.9 rounds of blocks).
+// running sum per ray: 6e-7).  2048^2 x 1500: 1.07 -> 0.80 ms, the layouts' 27 us included; the
+// kernel issues VALU in 0.83 and reads LDS in 0.74 of the clocks a CU is busy, which is 0.8 of
+// its time (2.9 rounds of blocks).
 //
 // Every plane's ray keeps its own exact sample range, delta and output; rays computed twice
 // (the middle ray of an odd detector, theta = 0 and pi/2, slices past the last) are stored
@@ -885,7 +886,6 @@ __device__ __forceinline__ void ss_planes_item(const SSRadonView& p, const ss_f3
     lds.wmeta[wv][0] = branch;
     lds.wmeta[wv][1] = ulo;
     lds.wmeta[wv][2] = uhi;
-    lds.wmeta[wv][3] = branch;
     lds.wpar[wv][0] = amin;
     lds.wpar[wv][1] = amax;
     lds.wpar[wv][2] = beta;
@@ -1268,7 +1268,7 @@ hipError_t ss_launch_radon(const SSDevPlan& p, const float2* gatherA, const floa
 //
 // Exactness of the 0 <= m <= R-2 predicate: a tile whose U range lies inside
 // [eps, R-1-eps] needs no test; one entirely outside contributes nothing; the rest
-// test each pixel, and pixels within 1e-3 bins of an edge re-evaluate the
+// test each pixel, and pixels within W 2^-20 bins of an edge (ss_bp_edge) re-evaluate the
 // reference's FP64 expression.
 // =====================================================================================
 
@@ -2298,7 +2298,7 @@ __device__ __forceinline__ RTPAngle ss_rtp_params(const SSDevPlan& p, int j, int
   return q;
 }
 
-// The planes of a launch (SSRtPlanes; ss_launch_radon_transpose chooses): a block's pixel tile
+// The planes of a launch (ss_rt_kind chooses): a block's pixel tile
 // and PL planes that share each pixel's geometry (kappa, floor, weights).  QUAD, PAIR and
 // SLICES as for the Radon (ss_plane): the half turn of pixel (r, c) has the ray coordinate
 // R - 1 - kappa, the mirror (r, n-1-c) has kappa at the angle pi - theta.  TURN: one slice and
@@ -2649,8 +2649,9 @@ static int ss_rt_lines(int n, int sl) {
 }
 
 // Planes of a pixel-driven transpose over angles [j0, j1) of nslices slices.  Every plane's
-// arithmetic is the same in each of them, so a slice's result does not depend on what it is
-// launched with.
+// arithmetic is the same in each of them, so up to SS_PLANES_STACK slices, which also share one
+// slice's angle groups (ss_rt_groups), have the bits of a launch of their own; larger stacks
+// choose their groups, and with them the order of the sums, by all their tiles.
 static int ss_rt_kind(const SSDevPlan& p, int j0, int j1, int nslices) {
   if (4 * (p.rt_window + 4) > 2 * kSSBpStage[p.rt_variant]) return SS_RT_ONE;  // a window of four does not fit
   if (ss_planes_stack(nslices)) return SS_PLANES_SLICES;

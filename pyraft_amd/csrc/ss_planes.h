@@ -125,7 +125,7 @@ typedef __attribute__((address_space(3))) const ss_f32x4* ss_lds_cell;
 struct SSPlanesLds {
   double red[RADON_WAVES];
   int64_t wpar[RADON_WAVES][3];  // as SSRadonLds
-  int wmeta[RADON_WAVES][4];
+  int wmeta[RADON_WAVES][3];
   int wred[2][RADON_WAVES];
   int2 table[RADON_TABLE];
   alignas(16) ss_f32x4 stage[PLANES_CAP + 2];  // chunk window; cells CAP, CAP + 1 stay 0
