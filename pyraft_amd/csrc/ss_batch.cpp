@@ -604,6 +604,11 @@ struct GraphEntry {
 constexpr long long SS_BATCH_PAIR_TILES = 512;
 constexpr long long SS_BATCH_ROWS_TILES = 8192;  // 4-row tiles from here on
 
+int whole_planes(const SSDevPlan& p, int j0, int j1) {
+  const int planes = ss_bp_launch_planes(p, j0, j1, 1);
+  return planes == 1 && p.bp_pair > 0 && ss_bp_groups(p, j0, j1, 1) > 1 ? 2 : planes;
+}
+
 int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace
@@ -695,11 +700,12 @@ int build_launch(raft_ss_batch* b, BatchLaunch& L, int kind, int S, int bsub, in
     if (S > 0) subset_range(p.g.nangles, S, bsub, &j0, &j1);
     blocks += ss_radon_blocks(p.nwaves, j0, j1);
   }
-  // Planes of the backprojection's tiles: whole ranges as a plan's launch of the slice takes them.
+  // Planes of the backprojection's tiles: whole ranges (whole_planes) as a plan's launch of the
+  // slice takes them (where that is undivided the bits agree), at least two in place of its groups.
   // Subset ranges are short, so a block's time is latency, and a launch of few tiles is not
   // shorter for having fewer: two planes from SS_BATCH_PAIR_TILES tiles on.
   auto bp_planes = [&](const raft_ss_plan& p, int j0, int j1, bool pairs) {
-    if (mode == SS_BP_PLAIN && j0 == 0 && j1 == p.g.nangles) return ss_bp_launch_planes(p.dev(v), j0, j1, 1);
+    if (mode == SS_BP_PLAIN && j0 == 0 && j1 == p.g.nangles) return whole_planes(p.dev(v), j0, j1);
     return pairs && p.bp_stage_v(v, 2) > 0 ? 2 : 1;
   };
   bool pairs = true;
@@ -1198,7 +1204,7 @@ extern "C" int raft_ss_batch_tune(raft_ss_batch* b, int reps, int flags, void* s
         sl.sino_off = b->sino_off[i];
         sl.lay_off = b->lay_off[i];
         SSBatchEntry e{(int)h.size(), 0, std::min(sl.p.g.nangles, 360), (int)total};
-        e.planes = ss_bp_launch_planes(sl.p, e.j0, e.j1, 1);
+        e.planes = whole_planes(sl.p, e.j0, e.j1);
         h.push_back(sl);
         L.entries.push_back(e);
         total += ss_bp_tiles(sl.p.g.n, v, e.planes);

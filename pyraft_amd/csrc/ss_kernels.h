@@ -179,13 +179,17 @@ hipError_t ss_launch_bp_weights(const SSDevPlan& p, int nsubsets, float* out, hi
 // SS_BP_SHORT_ANGLES, or with T >= SS_BP_SHORT_TILES tiles of 32 x 16 pixels (two planes) up to
 // SS_BP_SHORT_ANGLES + T / 8 and at most 160, launch undivided, with two planes in place of four
 // below SS_BP_SHORT_QUAD tiles of four (us, in groups with four planes / undivided with two / with
-// four: 512^2 x 24 13.0 / 10.0 / 10.0; 512^2 x 64 13.3 / 15.0 / 18.7; 789^2 x 40 18.7 / 11.6 / 13.8; 789^2 x 91
+// four: 512^2 x 40 12.9 / 11.0 / 13.6; 512^2 x 64 13.3 / 15.0 / 18.7; 789^2 x 40 18.7 / 11.6 / 13.8; 789^2 x 91
 // 24.1 / 20.3 / 23.7; 1024^2 x 128 31.6 / 29.3 / 34.2; 1024^2 x 180 35.5 / 38.9 / 43.7; 1448^2 x 40 26.7 / 20.6 /
-// 18.6).  In groups, four planes pay from SS_BP_QUAD_WORK tiles of four (32 x 16) x angles on (a
-// filtered backprojection, two / four planes: 135^2 x 47 16.5 / 17.7, 256^2 x 91 16.4 / 17.7, 256^2 x 128
-// 17.4 / 19.0, 256^2 x 180 19.3 / 18.6, 363^2 x 91 21.8 / 21.2).
+// 18.6; a filtered backprojection in groups / undivided, one plane: 182^2 x 20 15.2 / 13.7, x 24 15.1 / 14.6,
+// x 31 15.6 / 16.0).  In groups, four planes pay from SS_BP_QUAD_WORK tiles of four (32 x 16) x angles
+// on (filtered, two / four planes: 135^2 x 47 16.5 / 17.7, 256^2 x 91 16.4 / 17.7, 256^2 x 128 17.4 / 19.0,
+// 256^2 x 180 19.3 / 18.6, 363^2 x 91 21.8 / 21.2), and two from SS_BP_PAIR_WORK tiles of two x angles on
+// (one / two planes: 135^2 x 47 15.9 / 16.5, 182^2 x 47 15.9 / 16.7, 135^2 x 128 16.9 / 16.2, 256^2 x 91 17.9 /
+// 16.4; two slices of 182^2 x 39 over 2 rad 15.6 / 16.5).
+#define SS_BP_PAIR_WORK 3000
 #define SS_BP_QUAD_WORK 5000
-#define SS_BP_SHORT_ANGLES 32
+#define SS_BP_SHORT_ANGLES 24
 #define SS_BP_SHORT_TILES 240
 #define SS_BP_SHORT_QUAD 512
 #define SS_BP_GROUP_SCALE 0.22

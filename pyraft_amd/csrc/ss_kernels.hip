@@ -1778,6 +1778,7 @@ static bool ss_bp_short(const SSDevPlan& p, int j0, int j1, int nslices) {
 
 int ss_bp_launch_planes(const SSDevPlan& p, int j0, int j1, int nslices) {
   const int planes = ss_bp_planes(p, j0, j1), ns = std::max(nslices, 1);
+  if (planes > 1 && (long long)ss_bp_tiles(p.g.n, 1, 2) * ns * (j1 - j0) < SS_BP_PAIR_WORK) return 1;
   if (planes < 4 || p.bp_pair <= 0) return planes;
   const long long small = (long long)ss_bp_tiles(p.g.n, 1, 4) * ns, large = (long long)ss_bp_tiles(p.g.n, 0, 4) * ns;
   if (small * (j1 - j0) < SS_BP_QUAD_WORK) return 2;

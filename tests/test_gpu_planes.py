@@ -297,11 +297,13 @@ def test_small_radon_keeps_its_candidates(tmp_path):
 # one angle on either side of the line between undivided and divided launches: few angles at any
 # size, more where the tiles fill the chip; two planes and four
 @pytest.mark.parametrize("n,A,sc,groups", [
-    (40, 31, (0.0, 1.0, PI, -1.0), False), (40, 32, (0.0, 1.0, PI, -1.0), True),
-    (512, 64, (0.0, 1.0, PI, -1.0), False), (512, 65, (0.0, 1.0, PI, -1.0), True),
-    (789, 40, (0.0, 1.0, 2.0, -1.0), False), (789, 110, (0.0, 1.0, PI, -1.0), False),
-    (789, 111, (0.0, 1.0, PI, -1.0), True), (1448, 24, (0.0, 1.0, PI, -1.0), False),
-    (500, 60, (0.0, 1.03, PI, -0.97), False)])
+    (40, 23, (0.0, 1.0, PI, -1.0), False), (40, 24, (0.0, 1.0, PI, -1.0), True),
+    (512, 56, (0.0, 1.0, PI, -1.0), False), (512, 57, (0.0, 1.0, PI, -1.0), True),
+    (789, 40, (0.0, 1.0, 2.0, -1.0), False), (789, 102, (0.0, 1.0, PI, -1.0), False),
+    (789, 103, (0.0, 1.0, PI, -1.0), True), (1448, 24, (0.0, 1.0, PI, -1.0), False),
+    (135, 118, (0.0, 1.0, PI, -1.0), True), (135, 121, (0.0, 1.0, PI, -1.0), True),
+    (256, 155, (0.0, 1.0, PI, -1.0), True), (256, 158, (0.0, 1.0, PI, -1.0), True),
+    (500, 56, (0.0, 1.03, PI, -0.97), False)])
 def test_backprojection_few_angles(n, A, sc, groups):
     import torch
     from pyraft_amd.device import Plan
