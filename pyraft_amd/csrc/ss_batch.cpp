@@ -493,7 +493,10 @@ int ss_plan_radon_rows(const raft_ss_plan* p, int j0, int j1, int nslices, hipSt
         HIP_TRY(ss_launch_radon(d, gA, gB, j0, j1, nslices, SS_OUT_SINOT, sout, none, slabs, stream));
         return 0;
       };
-      return time_best(run, 3, stream, us);
+      // a mesh plan pays for this on its first call: one timed run each keeps that as short as the
+      // one-ray forms' three (3 slices of 521^2 x 264: 1080 us with those alone, 2110 with three runs
+      // of all)
+      return time_best(run, p->mesh && planes ? 1 : 3, stream, us);
     };
     // the first candidate of each form, then the others of a form that is not 1.3 times slower
     // (over the 1000 launches above that never lost against timing all)
