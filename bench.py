@@ -59,8 +59,8 @@ def roofline_of(kernel, updates, seconds, traffic, traffic_src, counters=None):
     Both kernels read their interpolation taps from LDS (8 B, one (tap, difference)
     record or staged pair, per update) and do ~6 FP32 operations per update; HBM traffic
     is a small fraction of the tap bytes because windows are staged once per block.
-    `frac` is the algorithmic demand on the unit over the unit's peak, <= 1 by
-    construction:
+    `frac` is the algorithmic demand on the unit over the unit's peak (the LDS figure is
+    that of 8-byte reads; the planes' 16-byte reads reach 1.6 times it):
       lds (the Radon):          8 B x updates / time  over  LDS_PEAK_GBS
       valu (the backprojection): 6 flops x updates / time  over  VALU_PEAK_TFLOPS
     VALU_PEAK_TFLOPS is the published FP32 figure, which counts packed FP32; these kernels
